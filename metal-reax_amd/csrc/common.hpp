@@ -282,20 +282,160 @@ __device__ inline double pair_dvec_list(const State& st, const double4& pi, int 
 }
 #pragma clang fp contract(on)
 
-// ---- wave (64-lane) reductions in a fixed butterfly order: deterministic run to run --------------------------------
-__device__ inline double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ inline float wave_sum(float v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ inline int wave_sum_int(int v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+// ---- lane exchanges and wave (64-lane) reductions in a fixed butterfly order: deterministic run to run ------------------
+// The exchanges are DPP moves inside a row of 16 lanes and v_permlane16/32_swap across rows, vector instructions, instead of
+// the LDS permutes behind __shfl (two per double and step, each a trip through the LDS pipe: a wave's eleven non-bonded sums
+// were 132 of them). Every sum adds the same pairs in the same order as the xor butterfly (offsets 32, 16, 8, 4, 2, 1).
 __device__ inline int lane_id() { return threadIdx.x & 63; }
+
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;                    // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int kDppShl4 = 0x104, kDppShr4 = 0x114;                  // row_shl:4 (lane i reads i + 4), row_shr:4 (reads i - 4)
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;                  // row_ror:4, row_ror:8 (xor 8 within a row)
+
+template <int C>
+__device__ inline int dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, C, 0xF, 0xF, false); }
+// xor 4 within 8 lanes: banks (groups of 4 lanes) 0 and 2 read from 4 lanes above, banks 1 and 3 from 4 below
+__device__ inline int dpp_xor4(int v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, v, kDppShl4, 0xF, 0x5, false);
+  return __builtin_amdgcn_update_dpp(lo, v, kDppShr4, 0xF, 0xA, false);
+}
+union Bits64 { double d; int i[2]; };
+union Bits32 { float f; int i; };
+template <int C>
+__device__ inline double dpp(double v) {
+  Bits64 b;
+  b.d = v;
+  b.i[0] = dpp<C>(b.i[0]); b.i[1] = dpp<C>(b.i[1]);
+  return b.d;
+}
+template <int C>
+__device__ inline float dpp(float v) {
+  Bits32 b;
+  b.f = v;
+  b.i = dpp<C>(b.i);
+  return b.f;
+}
+__device__ inline double dpp_xor4(double v) {
+  Bits64 b;
+  b.d = v;
+  b.i[0] = dpp_xor4(b.i[0]); b.i[1] = dpp_xor4(b.i[1]);
+  return b.d;
+}
+__device__ inline float dpp_xor4(float v) {
+  Bits32 b;
+  b.f = v;
+  b.i = dpp_xor4(b.i);
+  return b.f;
+}
+// a and b with the upper half of a and the lower half of b exchanged (32 lanes), or the odd rows of a and the even rows of b (16)
+__device__ inline void swap32(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = (int)r[0]; b = (int)r[1];
+}
+__device__ inline void swap16(int& a, int& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = (int)r[0]; b = (int)r[1];
+}
+template <bool k32>
+__device__ inline void swap_rows(double& a, double& b) {
+  Bits64 u, v;
+  u.d = a; v.d = b;
+  if (k32) { swap32(u.i[0], v.i[0]); swap32(u.i[1], v.i[1]); }
+  else { swap16(u.i[0], v.i[0]); swap16(u.i[1], v.i[1]); }
+  a = u.d; b = v.d;
+}
+template <bool k32>
+__device__ inline void swap_rows(float& a, float& b) {
+  Bits32 u, v;
+  u.f = a; v.f = b;
+  if (k32) swap32(u.i, v.i); else swap16(u.i, v.i);
+  a = u.f; b = v.f;
+}
+template <bool k32>
+__device__ inline void swap_rows(int& a, int& b) { if (k32) swap32(a, b); else swap16(a, b); }
+
+// the value of lane i ^ kOff
+template <int kOff, class T>
+__device__ inline T lane_xor(T v) {
+  if constexpr (kOff == 1) return dpp<kDppXor1>(v);
+  else if constexpr (kOff == 2) return dpp<kDppXor2>(v);
+  else if constexpr (kOff == 4) return dpp_xor4(v);
+  else if constexpr (kOff == 8) return dpp<kDppRor8>(v);
+  else {
+    T a = v, b = v;   // a: the even halves (rows) twice, b: the odd ones
+    swap_rows<kOff == 32>(a, b);
+    return (lane_id() & kOff) ? a : b;
+  }
+}
+// sums over aligned groups of G lanes, offsets G / 2 .. 1 in turn; every lane of the group gets the sum
+template <int G, class T>
+__device__ inline T group_sum(T v) {
+  if constexpr (G >= 64) { T a = v, b = v; swap_rows<true>(a, b); v = a + b; }
+  if constexpr (G >= 32) { T a = v, b = v; swap_rows<false>(a, b); v = a + b; }
+  if constexpr (G >= 16) v += dpp<kDppRor8>(v);
+  if constexpr (G >= 16) v += dpp<kDppRor4>(v);   // after the step by 8 the values repeat every 8 lanes: lane i + 4 is lane i ^ 4
+  else if constexpr (G == 8) v += dpp_xor4(v);
+  if constexpr (G >= 4) v += dpp<kDppXor2>(v);
+  if constexpr (G >= 2) v += dpp<kDppXor1>(v);
+  return v;
+}
+__device__ inline double wave_sum(double v) { return group_sum<64>(v); }
+__device__ inline float wave_sum(float v) { return group_sum<64>(v); }
+__device__ inline int wave_sum_int(int v) { return group_sum<64>(v); }
+template <class T>
+__device__ inline T wave_max(T v) {
+  v = max(v, lane_xor<32>(v)); v = max(v, lane_xor<16>(v)); v = max(v, lane_xor<8>(v));
+  v = max(v, lane_xor<4>(v)); v = max(v, lane_xor<2>(v)); v = max(v, lane_xor<1>(v));
+  return v;
+}
+// Wave sums of four values at once: the step by 32 keeps two of them in the halves of one register, the step by 16 all four in
+// its rows, so 21 vector instructions replace 72. Row r of 16 lanes gets the sum of v[r] (the same additions as wave_sum).
+__device__ inline double wave_sum4_rows(double v0, double v1, double v2, double v3) {
+  swap_rows<true>(v0, v2);
+  swap_rows<true>(v1, v3);
+  double s = v0 + v2, t = v1 + v3;   // lower half: sums of v0 (v1), upper half: of v2 (v3)
+  swap_rows<false>(s, t);
+  return group_sum<16>(s + t);
+}
+__device__ inline double read_lane(double v, int lane) {   // lane uniform over the wave
+  Bits64 b;
+  b.d = v;
+  b.i[0] = __builtin_amdgcn_readlane(b.i[0], lane); b.i[1] = __builtin_amdgcn_readlane(b.i[1], lane);
+  return b.d;
+}
+// wave sums of K values in place (every lane gets all of them), four at a time
+template <int K>
+__device__ inline void wave_sums(double (&v)[K]) {
+#pragma unroll
+  for (int k = 0; k < K; k += 4) {
+    const double r = wave_sum4_rows(v[k], k + 1 < K ? v[k + 1] : 0.0, k + 2 < K ? v[k + 2] : 0.0, k + 3 < K ? v[k + 3] : 0.0);
+#pragma unroll
+    for (int q = 0; q < 4 && k + q < K; ++q) v[k + q] = read_lane(r, 16 * q);
+  }
+}
+// acc plus v of the lanes of the aligned group of L lanes, added in lane order (a serial loop's order; every lane gets the sum)
+template <int L, class T>
+__device__ inline T group_sum_ordered(T acc, T v) {
+  if constexpr (L == 1) {
+    acc += v;
+  } else if constexpr (L == 2) {
+    acc += dpp<0xA0>(v); acc += dpp<0xF5>(v);                      // quad_perm [0,0,2,2], [1,1,3,3]
+  } else if constexpr (L == 4) {
+    acc += dpp<0x00>(v); acc += dpp<0x55>(v); acc += dpp<0xAA>(v); acc += dpp<0xFF>(v);   // quad_perm [l,l,l,l]
+  } else {
+    const int base = lane_id() / L * L;
+    for (int l = 0; l < L; ++l) acc += __shfl(v, base + l, 64);
+  }
+  return acc;
+}
+// the value of lane l of the aligned group of L lanes
+template <int L, int l, class T>
+__device__ inline T group_lane(T v) {
+  if constexpr (L == 1) return v;
+  else if constexpr (L == 2) return l == 0 ? dpp<0xA0>(v) : dpp<0xF5>(v);
+  else if constexpr (L == 4) return dpp<l * 0x55>(v);
+  else return __shfl(v, lane_id() / L * L + l, 64);
+}
 // number of set bits of `mask` below this lane
 __device__ inline int lanes_below(unsigned long long mask) { return __popcll(mask & ((1ull << lane_id()) - 1ull)); }
 

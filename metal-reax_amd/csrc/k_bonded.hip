@@ -229,12 +229,7 @@ __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * k
     if (fill > 0) bo_prime_batch<TB>(st, g, t, i, ti, fill, rj, rs, rd, rx, ry, rz, head, nb, sum_bo, ddx, ddy, ddz);
   }
   // fixed-order wave reductions
-  for (int off = 32; off > 0; off >>= 1) {
-    sum_bo += __shfl_xor(sum_bo, off, 64);
-    ddx += __shfl_xor(ddx, off, 64);
-    ddy += __shfl_xor(ddy, off, 64);
-    ddz += __shfl_xor(ddz, off, 64);
-  }
+  sum_bo = wave_sum(sum_bo); ddx = wave_sum(ddx); ddy = wave_sum(ddy); ddz = wave_sum(ddz);
   if (lane == 0) {
     st.b_cnt[i] = nb;
     if (nb > st.maxb) atomicMax(&st.flags[1], nb);
@@ -246,20 +241,18 @@ __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * k
 }
 
 // ---- atom groups: G lanes per atom (G a power of two >= the largest bond count), lane p owns bond slot p of its atom ----------
-// Sums over a group use xor shuffles with offsets below G, so they stay inside the group and run in a fixed order.
+// Sums over a group (group_sum) use lane exchanges with offsets below G, so they stay inside the group and run in a fixed order.
 template <int G>
-__device__ inline int gsum_int(int v) {
-  for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
+__device__ inline int gsum_int(int v) { return group_sum<G>(v); }
 template <int G>
-__device__ inline double gsum(double v) {
-  for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ inline int wave_max(int v) {
-  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-  return v;
+__device__ inline double gsum(double v) { return group_sum<G>(v); }
+
+// calls f(integral_constant l) for l = 0 .. 7 (the lanes of the largest atom group of the slot-parallel kernels)
+template <class F>
+__device__ inline void each_lane(F&& f) {
+  f(std::integral_constant<int, 0>{}); f(std::integral_constant<int, 1>{}); f(std::integral_constant<int, 2>{});
+  f(std::integral_constant<int, 3>{}); f(std::integral_constant<int, 4>{}); f(std::integral_constant<int, 5>{});
+  f(std::integral_constant<int, 6>{}); f(std::integral_constant<int, 7>{});
 }
 
 // ================================================================================================================
@@ -352,16 +345,15 @@ __global__ void __launch_bounds__(256) k_bo_correct(State st, Globals g, Tables 
   const int nb = live ? min(st.b_cnt[i], st.maxb) : 0;
   {   // the largest bond count of this step (flags[7]), one atomic per wave
     int c = live && p0 == 0 ? st.b_cnt[i] : 0;
-    for (int off = 32; off > 0; off >>= 1) c = max(c, __shfl_xor(c, off, 64));
+    c = wave_max(c);
     if (lane_id() == 0 && c > 0) atomicMax(&st.flags[7], c);
   }
   const int nbw = wave_max(nb);
-  const int base = lane_id() - p0;   // the group's first lane
   TB tbo = 0;
   for (int k0 = 0; k0 < nbw; k0 += L) {   // wave-uniform rounds of L slots
     const int p = k0 + p0;
     const TB o = p < nb ? bo_correct_slot<TB>(st, g, t, i, p) : TB(0);
-    for (int l = 0; l < L; ++l) tbo += __shfl(o, base + l, 64);   // slot order; absent slots add exact zeros
+    tbo = group_sum_ordered<L>(tbo, o);   // slot order; absent slots add exact zeros
   }
   if (!live || p0 != 0) return;
   const int ti = st.type[i];
@@ -402,7 +394,6 @@ __global__ void __launch_bounds__(256) k_atom_terms(State st, Globals g, Tables 
   const int ti = live ? st.type[i] : -1;
   const int nb = ti >= 0 ? min(st.b_cnt[i], st.maxb) : 0;
   const int nbw = wave_max(nb);
-  const int base = lane_id() - p0;
   const size_t nsl = (size_t)st.maxb * n;
   if (live && p0 == 0 && st.peratom)   // the reference-split virial shares, accumulated by the angle kernels that follow
     for (int c = 0; c < 6; ++c) st.vref[(size_t)c * n + i] = 0.0;
@@ -446,11 +437,13 @@ __global__ void __launch_bounds__(256) k_atom_terms(State st, Globals g, Tables 
         st.Cdbo[q] += cdbo;
       }
     }
-    for (int l = 0; l < L; ++l) {   // slot order; slots without these terms add exact zeros
-      e_bond += __shfl(eb, base + l, 64);
-      e_bond += __shfl(et, base + l, 64);
-      cdself += __shfl(cdt, base + l, 64);
-    }
+    // slot order; slots without these terms add exact zeros
+    auto add = [&](auto lc) {
+      constexpr int l = decltype(lc)::value;
+      if constexpr (l < L) { e_bond += group_lane<L, l>(eb); e_bond += group_lane<L, l>(et); }
+    };
+    each_lane(add);
+    cdself = group_sum_ordered<L>(cdself, cdt);
   }
   const DevSpecies& si = t.sp[ti >= 0 ? ti : 0];
   // lone pair
@@ -480,12 +473,9 @@ __global__ void __launch_bounds__(256) k_atom_terms(State st, Globals g, Tables 
           }
         }
       }
-      for (int l = 0; l < L; ++l) {
-        const double e = __shfl(ec, base + l, 64);
-        e_lp += e;
-        e_c2 += e;
-        cdself += __shfl(cdc, base + l, 64);
-      }
+      e_lp = group_sum_ordered<L>(e_lp, ec);
+      e_c2 = group_sum_ordered<L>(e_c2, ec);
+      cdself = group_sum_ordered<L>(cdself, cdc);
     }
   }
   // over / under coordination (reference bonded.cpp:282-318, terms.hpp:231-260)
@@ -502,10 +492,8 @@ __global__ void __launch_bounds__(256) k_atom_terms(State st, Globals g, Tables 
         a1 = (TR)P.p_ovun1 * (TR)P.De_s * (TR)st.bo[q];
         a2 = ((TR)st.Delta[j] - dfvl * (TR)st.Delta_lp_temp[j]) * ((TR)st.bo_pi[q] + (TR)st.bo_pi2[q]);
       }
-      for (int l = 0; l < L; ++l) {
-        sum1 += __shfl(a1, base + l, 64);
-        sum2 += __shfl(a2, base + l, 64);
-      }
+      sum1 = group_sum_ordered<L>(sum1, a1);
+      sum2 = group_sum_ordered<L>(sum2, a2);
     }
     if (ti >= 0) {
       const bool under = nb > 0 || g.enobonds;
@@ -1152,8 +1140,11 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
           }
         }
       }
-      c1 = wave_sum(c1); fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
-      if (lane == 0) { st.Cdbo[q] += c1; st.fpx[q] += fx; st.fpy[q] += fy; st.fpz[q] += fz; }
+      {   // row r of 16 lanes holds the r-th sum: its first lane adds it to the bond's slot
+        const double s = wave_sum4_rows(c1, fx, fy, fz);
+        double* const to = lane < 32 ? (lane < 16 ? st.Cdbo : st.fpx) : (lane < 48 ? st.fpy : st.fpz);
+        if (lane % 16 == 0) to[q] += s;
+      }
       if (PA) {
         const size_t nsl = (size_t)st.maxb * n;
         for (int c = 0; c < 6; ++c) {
@@ -1209,8 +1200,12 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
     }
   }
   if (fill > 0) batch(fill);
-  e_hb = wave_sum(e_hb); fjx = wave_sum(fjx); fjy = wave_sum(fjy); fjz = wave_sum(fjz);
-  for (int c = 0; c < 6; ++c) w[c] = wave_sum(w[c]);
+  {
+    double s[10] = {e_hb, fjx, fjy, fjz, w[0], w[1], w[2], w[3], w[4], w[5]};
+    wave_sums<10>(s);
+    e_hb = s[0]; fjx = s[1]; fjy = s[2]; fjz = s[3];
+    for (int c = 0; c < 6; ++c) w[c] = s[4 + c];
+  }
   if (lane == 0) {
     st.fs_x[j] += fjx; st.fs_y[j] += fjy; st.fs_z[j] += fjz;
     for (int c = 0; c < 6; ++c) st.vb[(size_t)c * n + j] += w[c];
@@ -1254,8 +1249,11 @@ __global__ void __launch_bounds__(256) k_hbond_acceptor(State st, Globals g, Tab
       for (int c = 0; c < 6; ++c) va[c] += st.vhc[c * nhc + o];
     }
   }
-  fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
-  if (lane == 0) { st.fs_x[k] += fx; st.fs_y[k] += fy; st.fs_z[k] += fz; }
+  {   // row r of 16 lanes holds the r-th component
+    const double s = wave_sum4_rows(fx, fy, fz, 0.0);
+    double* const to = lane < 32 ? (lane < 16 ? st.fs_x : st.fs_y) : st.fs_z;
+    if (lane % 16 == 0 && lane < 48) to[k] += s;
+  }
   if (st.peratom) {
     e = wave_sum(e);
     for (int c = 0; c < 6; ++c) va[c] = wave_sum(va[c]);
@@ -1291,7 +1289,7 @@ __global__ void __launch_bounds__(256) k_cdelta(State st) {
   const int i = gid / L, p0 = gid % L, n = st.n;
   const bool live = i < n;
   const int nb = live ? min(st.b_cnt[i], st.maxb) : 0;
-  const int nbw = wave_max(nb), base = lane_id() - p0;
+  const int nbw = wave_max(nb);
   double c = live ? st.CdD_self[i] : 0.0;
   for (int k0 = 0; k0 < nbw; k0 += L) {
     const int p = k0 + p0;
@@ -1300,7 +1298,7 @@ __global__ void __launch_bounds__(256) k_cdelta(State st) {
       const size_t q = sl(p, i, n);
       v = st.cdp[sl(st.b_sym[q], st.b_j[q], n)];
     }
-    for (int l = 0; l < L; ++l) c += __shfl(v, base + l, 64);
+    c = group_sum_ordered<L>(c, v);
   }
   if (live && p0 == 0) st.CdD[i] = c;
 }
@@ -1311,7 +1309,7 @@ __global__ void __launch_bounds__(256) k_dbond(State st) {
   const int i = gid / L, p0 = gid % L, n = st.n;
   const bool live = i < n;
   const int nb = live ? min(st.b_cnt[i], st.maxb) : 0;
-  const int nbw = wave_max(nb), base = lane_id() - p0;
+  const int nbw = wave_max(nb);
   double S = 0, Dx = 0, Dy = 0, Dz = 0;
   double Ex = 0, Ey = 0, Ez = 0;   // per-atom calls: sum of the slots' coefficients of dDeltap_self times their bond vectors
   double w[6] = {0, 0, 0, 0, 0, 0};
@@ -1331,15 +1329,19 @@ __global__ void __launch_bounds__(256) k_dbond(State st) {
       sc = T1 * st.dbop_c[q] + (C1pi * cpi) * st.dlnpi_c[q] + (C1pi2 * cpi2) * st.dlnpi2_c[q];
       dx = st.b_dx[q]; dy = st.b_dy[q]; dz = st.b_dz[q];
     }
-    for (int l = 0; l < L; ++l) {   // slot order; absent slots add exact zeros
-      const double sq = __shfl(Sq, base + l, 64), s = __shfl(sc, base + l, 64);
-      const double ax = __shfl(dx, base + l, 64), ay = __shfl(dy, base + l, 64), az = __shfl(dz, base + l, 64);
-      S += sq;
-      Ex += sq * ax; Ey += sq * ay; Ez += sq * az;
-      Dx += s * ax; Dy += s * ay; Dz += s * az;
-      // a central pair force: gradient c d on this end, virial d (x) c d, half at each end
-      vir_add(w, 0.5 * s, ax, ay, az, ax, ay, az);
-    }
+    auto add = [&](auto lc) {   // slot order; absent slots add exact zeros
+      constexpr int l = decltype(lc)::value;
+      if constexpr (l < L) {
+        const double sq = group_lane<L, l>(Sq), s = group_lane<L, l>(sc);
+        const double ax = group_lane<L, l>(dx), ay = group_lane<L, l>(dy), az = group_lane<L, l>(dz);
+        S += sq;
+        Ex += sq * ax; Ey += sq * ay; Ez += sq * az;
+        Dx += s * ax; Dy += s * ay; Dz += s * az;
+        // a central pair force: gradient c d on this end, virial d (x) c d, half at each end
+        vir_add(w, 0.5 * s, ax, ay, az, ax, ay, az);
+      }
+    };
+    each_lane(add);
   }
   if (!live || p0 != 0) return;
   for (int c = 0; c < 6; ++c) st.vb[(size_t)c * n + i] += w[c];

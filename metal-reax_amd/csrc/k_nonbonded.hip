@@ -168,18 +168,19 @@ template <> struct NbPrec<true> {
 // wave sums in a fixed butterfly order, then lane 0 stores the atom's gradient, energies and virial
 template <bool D>
 __device__ inline void nb_finish(const State& st, const Tables& t, int i, int ti, int lane, const NbAcc& a) {
-  double gx = wave_sum(a.gx), gy = wave_sum(a.gy), gz = wave_sum(a.gz), ev = wave_sum(a.ev), ee = wave_sum(a.ee);
-  double v0 = wave_sum(a.v[0]), v1 = wave_sum(a.v[1]), v2 = wave_sum(a.v[2]), v3 = wave_sum(a.v[3]), v4 = wave_sum(a.v[4]),
-         v5 = wave_sum(a.v[5]);
-  if (lane == 0) {
-    const int n = st.n;
-    st.gnb_x[i] = gx; st.gnb_y[i] = gy; st.gnb_z[i] = gz;
-    st.eatom[T_VDW * n + i] = ev;
-    st.eatom[T_ELE * n + i] = ee;
-    st.eatom[T_POL * n + i] = ti >= 0 ? NbPrec<D>::pol(t.sp[ti], st.q[i]) : 0.0;
-    st.vatom[0 * n + i] = v0; st.vatom[1 * n + i] = v1; st.vatom[2 * n + i] = v2;
-    st.vatom[3 * n + i] = v3; st.vatom[4 * n + i] = v4; st.vatom[5 * n + i] = v5;
-  }
+  // four sums at a time, row r of 16 lanes holding the r-th: its first lane stores it (the arrays' strides are n)
+  const int n = st.n, row = lane >> 4;
+  const bool first = (lane & 15) == 0;
+  const double s0 = wave_sum4_rows(a.gx, a.gy, a.gz, a.ev);
+  const double s1 = wave_sum4_rows(a.ee, a.v[0], a.v[1], a.v[2]);
+  const double s2 = wave_sum4_rows(a.v[3], a.v[4], a.v[5], 0.0);
+  if (!first) return;
+  double* const p0 = row < 2 ? (row == 0 ? st.gnb_x : st.gnb_y) : (row == 2 ? st.gnb_z : st.eatom + T_VDW * n);
+  p0[i] = s0;
+  double* const p1 = row == 0 ? st.eatom + T_ELE * n : st.vatom + (size_t)(row - 1) * n;
+  p1[i] = s1;
+  if (row < 3) st.vatom[(size_t)(3 + row) * n + i] = s2;
+  else st.eatom[T_POL * n + i] = ti >= 0 ? NbPrec<D>::pol(t.sp[ti], st.q[i]) : 0.0;
 }
 
 // Wave per atom over the skin list: the distance test runs on all lanes, pairs within nonb_cut are compacted (list order) into
@@ -436,8 +437,11 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
     }
   }
   if (fill > 0) batch(fill);
-  if (qb.refine) lo_sum = wave_sum(lo_sum);
-  if (fuse) { y0 = wave_sum(y0); y1 = wave_sum(y1); }
+  {
+    double s[3] = {lo_sum, y0, y1};
+    wave_sums<3>(s);
+    lo_sum = s[0]; y0 = s[1]; y1 = s[2];
+  }
   if (lane == 0) {
     qb.cnt[i] = m;
     if (qb.refine) qb.lorow[i] = lo_sum;

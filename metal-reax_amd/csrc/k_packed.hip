@@ -130,7 +130,7 @@ __device__ inline double sys_block_sum(double v, double* sh) {   // every thread
   return s;
 }
 __device__ inline double sys_block_max(double v, double* sh) {
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+  v = wave_max(v);
   __syncthreads();
   if (lane_id() == 0) sh[threadIdx.x / 64] = v;
   __syncthreads();

@@ -147,11 +147,7 @@ __device__ inline double2 row_product(int row, int n, int maxnb, const int* __re
         if (j[u] >= 0) { y0 += h[u] * x[u].x; y1 += h[u] * x[u].y; }
     }
   }
-  for (int off = kRowLanes / 2; off > 0; off >>= 1) {
-    y0 += __shfl_xor(y0, off, 64);
-    y1 += __shfl_xor(y1, off, 64);
-  }
-  return make_double2(y0, y1);
+  return make_double2(group_sum<kRowLanes>(y0), group_sum<kRowLanes>(y1));
 }
 
 // Grid of the product kernels: a multiple of the 8 XCDs. Workgroup b is dispatched to XCD b % 8, so it takes the virtual block
@@ -179,11 +175,7 @@ __global__ void __launch_bounds__(kThreads) k_check_gate(int n, QeqBuffers qb, i
     const double l = qb.lorow[i];
     s2 += l * l * qb.hinv[i];
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    m0 = fmax(m0, __shfl_xor(m0, off, 64));
-    m1 = fmax(m1, __shfl_xor(m1, off, 64));
-    s2 += __shfl_xor(s2, off, 64);
-  }
+  m0 = wave_max(m0); m1 = wave_max(m1); s2 = wave_sum(s2);
   constexpr int kW = kThreads / 64;
   if (lane_id() == 0) { sh[threadIdx.x / 64] = m0; sh[kW + threadIdx.x / 64] = m1; sh[2 * kW + threadIdx.x / 64] = s2; }
   __syncthreads();
@@ -202,11 +194,7 @@ __device__ inline bool check_skippable(QeqBuffers qb, int it, double tol, double
     m1 = fmax(m1, qb.partial_gate[3 * b + 1]);
     s2 += qb.partial_gate[3 * b + 2];
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    m0 = fmax(m0, __shfl_xor(m0, off, 64));
-    m1 = fmax(m1, __shfl_xor(m1, off, 64));
-    s2 += __shfl_xor(s2, off, 64);
-  }
+  m0 = wave_max(m0); m1 = wave_max(m1); s2 = wave_sum(s2);
   constexpr int kW = NT / 64;
   __syncthreads();
   if (lane_id() == 0) { sh[threadIdx.x / 64] = m0; sh[kW + threadIdx.x / 64] = m1; sh[2 * kW + threadIdx.x / 64] = s2; }
