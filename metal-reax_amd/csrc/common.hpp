@@ -439,6 +439,73 @@ __device__ inline T group_lane(T v) {
 // number of set bits of `mask` below this lane
 __device__ inline int lanes_below(unsigned long long mask) { return __popcll(mask & ((1ull << lane_id()) - 1ull)); }
 
+// ---- neighbour list construction -------------------------------------------------------------------------------------------
+// radii squared of the sub-lists built with the skin list: bond candidates, H-bond candidates of donors
+struct SubCut { double rb2, rh2; };
+// what the wave building atom i's lists carries: the atom, its place in the arrays, and the entries so far (wave-uniform counts)
+struct ListRow {
+  int i, ti, role;   // role: the atom's p_hbond (0 without H-bonds)
+  int count = 0, nbc = 0, nhc = 0;
+};
+__device__ inline ListRow list_row(const State& st, const Globals& g, const Tables& t, int i) {
+  ListRow r;
+  r.i = i;
+  r.ti = st.type[i];
+  r.role = r.ti >= 0 && g.hbond_cut > 0 ? t.sp[r.ti].p_hbond : 0;
+  return r;
+}
+// bond and H-bond candidates among the lanes' new entries (entry e of partner j at squared distance d2, type tj), in lane order
+__device__ inline void append_sub(const State& st, const Tables& t, const SubCut& cut, ListRow& r, bool keep, int j, int e, int tj,
+                                  double d2) {
+  const bool typed = keep && r.ti >= 0 && tj >= 0;
+  const bool bk = typed && d2 <= cut.rb2;
+  bool hk = false;   // donors list acceptors; acceptor rows come from the transpose
+  if (typed && r.role == 1 && d2 <= cut.rh2) hk = t.sp[tj].p_hbond == 2;
+  const unsigned long long mb = __ballot(bk), mh = __ballot(hk);
+  if (bk) {
+    const int p = r.nbc + lanes_below(mb);
+    if (p < st.maxbc) { const size_t o = (size_t)r.i * st.maxbc + p; st.bc_j[o] = j; st.bc_s[o] = e; }
+  }
+  if (hk) {
+    const int p = r.nhc + lanes_below(mh);
+    if (p < st.maxhc) { const size_t o = (size_t)r.i * st.maxhc + p; st.hc_j[o] = j; st.hc_s[o] = e; }
+  }
+  r.nbc += __popcll(mb);
+  r.nhc += __popcll(mh);
+}
+// appends the lanes' kept images (partner j shifted by code sc) to the skin list, in lane order; returns their entries
+__device__ inline int append_skin(const State& st, ListRow& r, unsigned long long m, bool keep, int j, int sc) {
+  int e = 0;
+  if (keep) {
+    const int slot = r.count + lanes_below(m);
+    e = canonical_first(r.i, j, sc, st.tag) ? (sc | kCanon) : sc;
+    if (slot < st.maxnb) { const size_t o = (size_t)r.i * st.maxnb + slot; st.nb_j[o] = j; st.nb_s[o] = e; }
+  }
+  r.count += __popcll(m);
+  return e;
+}
+// the same, and the sub-lists with them
+__device__ inline void append_entries(const State& st, const Tables& t, const SubCut& cut, ListRow& r, bool keep, int j, int sc, int tj,
+                                      double d2) {
+  const unsigned long long m = __ballot(keep);
+  if (!m) return;
+  const int e = append_skin(st, r, m, keep, j, sc);
+  append_sub(st, t, cut, r, keep, j, e, tj, d2);
+}
+// the counts of a finished row, and the capacity flags of what did not fit
+__device__ inline void close_skin(const State& st, const ListRow& r) {
+  if (lane_id() != 0) return;
+  st.nb_cnt[r.i] = r.count;
+  if (r.count > st.maxnb) atomicMax(&st.flags[0], r.count);
+}
+__device__ inline void close_sub(const State& st, const ListRow& r) {
+  if (lane_id() != 0) return;
+  st.bc_cnt[r.i] = r.nbc;
+  st.hc_cnt[r.i] = r.nhc;
+  if (r.nbc > st.maxbc) atomicMax(&st.flags[4], r.nbc);
+  if (r.nhc > st.maxhc) atomicMax(&st.flags[5], r.nhc);
+}
+
 // slot p of atom i in the slot-major per-bond arrays
 __device__ inline size_t sl(int p, int i, int n) { return (size_t)p * (size_t)n + (size_t)i; }
 

@@ -747,7 +747,8 @@ struct Engine {
       t0 = timer.begin(PH_NBR);
       launch_fill_int(st.flags, 8, 0, stream);
       if (need_full) launch_pk_nbr(st, d_cells.p, d_sys_start.p, d_ext.p, d_reb.p, rs, stream);
-      launch_sublists(st, g, tab, rb, rh, stream);
+      launch_sublists(st, g, tab, rb, rh, stream);   // of every system, at the current positions
+      launch_acceptor_rows(st, g, tab, stream);
       timer.end(PH_NBR, t0);
       int flags[8];
       HIPCHK(hipMemcpyAsync(flags, st.flags, sizeof(flags), hipMemcpyDeviceToHost, stream));
@@ -927,16 +928,17 @@ struct Engine {
           launch_bin(st, cell, grid, bins, stream);
           if (sort_atoms) {   // atoms into the order of their cells
             permute(bins.sidx);
-            launch_bin_identity(n, bins, stream);
             launch_pos4(st, stream);
             sorted = true;
           }
-          launch_nbr_cells(st, cell, grid, bins, rs, stream);
+          launch_nbr_cells(st, g, tab, cell, grid, bins, sorted, rs, rb, rh, stream);
         } else {
-          launch_nbr_brute(st, cell, sm, rs, stream);
+          launch_nbr_brute(st, g, tab, cell, sm, rs, rb, rh, stream);
         }
+      } else {
+        launch_sublists(st, g, tab, rb, rh, stream);   // a sub-list grew
       }
-      launch_sublists(st, g, tab, rb, rh, stream);
+      launch_acceptor_rows(st, g, tab, stream);
       timer.end(PH_NBR, t0);
       int flags[8];
       if (sorted) HIPCHK(hipMemcpyAsync(perm_h.data(), d_perm.p, n * sizeof(int), hipMemcpyDeviceToHost, stream));

@@ -55,6 +55,7 @@ __global__ void k_pk_wrap(State st, const Cell* cells, const int* reb) {
 // image (from the fractional coordinate difference, in (-1, 1) after the wrap) and the ext[d] images on either side of it along
 // each periodic direction (ext[d] = floor(rs / h_d + 1/2), the most that can reach within rs). Entries in (candidate, image)
 // order, compacted with a ballot; the entry format of the single-system lists (shift code | kCanon).
+// (the image is taken from the listing atom's side, as in the single-system searches; only kept entries need the tags)
 __global__ void __launch_bounds__(256) k_pk_nbr(State st, const Cell* cells, const int* sys_start, const int4* ext, const int* reb,
                                                double rs2) {
   const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -66,16 +67,18 @@ __global__ void __launch_bounds__(256) k_pk_nbr(State st, const Cell* cells, con
   const int4 e = ext[s];
   const int lo = sys_start[s], hi = sys_start[s + 1];
   const double4 pi = st.pos[i];
+  const double4* __restrict__ shv = st.shv + (size_t)pos_sys(pi.w) * st.shv_stride;
   double fi[3];
   for (int d = 0; d < 3; ++d) fi[d] = c.per[d] ? frac_coord(c, d, pi.x, pi.y, pi.z) : 0.0;
-  int count = 0;
-  const size_t base = (size_t)i * st.maxnb;
+  ListRow row;
+  row.i = i;
   for (int j0 = lo; j0 < hi; j0 += 64) {
     const int j = j0 + lane;
     const bool valid = j < hi;
     int k0[3] = {0, 0, 0};
+    double4 pj = pi;
     if (valid) {
-      const double4 pj = st.pos[j];
+      pj = st.pos[j];
       for (int d = 0; d < 3; ++d)
         if (c.per[d]) k0[d] = -(int)rint(frac_coord(c, d, pj.x, pj.y, pj.z) - fi[d]);
     }
@@ -88,24 +91,16 @@ __global__ void __launch_bounds__(256) k_pk_nbr(State st, const Cell* cells, con
           // cannot reach within rs
           const bool in_table = abs(s0) <= st.smx0 && abs(s1) <= st.smx1 && abs(s2) <= st.smx2;
           bool keep = false;
-          int ent = 0;
           if (valid && in_table && !(j == i && sc == 0)) {
-            ent = canonical_first(i, j, sc, st.tag) ? (sc | kCanon) : sc;
-            double ddx, ddy, ddz;
-            keep = pair_dvec_list(st, pi, j, ent, ddx, ddy, ddz) <= rs2;
+            const double4 S = shv[shift_index(st, sc)];
+            const double ex = (pj.x + S.x) - pi.x, ey = (pj.y + S.y) - pi.y, ez = (pj.z + S.z) - pi.z;
+            keep = ex * ex + ey * ey + ez * ez <= rs2;
           }
           const unsigned long long m = __ballot(keep);
-          if (keep) {
-            const int slot = count + lanes_below(m);
-            if (slot < st.maxnb) { st.nb_j[base + slot] = j; st.nb_s[base + slot] = ent; }
-          }
-          count += __popcll(m);
+          if (m) append_skin(st, row, m, keep, j, sc);
         }
   }
-  if (lane == 0) {
-    st.nb_cnt[i] = count;
-    if (count > st.maxnb) atomicMax(&st.flags[0], count);
-  }
+  close_skin(st, row);
 }
 
 __global__ void k_pk_ref(State st, MdBuffers md, const int* reb) {
@@ -255,7 +250,7 @@ void launch_pk_wrap(const State& st, const Cell* cells, const int* reb, hipStrea
   hipLaunchKernelGGL(k_pk_wrap, dim3(nblk(st.n, 256)), dim3(256), 0, s, st, cells, reb);
 }
 void launch_pk_nbr(const State& st, const Cell* cells, const int* sys_start, const int4* ext, const int* reb, double rs, hipStream_t s) {
-  hipLaunchKernelGGL(k_pk_nbr, dim3(nblk((long long)st.n * 64, 256)), dim3(256), 0, s, st, cells, sys_start, ext, reb, rs * rs);
+  hipLaunchKernelGGL(k_pk_nbr, dim3(nblk((long long)st.n * 64, 256)), dim3(256), 0, s, st, cells, sys_start, ext, reb, rs * rs * (1.0 + 1e-12));
 }
 void launch_pk_ref(const State& st, MdBuffers& md, const int* reb, hipStream_t s) {
   hipLaunchKernelGGL(k_pk_ref, dim3(nblk(st.n, 256)), dim3(256), 0, s, st, md, reb);

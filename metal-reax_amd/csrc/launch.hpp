@@ -24,8 +24,13 @@ void launch_wrap(const State& st, const Cell& c, hipStream_t s);
 void launch_fill_int(int* p, int n, int v, hipStream_t s);
 size_t bin_temp_bytes(int n);
 void launch_bin(const State& st, const Cell& c, const BinGrid& g, BinBuffers& b, hipStream_t s);
-void launch_nbr_cells(const State& st, const Cell& c, const BinGrid& g, const BinBuffers& b, double rs, hipStream_t s);
-void launch_nbr_brute(const State& st, const Cell& c, const int sm[3], double rs, hipStream_t s);
+// skin list and sub-lists of every atom (radii rs, rb for bond and rh for H-bond candidates). sorted: the atoms are in the order of
+// their cells, so an atom's key is b.skeys of its index and the order needs no index
+SubCut sub_cut(double rb, double rh);
+void launch_nbr_cells(const State& st, const Globals& gl, const Tables& t, const Cell& c, const BinGrid& g, const BinBuffers& b, bool sorted,
+                      double rs, double rb, double rh, hipStream_t s);
+void launch_nbr_brute(const State& st, const Globals& g, const Tables& t, const Cell& c, const int sm[3], double rs, double rb, double rh,
+                      hipStream_t s);
 void launch_pos4(const State& st, hipStream_t s);                                   // pos = (x, y, z, type)
 struct PermuteSet {   // per-atom arrays moved together by launch_permute
   int n = 0, nd = 0, ni = 0, nl = 0;
@@ -34,10 +39,11 @@ struct PermuteSet {   // per-atom arrays moved together by launch_permute
   long long* l[2];
 };
 void launch_permute(const PermuteSet& ps, const int* src, double* sd, int* si, long long* sl, hipStream_t s);
-void launch_bin_identity(int n, BinBuffers& b, hipStream_t s);
 void launch_positions_in(const State& st, const double* ux, const int* perm, hipStream_t s);
 void launch_shift_table(const Cell& c, double4* shv, const int smx[3], hipStream_t s);
+// the sub-lists of all atoms from the skin list (packed systems, and after a sub-list's capacity grew); the acceptors' rows of the H-bond candidates
 void launch_sublists(const State& st, const Globals& g, const Tables& t, double rb, double rh, hipStream_t s);
+void launch_acceptor_rows(const State& st, const Globals& g, const Tables& t, hipStream_t s);
 
 // ---- bond-order chain and bonded terms (k_bonded.hip)
 void launch_bond_build(Precision p, const State& st, const Cell& c, const Globals& g, const Tables& t, hipStream_t s);
@@ -117,7 +123,8 @@ void launch_pk_qeq_finish(const State& st, QeqBuffers& qb, const PackedQeq& pq, 
 // packed systems: neighbour search, integrator and energy sums per system (k_packed.hip)
 void launch_pk_shift_table(const Cell* cells, int S, double4* shv, const int smx[3], hipStream_t s);
 void launch_pk_wrap(const State& st, const Cell* cells, const int* reb, hipStream_t s);
-void launch_pk_nbr(const State& st, const Cell* cells, const int* sys_start, const int4* ext, const int* reb, double rs, hipStream_t s);
+void launch_pk_nbr(const State& st, const Cell* cells, const int* sys_start, const int4* ext, const int* reb, double rs,
+                   hipStream_t s);   // the skin list only (launch_sublists follows)
 // fuse = 1: also the charge solve's start from the guess in x (launch_qeq_guess before it), finished by launch_qeq_init_fused
 void launch_qeq_build(const State& st, const Cell& c, const Globals& g, const Tables& t, QeqBuffers& qb, int fuse, hipStream_t s);
 inline int qeq_build_blocks(int n) { return (int)(((long long)n * 64 + 255) / 256); }
