@@ -261,7 +261,10 @@ struct Engine {
   hipStream_t sb = nullptr;
   hipEvent_t ev_fork = nullptr, ev_bonded = nullptr, ev_cg = nullptr;
   int* cgf_h = nullptr;      // pinned: packed systems' any-active flags read back per batch
-  double* cgs_h = nullptr;   // pinned: CG scalars and activity flags (the device layout of QeqBuffers::scal) read back per batch
+  // pinned: the CG scalars and activity flags (the device layout of QeqBuffers::scal) and the refinement gate's partials, written
+  // by the kernels themselves
+  double* cgs_h = nullptr;
+  double* gate_h = nullptr;
 
   Engine(int dev) : device(dev) {
     const char* sort_env = std::getenv("RXA_ATOM_SORT");
@@ -298,6 +301,7 @@ struct Engine {
     if (pk_h) (void)hipHostFree(pk_h);
     if (rebany_h) (void)hipHostFree(rebany_h);
     if (cgs_h) (void)hipHostFree(cgs_h);
+    if (gate_h) (void)hipHostFree(gate_h);
     if (sb) (void)hipStreamDestroy(sb);
     if (ev_flags) (void)hipEventDestroy(ev_flags);
     if (ev_disp) (void)hipEventDestroy(ev_disp);
@@ -1102,23 +1106,25 @@ struct Engine {
 
   // ---------------------------------------------------------------------------------------------------------------
   void alloc_qeq_matrix() {
+    qb.stride = row_stride(maxnb);
     qb.narrow = n <= 65535 ? 1 : 0;
-    q_int.alloc(qb.narrow ? (size_t)n : (size_t)n * maxnb + n);
+    const size_t head = ((size_t)n + 31) / 32 * 32;   // the columns start on a 128-byte line
+    q_int.alloc(head + (qb.narrow ? 0 : (size_t)n * qb.stride));
     qb.cnt = q_int.p;
-    qb.col = qb.narrow ? nullptr : q_int.p + n;
-    if (qb.narrow) { q_u16.alloc((size_t)n * maxnb); qb.col16 = q_u16.p; } else { q_u16.release(); qb.col16 = nullptr; }
+    qb.col = qb.narrow ? nullptr : q_int.p + head;
+    if (qb.narrow) { q_u16.alloc((size_t)n * qb.stride); qb.col16 = q_u16.p; } else { q_u16.release(); qb.col16 = nullptr; }
     // FP32 values and their FP32 remainders (mixed / FP32), or FP64 values in the double pool (FP64)
     if (qb.fp32) {
-      q_f32.alloc(2 * (size_t)n * maxnb);
+      q_f32.alloc(2 * (size_t)n * qb.stride);
       qb.val32 = q_f32.p;
-      qb.lo32 = q_f32.p + (size_t)n * maxnb;
+      qb.lo32 = q_f32.p + (size_t)n * qb.stride;
     } else {
       q_f32.release();
       qb.val32 = nullptr;
       qb.lo32 = nullptr;
     }
     q_fp32_alloc = qb.fp32;
-    q_key.alloc((size_t)n * maxnb);
+    q_key.alloc((size_t)n * qb.stride);
     qb.key = q_key.p;
     // val shares the double pool
     alloc_qeq_doubles();
@@ -1127,9 +1133,9 @@ struct Engine {
     // sub-arrays start on 256-byte boundaries (the CG reads (s, t) pairs as 16-byte loads)
     auto rnd = [](size_t k) { return (k + 31) & ~(size_t)31; };
     const size_t nmv = 4 * (size_t)qeq_mv_partials(n), nqb = 4 * (size_t)qeq_build_blocks(n);
-    const size_t nval = qb.fp32 ? 0 : (size_t)n * maxnb;   // FP64 values (FP64 mode only)
+    const size_t nval = qb.fp32 ? 0 : (size_t)n * qb.stride;   // FP64 values (FP64 mode only)
     const size_t sz = (nval ? rnd(nval) : 0) + 3 * rnd(n) + 6 * rnd(2 * (size_t)n) + rnd(4 * kCgBlocks) + 2 * rnd(nmv) + rnd(nqb) +
-                      2 * rnd(4 * (size_t)n) + rnd(n) + rnd(2 * (size_t)n) + rnd(3 * kCgBlocks);
+                      2 * rnd(4 * (size_t)n) + rnd(n) + rnd(2 * (size_t)n);
     std::vector<double> keep;
     const bool had_hist = q_dbl.p && hist_count > 0 && q_dbl_n == n;   // history of the same atoms only
     if (had_hist) {
@@ -1160,7 +1166,6 @@ struct Engine {
     qb.t_hist = take(4 * (size_t)n);
     qb.lorow = take(n);
     qb.x0 = take(2 * (size_t)n);
-    qb.partial_gate = take(3 * kCgBlocks);
     static_assert(2 * sizeof(int) <= sizeof(double), "");
     if (had_hist) {
       h2d(qb.s_hist, keep.data(), 4 * (size_t)n * sizeof(double));
@@ -1253,22 +1258,40 @@ struct Engine {
       cgf_h = nullptr;
       cgs_h = nullptr;
       HIPCHK(hipHostMalloc((void**)&cgf_h, ((size_t)cap + 2) * sizeof(int), hipHostMallocDefault));
-      HIPCHK(hipHostMalloc((void**)&cgs_h, qeq_scal_doubles(cap) * sizeof(double), hipHostMallocDefault));
+      HIPCHK(hipHostMalloc((void**)&cgs_h, qeq_scal_doubles(cap) * sizeof(double), hipHostMallocCoherent));
+      std::memset(cgs_h, 0, qeq_scal_doubles(cap) * sizeof(double));
+      if (!gate_h) HIPCHK(hipHostMalloc((void**)&gate_h, 3 * qeq_gate_partials() * sizeof(double), hipHostMallocCoherent));
       qeq_imax_cap = cap;
     }
     qb.scal = q_scal.p;
+    qb.scal_host = cgs_h;
+    qb.gate_host = gate_h;
     pq.any = d_cg_any.p;
   }
   int cg_guess = 8;
   int cg_it = 0, cg_batch = 0;
-  // refinement: the last batch ended with update(cg_it) and a check of slot cg_it, so the next launch is the product of
-  // iteration cg_it + 1 in its checking form
-  bool cg_checked = false;
+  // refinement: the last batch ended with update(cg_it), so the next launch is the product of iteration cg_it + 1; after a
+  // check (slot cg_it) in the form that takes up its restart flags
+  bool cg_updated = false, cg_checked = false;
   // activity flags, restart records and sig of iteration slot k in the read-back scalars (the layout of QeqBuffers::scal)
   const int* cg_act(int k) const { return reinterpret_cast<const int*>(cgs_h + 8 + kScalSlot * (size_t)k + 2); }
   const int* cg_rst(int k) const { return reinterpret_cast<const int*>(cgs_h + 8 + kScalSlot * (size_t)k + 3); }
   double cg_sig(int k, int sys) const { return cgs_h[8 + kScalSlot * (size_t)k + sys]; }
-  // launches the next batch of iterations, then the asynchronous readback of the flags and scalars (pinned) and its event
+  // Refinement: both systems have stopped (activity of slot cg_it - 1) and the last update left the gate's partials: whether the
+  // bound proves that the true residuals pass, so that the check's product would change nothing
+  bool check_skippable(double tol) const {
+    double m[2] = {0.0, 0.0}, s2 = 0.0;
+    for (int b = 0; b < qeq_gate_partials(); ++b) {
+      m[0] = std::max(m[0], gate_h[3 * b]);
+      m[1] = std::max(m[1], gate_h[3 * b + 1]);
+      s2 += gate_h[3 * b + 2];
+    }
+    const double S = std::sqrt(s2);
+    bool ok = true;
+    for (int s = 0; s < 2; ++s) ok = ok && std::sqrt(cg_sig(cg_it - 1, s)) + m[s] * S <= (1.0 - 1e-3) * tol * cgs_h[s];
+    return ok;
+  }
+  // launches the next batch of iterations and records the event after which the host may read its flags and scalars
   void cg_launch_batch(int imax) {
     if (packed) {   // iteration it sets any[it]: some system active for the next one
       for (int b = 0; b < cg_batch && cg_it < imax; ++b) {
@@ -1289,26 +1312,22 @@ struct Engine {
     }
     for (int b = 0; b < cg_batch && cg_it < imax; ++b) {
       hipEvent_t t0 = timer.begin(PH_QEQ_CG);
-      if (!cg_checked) launch_qeq_update(st, qb, cg_it, stream);
+      if (!cg_updated) launch_qeq_update(st, qb, cg_it, false, stream);
       timer.end(PH_QEQ_CG, t0);
       ++cg_it;
       t0 = timer.begin(PH_QEQ_SPMV);
       if (cg_checked) launch_qeq_mvdir_chk(st, qb, cg_it, imax, cg_tol, stream);
       else launch_qeq_mvdir(st, qb, cg_it, imax, cg_tol, stream);
       timer.end(PH_QEQ_SPMV, t0);
-      cg_checked = false;
+      cg_updated = cg_checked = false;
       bonded_poll();
     }
-    int slots = cg_it;
-    if (qb.refine) {   // close the batch with the update of iteration cg_it and a refinement check in slot cg_it
+    if (qb.refine && !cg_updated) {   // close the batch with the update of iteration cg_it and the gate of a check
       hipEvent_t t0 = timer.begin(PH_QEQ_CG);
-      if (!cg_checked) launch_qeq_update(st, qb, cg_it, stream);
-      launch_qeq_restart(st, qb, cg_it, imax, cg_tol, stream);
+      launch_qeq_update(st, qb, cg_it, true, stream);
       timer.end(PH_QEQ_CG, t0);
-      cg_checked = true;
-      slots = cg_it + 1;
+      cg_updated = true;
     }
-    HIPCHK(hipMemcpyAsync(cgs_h, qb.scal, (8 + kScalSlot * (size_t)slots) * sizeof(double), hipMemcpyDeviceToHost, stream));
     HIPCHK(hipEventRecord(ev_cg, stream));
     ++cg_batches;
   }
@@ -1340,7 +1359,7 @@ struct Engine {
   void cg_start(int imax, double tol) {
     cg_tol = tol;
     cg_it = 1;
-    cg_checked = false;
+    cg_updated = cg_checked = false;
     cg_batch = std::max(1, cg_guess);
     hipEvent_t t0 = timer.begin(PH_QEQ_SPMV);
     launch_qeq_mvdir(st, qb, 1, imax, tol, stream);
@@ -1348,14 +1367,27 @@ struct Engine {
     cg_launch_batch(imax);
   }
   void cg_wait_end(int imax) {
+    bool verified = false;   // refinement: the check's product gave the true residuals (slot cg_it)
     while (true) {
       HIPCHK(hipEventSynchronize(ev_cg));
-      if (qb.refine) {   // done when the batch's check found both true residuals within tol (or the budget is spent)
+      const int* a = cg_act(cg_it - 1);
+      const bool stopped = !a[0] && !a[1];
+      if (!qb.refine) {
+        if (stopped || cg_it >= imax) break;
+      } else if (stopped) {   // done when both true residuals are within tol (or the budget is spent)
+        if (check_skippable(cg_tol)) break;
+        hipEvent_t t0 = timer.begin(PH_QEQ_CG);
+        launch_qeq_restart(st, qb, cg_it, imax, cg_tol, stream);
+        timer.end(PH_QEQ_CG, t0);
+        HIPCHK(hipEventRecord(ev_cg, stream));
+        HIPCHK(hipEventSynchronize(ev_cg));
         const int* r = cg_rst(cg_it);
+        verified = true;
         if ((r[0] == 0 && r[1] == 0) || cg_it >= imax) break;
-      } else {
-        const int* a = cg_act(cg_it - 1);
-        if ((!a[0] && !a[1]) || cg_it >= imax) break;
+        verified = false;
+        cg_checked = true;
+      } else if (cg_it >= imax) {
+        break;
       }
       cg_batch = 2;
       cg_launch_batch(imax);
@@ -1365,7 +1397,7 @@ struct Engine {
       for (int k = 0; k < cg_it; ++k) done += cg_act(k)[s] == 1;
       last_iters[s] = done + 1;   // the stock loop index at exit
       // the relative residual the solve stopped on: the true one of the last check under refinement, else the recursion's
-      last_rel[s] = std::sqrt(qb.refine ? cg_sig(cg_it, s) : cg_sig(last_iters[s] - 1, s)) / cgs_h[s];
+      last_rel[s] = std::sqrt(verified ? cg_sig(cg_it, s) : cg_sig(qb.refine ? cg_it - 1 : last_iters[s] - 1, s)) / cgs_h[s];
     }
     cg_guess = std::max(last_iters[0], last_iters[1]) - 1;
   }

@@ -281,13 +281,13 @@ __device__ inline double pair_dvec_key(const State& st, const double4 pi, const 
 // l + 64, ..., the assignment of the skin-list kernel's compacted batches, so the sums are the same.
 template <bool D, class TC>
 __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tables& t, const TC* __restrict__ col,
-                                    const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int i) {
+                                    const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride, int i) {
   using Q = typename NbPrec<D>::Q;
   const int lane = lane_id();
   const int ti = st.type[i];
   NbAcc a;
   if (ti >= 0) {
-    const size_t base = (size_t)i * st.maxnb;
+    const size_t base = (size_t)i * stride;   // keys in list order, columns as row_slot puts them
     const int cnt = rcnt[i];
     const Q qi = (Q)st.q[i];
     const double4 pi = st.pos[i];
@@ -296,10 +296,10 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
     // two-deep software pipeline as in the matrix build: columns/keys two strides ahead, positions and charges one ahead
     // (lanes past the row's end carry the row atom itself and key 0, valid indices never used)
     int jB = i, kyB = 0, jC = i, kyC = 0;
-    if (lane < cnt) { jC = (int)col[base + lane]; kyC = key[base + lane]; }
+    if (lane < cnt) { jC = (int)col[base + row_slot(lane, cnt)]; kyC = key[base + lane]; }
     double4 pC = st.pos[jC];
     Q qC = (Q)st.q[jC];
-    if (lane + 64 < cnt) { jB = (int)col[base + lane + 64]; kyB = key[base + lane + 64]; }
+    if (lane + 64 < cnt) { jB = (int)col[base + row_slot(lane + 64, cnt)]; kyB = key[base + lane + 64]; }
     for (int k = lane; k < cnt; k += 64) {
       const double4 pj = pC;
       const Q qj = qC;
@@ -308,7 +308,7 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
       pC = st.pos[jC];
       qC = (Q)st.q[jC];
       jB = i; kyB = 0;
-      if (k + 128 < cnt) { jB = (int)col[base + k + 128]; kyB = key[base + k + 128]; }
+      if (k + 128 < cnt) { jB = (int)col[base + row_slot(k + 128, cnt)]; kyB = key[base + k + 128]; }
       double dx, dy, dz;
       const double r2 = pair_dvec_key(st, pi, pj, ky, dx, dy, dz);
       if (r2 <= cut2) {
@@ -323,18 +323,18 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
 // (5 waves per SIMD: 96 VGPRs without spills; the compiler's choice, 106 VGPRs and 4 waves, is slower)
 template <class TC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_nonbonded_rows(State st, Globals g, Tables t, const TC* __restrict__ col,
-                                                        const unsigned short* __restrict__ key, const int* __restrict__ rcnt) {
+                                                        const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
   const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   if (i >= st.n) return;
-  nb_rows_wave<false, TC>(st, g, t, col, key, rcnt, i);
+  nb_rows_wave<false, TC>(st, g, t, col, key, rcnt, stride, i);
 }
 
 template <class TC>
 __global__ void __launch_bounds__(256) k_nonbonded_rows_d(State st, Globals g, Tables t, const TC* __restrict__ col,
-                                                          const unsigned short* __restrict__ key, const int* __restrict__ rcnt) {
+                                                          const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
   const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   if (i >= st.n) return;
-  nb_rows_wave<true, TC>(st, g, t, col, key, rcnt, i);
+  nb_rows_wave<true, TC>(st, g, t, col, key, rcnt, stride, i);
 }
 
 constexpr int kQbWaves = 4, kQbRing = 128;
@@ -351,7 +351,7 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
                                      int* rj, int* rk, double* rr, double (&acc)[4]) {
   const int lane = lane_id();
   const int ti = st.type[i];
-  const size_t base = (size_t)i * st.maxnb;
+  const size_t base = (size_t)i * st.maxnb, rbase = (size_t)i * qb.stride;
   const int cnt = ti >= 0 ? min(st.nb_cnt[i], st.maxnb) : 0;
   const double swb2 = g.q_swb * g.q_swb;
   const double* T = g.qtap;
@@ -370,7 +370,7 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
       double Tap = T[7] * r + T[6];
       Tap = Tap * r + T[5]; Tap = Tap * r + T[4]; Tap = Tap * r + T[3]; Tap = Tap * r + T[2]; Tap = Tap * r + T[1]; Tap = Tap * r + T[0];
       const double h = (Tap * 14.4) * rcbrt_f64(r * r * r + shld[kt >> 16]);
-      const size_t o = base + m + lane;
+      const size_t o = rbase + m + (count == kRowGroup ? group_slot(lane) : lane);   // row_slot: m counts full groups
       if (qb.narrow) qb.col16[o] = (unsigned short)j; else qb.col[o] = j;
       double hv = h;   // the value the start's product uses
       if (qb.fp32) {
@@ -392,7 +392,7 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
         y0 += hv * xj.x;
         y1 += hv * xj.y;
       }
-      if (qb.keyed) qb.key[o] = (unsigned short)(kt & 0xFFFF);
+      if (qb.keyed) qb.key[rbase + m + lane] = (unsigned short)(kt & 0xFFFF);
     }
     m += count;
   };
@@ -534,11 +534,11 @@ void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals
 void launch_nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
   const dim3 grid(nblk((long long)st.n * 64, 256)), blk(256);
   if (p == Precision::FP64) {
-    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows_d<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt);
-    else hipLaunchKernelGGL(k_nonbonded_rows_d<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt);
+    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows_d<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+    else hipLaunchKernelGGL(k_nonbonded_rows_d<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
   } else {
-    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt);
-    else hipLaunchKernelGGL(k_nonbonded_rows<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt);
+    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+    else hipLaunchKernelGGL(k_nonbonded_rows<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
   }
 }
 

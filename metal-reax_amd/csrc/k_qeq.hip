@@ -34,6 +34,11 @@ inline __host__ __device__ int mv_blocks(int n) { return (n + kMvRowsPerBlock - 
 __device__ inline double& SIG(double* scal, int k, int sys) { return scal[8 + kScalSlot * k + sys]; }
 __device__ inline int* ACT(double* scal, int k) { return reinterpret_cast<int*>(scal + 8 + kScalSlot * k + 2); }
 __device__ inline int* RST(double* scal, int k) { return reinterpret_cast<int*>(scal + 8 + kScalSlot * k + 3); }
+// the kernel that sets a scalar of the solve sets it in the host's copy too (pinned memory, same layout): the host reads it after
+// an event, without a copy on the stream (a copy kernel of 4 us and its dispatch per batch of iterations)
+__device__ inline void put_sig(const QeqBuffers& qb, int k, int sys, double v) { SIG(qb.scal, k, sys) = v; SIG(qb.scal_host, k, sys) = v; }
+__device__ inline void put_act(const QeqBuffers& qb, int k, int sys, int v) { ACT(qb.scal, k)[sys] = v; ACT(qb.scal_host, k)[sys] = v; }
+__device__ inline void put_rst(const QeqBuffers& qb, int k, int sys, int v) { RST(qb.scal, k)[sys] = v; RST(qb.scal_host, k)[sys] = v; }
 
 template <int K, int NT = kThreads>
 __device__ inline void block_reduce(double (&v)[K], double* sh) {
@@ -53,12 +58,34 @@ __device__ inline void block_reduce(double (&v)[K], double* sh) {
 }
 
 // every block re-reduces the `np` partials of a previous launch (K values per block) in the same fixed order: thread t sums
-// partials t, t + NT, ... in sequence, then block_reduce's fixed order
+// partials t, t + NT, ... in sequence, then block_reduce's fixed order. Four partials per thread are in flight at a time (one
+// by one, the 12,000 partials of 192,000 rows are 47 round trips to the L2 in a row): update kernel 28.7 -> 16.1 us per launch at
+// 192,000 atoms, 9.1 -> 7.1 us at 24,000 (its first row loaded ahead too), CG start 61 -> 46 us at 192,000.
+constexpr int kPartInFlight = 4;
+template <int K, int NT = kThreads>
+__device__ inline void thread_partials(const double* part, double (&v)[K], int np) {
+  for (int k = 0; k < K; ++k) v[k] = 0.0;
+  int b = threadIdx.x;
+  double u[kPartInFlight][K];
+  for (; b + (kPartInFlight - 1) * NT < np; b += kPartInFlight * NT) {
+#pragma unroll
+    for (int f = 0; f < kPartInFlight; ++f)
+      for (int k = 0; k < K; ++k) u[f][k] = part[(size_t)(b + f * NT) * K + k];
+#pragma unroll
+    for (int f = 0; f < kPartInFlight; ++f)
+      for (int k = 0; k < K; ++k) v[k] += u[f][k];
+  }
+#pragma unroll
+  for (int f = 0; f < kPartInFlight - 1; ++f)
+    for (int k = 0; k < K; ++k) u[f][k] = b + f * NT < np ? part[(size_t)(b + f * NT) * K + k] : 0.0;
+#pragma unroll
+  for (int f = 0; f < kPartInFlight - 1; ++f)
+    if (b + f * NT < np)
+      for (int k = 0; k < K; ++k) v[k] += u[f][k];
+}
 template <int K, int NT = kThreads>
 __device__ inline void reduce_partials(const double* part, double (&v)[K], double* sh, int np = kCgBlocks) {
-  for (int k = 0; k < K; ++k) v[k] = 0.0;
-  for (int b = threadIdx.x; b < np; b += NT)
-    for (int k = 0; k < K; ++k) v[k] += part[b * K + k];
+  thread_partials<K, NT>(part, v, np);
   block_reduce<K, NT>(v, sh);
 }
 
@@ -86,65 +113,99 @@ __global__ void __launch_bounds__(kThreads) k_cg_guess(int n, QeqBuffers qb, int
   }
 }
 
-// Product layout: kRowLanes lanes per row (64 / kRowLanes rows per wave side by side), each lane keeping kInFlight entries of its
-// row in flight (independent loads) and striding the row by kRowLanes; the row sum is a xor butterfly inside the lane group.
-// Measured on the 24,000-atom water matrix (422 entries per row): 16 lanes x 8 entries is 1.3x faster than one wave per row.
+// Product layout: kRowLanes lanes per row (64 / kRowLanes rows per wave side by side); lane l adds the entries l, l + 16, ... of its
+// row in turn, four of them from one vector load of columns and one of values (row_slot), two such groups in flight; the row sum
+// is a xor butterfly inside the lane group.
 constexpr int kRowLanes = 16;
-constexpr int kInFlight = 8;
+constexpr int kRowGroups = 2;   // groups of 64 entries in flight
 
 // Matrix value accessors: FP64 values, FP32 values, or the two-float pair hi + lo (FP64 to about 48 bits) of the refinement's
-// residuals. Products and sums are FP64 in every case.
+// residuals. Raw: a value as stored, kept in that form until it is used; four: a lane's four values of a full group, side by
+// side. Products and sums are FP64 in every case.
 struct ValD {
+  using Raw = double;
   const double* v;
-  __device__ double operator()(size_t k) const { return v[k]; }
+  __device__ Raw one(size_t o) const { return v[o]; }
+  __device__ void four(size_t o, Raw (&h)[4]) const {
+    const double2* p = reinterpret_cast<const double2*>(v + o);
+    const double2 a = p[0], b = p[1];
+    h[0] = a.x; h[1] = a.y; h[2] = b.x; h[3] = b.y;
+  }
+  static __device__ Raw zero() { return 0.0; }
+  static __device__ double wide(Raw r) { return r; }
 };
 struct ValF {
+  using Raw = float;
   const float* v;
-  __device__ double operator()(size_t k) const { return (double)v[k]; }
+  __device__ Raw one(size_t o) const { return v[o]; }
+  __device__ void four(size_t o, Raw (&h)[4]) const {
+    const float4 a = *reinterpret_cast<const float4*>(v + o);
+    h[0] = a.x; h[1] = a.y; h[2] = a.z; h[3] = a.w;
+  }
+  static __device__ Raw zero() { return 0.0f; }
+  static __device__ double wide(Raw r) { return (double)r; }
 };
 struct ValDS {
+  struct Raw { float hi, lo; };
   const float* hi;
   const float* lo;
-  __device__ double operator()(size_t k) const { return (double)hi[k] + (double)lo[k]; }
+  __device__ Raw one(size_t o) const { return {hi[o], lo[o]}; }
+  __device__ void four(size_t o, Raw (&h)[4]) const {
+    const float4 a = *reinterpret_cast<const float4*>(hi + o), b = *reinterpret_cast<const float4*>(lo + o);
+    h[0] = {a.x, b.x}; h[1] = {a.y, b.y}; h[2] = {a.z, b.z}; h[3] = {a.w, b.w};
+  }
+  static __device__ Raw zero() { return {0.0f, 0.0f}; }
+  static __device__ double wide(Raw r) { return (double)r.hi + (double)r.lo; }
 };
+__device__ inline void four_columns(const unsigned short* p, int (&j)[4]) {
+  const ushort4 c = *reinterpret_cast<const ushort4*>(p);
+  j[0] = c.x; j[1] = c.y; j[2] = c.z; j[3] = c.w;
+}
+__device__ inline void four_columns(const int* p, int (&j)[4]) {
+  const int4 c = *reinterpret_cast<const int4*>(p);
+  j[0] = c.x; j[1] = c.y; j[2] = c.z; j[3] = c.w;
+}
 
 // (H v)_row for both systems (v interleaved), off-diagonal part, summed over the row's lane group (all its lanes get the sum);
-// rows >= n give zero. Columns 32 or 16 bits (TC).
+// rows >= n give zero. Columns 32 or 16 bits (TC). Places past the row's end take the row's own column and value 0: they add
+// exact zeros. Bound by the gathers of v (16 bytes per entry through the L1) and the matrix stream: per product launch (HIP
+// events) 24,000 water rows of 422 entries 19.1 us, 192,000 rows with 32-bit columns 164 us (4.0 TB/s of matrix); with one
+// entry per load 20.3 and 172 us. Groups in flight: 1 gives 19.9 and 179 us, 4 gives 22.2 and 174 us (occupancy).
 template <class VA, class TC>
-__device__ inline double2 row_product(int row, int n, int maxnb, const int* __restrict__ cnt, const TC* __restrict__ col,
+__device__ inline double2 row_product(int row, int n, int stride, const int* __restrict__ cnt, const TC* __restrict__ col,
                                       const VA val, const double2* __restrict__ v2) {
-  const int li = lane_id() % kRowLanes;
   double y0 = 0, y1 = 0;
   if (row < n) {
-    const size_t base = (size_t)row * maxnb;
-    const int c = cnt[row];
-    int k = li;
-    for (; k + (kInFlight - 1) * kRowLanes < c; k += kInFlight * kRowLanes) {
-      int j[kInFlight];
-      double h[kInFlight];
-      double2 x[kInFlight];
+    const int li = lane_id() % kRowLanes, c = cnt[row];
+    const size_t base = (size_t)row * stride;
+    for (int k0 = 0; k0 < c; k0 += kRowGroups * kRowGroup) {
+      int j[kRowGroups][4];
+      typename VA::Raw h[kRowGroups][4];
+      double2 x[kRowGroups][4];
 #pragma unroll
-      for (int u = 0; u < kInFlight; ++u) { j[u] = col[base + k + u * kRowLanes]; h[u] = val(base + k + u * kRowLanes); }
+      for (int f = 0; f < kRowGroups; ++f) {
+        const int g = k0 + f * kRowGroup;
+        if (g + kRowGroup <= c) {
+          four_columns(col + base + g + 4 * li, j[f]);
+          val.four(base + g + 4 * li, h[f]);
+        } else {   // the row's last entries, in list order
 #pragma unroll
-      for (int u = 0; u < kInFlight; ++u) x[u] = v2[j[u]];
-#pragma unroll
-      for (int u = 0; u < kInFlight; ++u) { y0 += h[u] * x[u].x; y1 += h[u] * x[u].y; }
-    }
-    if (k < c) {   // at most kInFlight - 1 entries left: one more pass with their loads in flight together, same sum order
-      int j[kInFlight];
-      double h[kInFlight];
-      double2 x[kInFlight];
-#pragma unroll
-      for (int u = 0; u < kInFlight; ++u) {
-        const int kk = k + u * kRowLanes;
-        j[u] = kk < c ? (int)col[base + kk] : -1;
-        h[u] = kk < c ? val(base + kk) : 0.0;
+          for (int u = 0; u < 4; ++u) {
+            const int k = g + u * kRowLanes + li;
+            j[f][u] = row;
+            h[f][u] = VA::zero();
+            if (k < c) { j[f][u] = (int)col[base + k]; h[f][u] = val.one(base + k); }
+          }
+        }
       }
 #pragma unroll
-      for (int u = 0; u < kInFlight; ++u) x[u] = j[u] >= 0 ? v2[j[u]] : make_double2(0.0, 0.0);
+      for (int f = 0; f < kRowGroups; ++f)
 #pragma unroll
-      for (int u = 0; u < kInFlight; ++u)
-        if (j[u] >= 0) { y0 += h[u] * x[u].x; y1 += h[u] * x[u].y; }
+        for (int u = 0; u < 4; ++u) x[f][u] = v2[j[f][u]];
+#pragma unroll
+      for (int f = 0; f < kRowGroups; ++f)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { y0 += VA::wide(h[f][u]) * x[f][u].x; y1 += VA::wide(h[f][u]) * x[f][u].y; }
     }
   }
   return make_double2(group_sum<kRowLanes>(y0), group_sum<kRowLanes>(y1));
@@ -162,70 +223,39 @@ __device__ inline int product_row() { return (int)((mv_vblock() * blockDim.x + t
 // values hi, so its recursive residual is r0 - hi (x - x0) while the true one is b - A x = r0 - A (x - x0): they differ by
 // lo (x - x0), whose M^-1-norm is at most max_j |x_j - x0_j| * S with S^2 = sum_i (sum_j |lo_ij|)^2 / eta_i. When the recursion's
 // sqrt(r.M^-1 r) plus that bound is within tol |b| (with a margin of 1e-3 for the recursion's own FP64 rounding), the true
-// residual passes the stock test and the check's product would change nothing: the check is skipped. k_check_gate leaves per
-// block max |x - x0| of both systems and the partial sum of S^2 (only once both systems stopped, like the check itself).
-__global__ void __launch_bounds__(kThreads) k_check_gate(int n, QeqBuffers qb, int it) {
-  __shared__ double sh[3 * kThreads / 64];
-  const int* a = ACT(qb.scal, it - 1);
-  if (a[0] != 0 || a[1] != 0) return;   // uniform over the grid
+// residual passes the stock test and the check's product would change nothing: the check is skipped. The update kernel that ends
+// a batch leaves, once both systems have stopped, per block max |x - x0| of both systems and the partial sum of S^2 in host
+// memory (gate_partials), where the host takes the decision (check_skippable of the engine) and queues the check only if needed.
+__device__ inline void gate_partials(int n, const QeqBuffers& qb, double* sh) {
   double m0 = 0.0, m1 = 0.0, s2 = 0.0;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += gridDim.x * kThreads) {
+  for (int i = blockIdx.x * kUpdThreads + threadIdx.x; i < n; i += gridDim.x * kUpdThreads) {
     m0 = fmax(m0, fabs(qb.x[2 * i] - qb.x0[2 * i]));
     m1 = fmax(m1, fabs(qb.x[2 * i + 1] - qb.x0[2 * i + 1]));
     const double l = qb.lorow[i];
     s2 += l * l * qb.hinv[i];
   }
   m0 = wave_max(m0); m1 = wave_max(m1); s2 = wave_sum(s2);
-  constexpr int kW = kThreads / 64;
+  constexpr int kW = kUpdThreads / 64;
   if (lane_id() == 0) { sh[threadIdx.x / 64] = m0; sh[kW + threadIdx.x / 64] = m1; sh[2 * kW + threadIdx.x / 64] = s2; }
   __syncthreads();
   if (threadIdx.x == 0) {
     double v[3] = {sh[0], sh[kW], sh[2 * kW]};
     for (int w = 1; w < kW; ++w) { v[0] = fmax(v[0], sh[w]); v[1] = fmax(v[1], sh[kW + w]); v[2] += sh[2 * kW + w]; }
-    for (int k = 0; k < 3; ++k) qb.partial_gate[blockIdx.x * 3 + k] = v[k];
+    for (int k = 0; k < 3; ++k) qb.gate_host[blockIdx.x * 3 + k] = v[k];
   }
-}
-// the check is skipped for both systems (every thread computes the same answer from the gate's partials, in a fixed order)
-template <int NT>
-__device__ inline bool check_skippable(QeqBuffers qb, int it, double tol, double* sh) {
-  double m0 = 0.0, m1 = 0.0, s2 = 0.0;
-  for (int b = threadIdx.x; b < kCgBlocks; b += NT) {
-    m0 = fmax(m0, qb.partial_gate[3 * b]);
-    m1 = fmax(m1, qb.partial_gate[3 * b + 1]);
-    s2 += qb.partial_gate[3 * b + 2];
-  }
-  m0 = wave_max(m0); m1 = wave_max(m1); s2 = wave_sum(s2);
-  constexpr int kW = NT / 64;
-  __syncthreads();
-  if (lane_id() == 0) { sh[threadIdx.x / 64] = m0; sh[kW + threadIdx.x / 64] = m1; sh[2 * kW + threadIdx.x / 64] = s2; }
-  __syncthreads();
-  double v[3] = {sh[0], sh[kW], sh[2 * kW]};
-  for (int w = 1; w < kW; ++w) { v[0] = fmax(v[0], sh[w]); v[1] = fmax(v[1], sh[kW + w]); v[2] += sh[2 * kW + w]; }
-  __syncthreads();
-  const double S = sqrt(v[2]);
-  bool ok = true;
-  for (int s = 0; s < 2; ++s) ok = ok && sqrt(SIG(qb.scal, it - 1, s)) + v[s] * S <= (1.0 - 1e-3) * tol * qb.scal[s];
-  return ok;
 }
 
 // w = (diag(eta) + H) v for both systems. kMode 0 writes w. kMode 1 (CG start) and 2 (refinement check) fuse the start in: the
 // row's owner writes r = b - w and p = r / eta instead of w, and each block leaves the partials of b.b and r.p of its rows
-// (1: partial_mv, 2: partial_rs). kMode 2 runs only when neither system is active in iteration `it` (activity slot it - 1): the
-// check waits until both systems have stopped and otherwise leaves the iteration's vectors alone.
+// (1: partial_mv, 2: partial_rs). kMode 2 is queued only once both systems have stopped.
 template <class VA, class TC, int kMode>
-__global__ void __launch_bounds__(kMvThreads) k_spmv2(int n, int maxnb, const int* __restrict__ cnt, const TC* __restrict__ col,
+__global__ void __launch_bounds__(kMvThreads) k_spmv2(int n, int stride, const int* __restrict__ cnt, const TC* __restrict__ col,
                                                      const VA val, const double* __restrict__ eta, const double* v, double* w,
-                                                     QeqBuffers qb, int it, double tol) {
-  if (kMode == 2) {
-    const int* a = ACT(qb.scal, it - 1);
-    if (a[0] != 0 || a[1] != 0) return;   // uniform over the grid
-    __shared__ double shg[3 * kMvThreads / 64];
-    if (check_skippable<kMvThreads>(qb, it, tol, shg)) return;   // uniform: the bound already passes both systems
-  }
+                                                     QeqBuffers qb) {
   const double2* __restrict__ v2 = reinterpret_cast<const double2*>(v);
   double2* w2 = reinterpret_cast<double2*>(w);
   const int i = product_row();
-  const double2 y = row_product<VA, TC>(i, n, maxnb, cnt, col, val, v2);
+  const double2 y = row_product<VA, TC>(i, n, stride, cnt, col, val, v2);
   double acc[4] = {0, 0, 0, 0};
   if (i < n && lane_id() % kRowLanes == 0) {
     const double2 xi = v2[i];
@@ -266,10 +296,13 @@ __global__ void __launch_bounds__(kMvThreads) k_spmv2(int n, int maxnb, const in
 // chk = 1: a refinement check ran before this launch (after update(it - 1)); if it restarted the solve (its record in slot
 // it - 1 is not the marker -1), iteration it starts afresh from the true residual (beta 0, activity from the record), else the
 // iteration continues as usual.
+// The previous update's partials and the activity flags are loaded together at the start, the row's own vector entries before the
+// walk, and lanes 0 and 8 of a row's group finish one system each.
 template <class VA, class TC>
-__global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int maxnb, const TC* __restrict__ col, const VA val, QeqBuffers qb,
+__global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, const TC* __restrict__ col, const VA val, QeqBuffers qb,
                                                         int it, int imax, double tol, int chk) {
   __shared__ double sh[2 * kMvThreads / 64];
+  const int i = product_row();
   int act[2];
   double beta[2] = {0.0, 0.0};
   bool fresh = it == 1;
@@ -278,46 +311,49 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int maxnb, const
   } else if (chk && RST(qb.scal, it - 1)[0] >= 0) {
     fresh = true;
     act[0] = RST(qb.scal, it - 1)[0]; act[1] = RST(qb.scal, it - 1)[1];
-    if (blockIdx.x == 0 && threadIdx.x == 0) { ACT(qb.scal, it - 1)[0] = act[0]; ACT(qb.scal, it - 1)[1] = act[1]; }
+    if (blockIdx.x == 0 && threadIdx.x == 0) { put_act(qb, it - 1, 0, act[0]); put_act(qb, it - 1, 1, act[1]); }
   } else {
+    double sn[2];
+    thread_partials<2, kMvThreads>(qb.partial + 2 * kCgBlocks, sn, kUpdBlocks);
     const int* pa = ACT(qb.scal, it - 2);
     const int pact[2] = {pa[0], pa[1]};
+    const double sp[2] = {SIG(qb.scal, it - 2, 0), SIG(qb.scal, it - 2, 1)};
     if (!pact[0] && !pact[1]) {   // both stopped before: nothing to reduce, the slots of it - 1 carry the last values on
       if (blockIdx.x == 0 && threadIdx.x == 0)
-        for (int s = 0; s < 2; ++s) { SIG(qb.scal, it - 1, s) = SIG(qb.scal, it - 2, s); ACT(qb.scal, it - 1)[s] = 0; }
+        for (int s = 0; s < 2; ++s) { put_sig(qb, it - 1, s, sp[s]); put_act(qb, it - 1, s, 0); }
       return;
     }
-    double sn[2];
-    reduce_partials<2, kMvThreads>(qb.partial + 2 * kCgBlocks, sn, sh, kUpdBlocks);
+    block_reduce<2, kMvThreads>(sn, sh);
     for (int s = 0; s < 2; ++s) {
       act[s] = pact[s] && it < imax && sqrt(sn[s]) / qb.scal[s] > tol ? 1 : 0;
-      if (pact[s]) beta[s] = sn[s] / SIG(qb.scal, it - 2, s);
+      if (pact[s]) beta[s] = sn[s] / sp[s];
     }
     if (blockIdx.x == 0 && threadIdx.x == 0)
       for (int s = 0; s < 2; ++s) {
-        SIG(qb.scal, it - 1, s) = pact[s] ? sn[s] : SIG(qb.scal, it - 2, s);
-        ACT(qb.scal, it - 1)[s] = act[s];
+        put_sig(qb, it - 1, s, pact[s] ? sn[s] : sp[s]);
+        put_act(qb, it - 1, s, act[s]);
       }
   }
   if (!act[0] && !act[1]) return;
-  const double2* __restrict__ p2 = reinterpret_cast<const double2*>(qb.p);
-  const int i = product_row();
-  const double2 y = row_product<VA, TC>(i, n, maxnb, qb.cnt, col, val, p2);
+  const int li = lane_id() % kRowLanes, s = li / (kRowLanes / 2), k = 2 * i + s;   // this lane's system
+  const bool mine = i < n && li % (kRowLanes / 2) == 0 && act[s];
+  double p = 0, e = 0, d = 0, q = 0;
+  if (mine) {
+    p = qb.p[k];
+    e = qb.eta[i];
+    if (!fresh) { d = qb.d[k]; q = qb.q[k]; }
+  }
+  const double2 y = row_product<VA, TC>(i, n, stride, qb.cnt, col, val, reinterpret_cast<const double2*>(qb.p));
   double dq[2] = {0.0, 0.0};
-  if (i < n && lane_id() % kRowLanes == 0) {
-    const double2 pi = p2[i];
-    const double ei = qb.eta[i];
-    const double w[2] = {y.x + ei * pi.x, y.y + ei * pi.y}, pv[2] = {pi.x, pi.y};
-    for (int s = 0; s < 2; ++s) {
-      if (!act[s]) continue;
-      const int k = 2 * i + s;
-      if (fresh && it > 1) qb.x0[k] = qb.x[k];   // a restart: the correction is measured from here
-      const double d = fresh ? pv[s] : pv[s] + beta[s] * qb.d[k];
-      const double q = fresh ? w[s] : w[s] + beta[s] * qb.q[k];
-      qb.d[k] = d;
-      qb.q[k] = q;
-      dq[s] = d * q;
-    }
+  if (mine) {
+    const double w = (s ? y.y : y.x) + e * p;
+    if (fresh && it > 1) qb.x0[k] = qb.x[k];   // a restart: the correction is measured from here
+    const double b = beta[s];
+    d = fresh ? p : p + b * d;
+    q = fresh ? w : w + b * q;
+    qb.d[k] = d;
+    qb.q[k] = q;
+    dq[s] = d * q;
   }
   block_reduce<2, kMvThreads>(dq, sh);
   if (threadIdx.x == 0 && mv_vblock() < mv_blocks(n)) { qb.partial_mv[mv_vblock() * 2] = dq[0]; qb.partial_mv[mv_vblock() * 2 + 1] = dq[1]; }
@@ -325,14 +361,18 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int maxnb, const
 
 // single-vector matvec (the fix's sparse_matvec), owned rows
 template <class VA, class TC>
-__global__ void __launch_bounds__(kThreads) k_spmv1(int n, int maxnb, const int* cnt, const TC* col, const VA val, const double* eta,
+__global__ void __launch_bounds__(kThreads) k_spmv1(int n, int stride, const int* cnt, const TC* col, const VA val, const double* eta,
                                                    const double* v, double* w) {
   const int lane = lane_id();
   const int i = (blockIdx.x * kThreads + threadIdx.x) >> 6;
   if (i >= n) return;
-  const size_t base = (size_t)i * maxnb;
+  const size_t base = (size_t)i * stride;
+  const int c = cnt[i];
   double y = 0;
-  for (int k = lane; k < cnt[i]; k += 64) y += val(base + k) * v[col[base + k]];
+  for (int k = lane; k < c; k += 64) {
+    const size_t o = base + row_slot(k, c);
+    y += VA::wide(val.one(o)) * v[col[o]];
+  }
   y = wave_sum(y);
   if (lane == 0) w[i] = y + eta[i] * v[i];
 }
@@ -346,65 +386,71 @@ __global__ void __launch_bounds__(NT) k_cg_init_fin(QeqBuffers qb, const double*
     for (int s = 0; s < 2; ++s) {
       const double bn = sqrt(v[s]);
       qb.scal[s] = bn;
-      SIG(qb.scal, 0, s) = v[2 + s];
-      ACT(qb.scal, 0)[s] = (1 < imax && sqrt(v[2 + s]) / bn > tol) ? 1 : 0;
+      qb.scal_host[s] = bn;
+      put_sig(qb, 0, s, v[2 + s]);
+      put_act(qb, 0, s, (1 < imax && sqrt(v[2 + s]) / bn > tol) ? 1 : 0);
     }
   }
 }
 
-// End of a refinement check (after update(it)): if either system was active in iteration it, the marker -1 (the iteration
-// continues); else the true residual's r.p gives sig of slot it and each system's restart flag for iteration it + 1 (the stock
-// condition with the true residual: it + 1 < imax and sqrt(r.M^-1 r)/|b| > tol).
+// End of a refinement check (both systems stopped before iteration it): the true residual's r.p gives sig of slot it and each
+// system's restart flag for iteration it + 1 (the stock condition with the true residual: it + 1 < imax and
+// sqrt(r.M^-1 r)/|b| > tol).
 __global__ void __launch_bounds__(kThreads) k_cg_check_fin(QeqBuffers qb, int nparts, int it, int imax, double tol) {
   __shared__ double sh[4 * kThreads / 64];
-  const int* pa = ACT(qb.scal, it - 1);
-  int* rs = RST(qb.scal, it);
-  if (pa[0] != 0 || pa[1] != 0) {
-    if (threadIdx.x == 0) { rs[0] = -1; rs[1] = -1; }
-    return;
-  }
-  if (check_skippable<kThreads>(qb, it, tol, sh)) {   // verified by the bound: the recursion's r.M^-1 r stands
-    if (threadIdx.x == 0)
-      for (int s = 0; s < 2; ++s) { SIG(qb.scal, it, s) = SIG(qb.scal, it - 1, s); rs[s] = 0; }
-    return;
-  }
   double v[4];
   reduce_partials<4>(qb.partial_rs, v, sh, nparts);
   if (threadIdx.x == 0) {
+    int restart = 0;
     for (int s = 0; s < 2; ++s) {
       const double bn = sqrt(v[s]);
-      SIG(qb.scal, it, s) = v[2 + s];
-      rs[s] = (it + 1 < imax && sqrt(v[2 + s]) / bn > tol) ? 1 : 0;
+      const int r = (it + 1 < imax && sqrt(v[2 + s]) / bn > tol) ? 1 : 0;
+      put_sig(qb, it, s, v[2 + s]);
+      put_rst(qb, it, s, r);
+      restart |= r;
     }
     // running counts since the scalars were allocated: checks whose product ran, and restarts
     qb.scal[4] += 1.0;
-    if (rs[0] || rs[1]) qb.scal[5] += 1.0;
+    if (restart) qb.scal[5] += 1.0;
+    qb.scal_host[4] = qb.scal[4];
+    qb.scal_host[5] = qb.scal[5];
   }
 }
 
 // x += alpha d, r -= alpha q, p = r / eta, partial r.p   (iteration it >= 1); few large blocks, since every block first
-// re-reduces all partials of the product
-__global__ void __launch_bounds__(kUpdThreads) k_cg_update(int n, QeqBuffers qb, int it) {
-  __shared__ double sh[2 * kUpdThreads / 64];
+// re-reduces all partials of the product. A thread's first row (the only one up to 61,440 atoms) is loaded before that. gate: the
+// update that ends a batch under refinement (gate_partials above).
+__global__ void __launch_bounds__(kUpdThreads) k_cg_update(int n, QeqBuffers qb, int it, int gate) {
+  __shared__ double sh[3 * kUpdThreads / 64];
+  const double2* const x2 = reinterpret_cast<const double2*>(qb.x);
+  const double2* const r2 = reinterpret_cast<const double2*>(qb.r);
+  const double2* const d2 = reinterpret_cast<const double2*>(qb.d);
+  const double2* const q2 = reinterpret_cast<const double2*>(qb.q);
+  int i = blockIdx.x * kUpdThreads + threadIdx.x;
+  double2 x, r, d, q;
+  double hi = 0;
+  x = r = d = q = make_double2(0.0, 0.0);
+  auto load = [&]() { x = x2[i]; r = r2[i]; d = d2[i]; q = q2[i]; hi = qb.hinv[i]; };
+  if (i < n) load();
+  double dq[2];
+  thread_partials<2, kUpdThreads>(qb.partial_mv, dq, mv_blocks(n));
   const int* act = ACT(qb.scal, it - 1);
   const int a[2] = {act[0], act[1]};
-  if (!a[0] && !a[1]) return;
-  double dq[2];
-  reduce_partials<2, kUpdThreads>(qb.partial_mv, dq, sh, mv_blocks(n));
+  const double sg[2] = {SIG(qb.scal, it - 1, 0), SIG(qb.scal, it - 1, 1)};
+  if (!a[0] && !a[1]) {
+    if (gate) gate_partials(n, qb, sh);
+    return;
+  }
+  block_reduce<2, kUpdThreads>(dq, sh);
   double alpha[2];
-  for (int s = 0; s < 2; ++s) alpha[s] = a[s] ? SIG(qb.scal, it - 1, s) / dq[s] : 0.0;
+  for (int s = 0; s < 2; ++s) alpha[s] = a[s] ? sg[s] / dq[s] : 0.0;
   double acc[2] = {0, 0};
-  for (int i = blockIdx.x * kUpdThreads + threadIdx.x; i < n; i += gridDim.x * kUpdThreads) {
-    const double hi = qb.hinv[i];
-    for (int s = 0; s < 2; ++s) {
-      if (!a[s]) continue;
-      const int k = 2 * i + s;
-      qb.x[k] += alpha[s] * qb.d[k];
-      qb.r[k] -= alpha[s] * qb.q[k];
-      const double p = qb.r[k] * hi;
-      qb.p[k] = p;
-      acc[s] += qb.r[k] * p;
-    }
+  for (; i < n; ) {
+    double p = 0;
+    if (a[0]) { x.x += alpha[0] * d.x; r.x -= alpha[0] * q.x; p = r.x * hi; acc[0] += r.x * p; qb.x[2 * i] = x.x; qb.r[2 * i] = r.x; qb.p[2 * i] = p; }
+    if (a[1]) { x.y += alpha[1] * d.y; r.y -= alpha[1] * q.y; p = r.y * hi; acc[1] += r.y * p; qb.x[2 * i + 1] = x.y; qb.r[2 * i + 1] = r.y; qb.p[2 * i + 1] = p; }
+    i += gridDim.x * kUpdThreads;
+    if (i < n) load();
   }
   block_reduce<2, kUpdThreads>(acc, sh);
   if (threadIdx.x == 0) { qb.partial[2 * kCgBlocks + blockIdx.x * 2] = acc[0]; qb.partial[2 * kCgBlocks + blockIdx.x * 2 + 1] = acc[1]; }
@@ -505,7 +551,7 @@ __global__ void __launch_bounds__(kSysThreads) k_pk_cg_seg(int kind, int S, cons
 
 // w = (diag(eta) + H) p, d = p + beta d, q = w + beta q and d.q per row of the active solves (iteration it)
 template <class VA, class TC>
-__global__ void __launch_bounds__(kMvThreads) k_pk_cg_mvdir(int n, int maxnb, const TC* __restrict__ col, const VA val, QeqBuffers qb,
+__global__ void __launch_bounds__(kMvThreads) k_pk_cg_mvdir(int n, int stride, const TC* __restrict__ col, const VA val, QeqBuffers qb,
                                                            const int* sysid, const double* pk, const int* pki, double* rowv, int it) {
   const int i = product_row();
   int act[2] = {0, 0}, sy = 0;
@@ -516,7 +562,7 @@ __global__ void __launch_bounds__(kMvThreads) k_pk_cg_mvdir(int n, int maxnb, co
   }
   if (!act[0] && !act[1]) return;   // uniform over the row's lane group
   const double2* __restrict__ p2 = reinterpret_cast<const double2*>(qb.p);
-  const double2 y = row_product<VA, TC>(i, n, maxnb, qb.cnt, col, val, p2);
+  const double2 y = row_product<VA, TC>(i, n, stride, qb.cnt, col, val, p2);
   if (lane_id() % kRowLanes != 0) return;
   const double2 pi = p2[i];
   const double ei = qb.eta[i];
@@ -536,7 +582,7 @@ __global__ void __launch_bounds__(kMvThreads) k_pk_cg_mvdir(int n, int maxnb, co
 // refinement check, rows of the systems with a stopped solve: the true residual r = b - (diag(eta) + H) x with the two-float
 // matrix, p = r / eta and r.p for those solves (the rows of the other solves are left alone)
 template <class TC>
-__global__ void __launch_bounds__(kMvThreads) k_pk_cg_check(int n, int maxnb, const TC* __restrict__ col, const ValDS val, QeqBuffers qb,
+__global__ void __launch_bounds__(kMvThreads) k_pk_cg_check(int n, int stride, const TC* __restrict__ col, const ValDS val, QeqBuffers qb,
                                                            const int* sysid, const int* pki, double* rowv) {
   const int i = product_row();
   int chk[2] = {0, 0};
@@ -547,7 +593,7 @@ __global__ void __launch_bounds__(kMvThreads) k_pk_cg_check(int n, int maxnb, co
   }
   if (!chk[0] && !chk[1]) return;   // uniform over the row's lane group
   const double2* __restrict__ x2 = reinterpret_cast<const double2*>(qb.x);
-  const double2 y = row_product<ValDS, TC>(i, n, maxnb, qb.cnt, col, val, x2);
+  const double2 y = row_product<ValDS, TC>(i, n, stride, qb.cnt, col, val, x2);
   if (lane_id() % kRowLanes != 0) return;
   const double2 xi = x2[i];
   const double ei = qb.eta[i], hi = qb.hinv[i];
@@ -648,10 +694,10 @@ template <class P>
 using col_t = typename std::remove_const<typename std::remove_pointer<P>::type>::type;
 
 template <int kMode>
-void spmv2(int n, int maxnb, QeqBuffers& qb, bool ds, const double* x, double* y, int it, hipStream_t s, double tol = 0.0) {
+void spmv2(int n, QeqBuffers& qb, bool ds, const double* x, double* y, hipStream_t s) {
   with_matrix(qb, ds, [&](auto v, auto col) {
-    hipLaunchKernelGGL((k_spmv2<decltype(v), col_t<decltype(col)>, kMode>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, maxnb, qb.cnt,
-                       col, v, qb.eta, x, y, qb, it, tol);
+    hipLaunchKernelGGL((k_spmv2<decltype(v), col_t<decltype(col)>, kMode>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, qb.stride, qb.cnt,
+                       col, v, qb.eta, x, y, qb);
   });
 }
 
@@ -661,14 +707,14 @@ void launch_qeq_matvec1(const State& st, const QeqBuffers& qb, const double* x, 
   // the fix's sparse_matvec: FP64 values where the engine keeps them (FP64 mode, or the two-float pair under refinement)
   with_matrix(qb, qb.fp32 && qb.refine, [&](auto v, auto col) {
     hipLaunchKernelGGL((k_spmv1<decltype(v), col_t<decltype(col)>>), dim3((st.n * 64 + kThreads - 1) / kThreads), dim3(kThreads), 0, s,
-                       st.n, st.maxnb, qb.cnt, col, v, qb.eta, x, y);
+                       st.n, qb.stride, qb.cnt, col, v, qb.eta, x, y);
   });
 }
 
 void launch_qeq_init(const State& st, QeqBuffers& qb, int imax, double tol, int use_hist, hipStream_t s) {
   const int n = st.n;
   hipLaunchKernelGGL(k_cg_guess, dim3(kCgBlocks), dim3(kThreads), 0, s, n, qb, use_hist);
-  spmv2<1>(n, st.maxnb, qb, qb.fp32 && qb.refine, qb.x, qb.q, 0, s);
+  spmv2<1>(n, qb, qb.fp32 && qb.refine, qb.x, qb.q, s);
   hipLaunchKernelGGL(k_cg_init_fin<kThreads>, dim3(1), dim3(kThreads), 0, s, qb, (const double*)qb.partial_mv, mv_blocks(n), imax, tol);
 }
 
@@ -686,7 +732,7 @@ namespace {
 void mvdir_launch(const State& st, QeqBuffers& qb, int it, int imax, double tol, int chk, hipStream_t s) {
   const int n = st.n;
   with_matrix(qb, false, [&](auto v, auto col) {
-    hipLaunchKernelGGL((k_cg_mvdir<decltype(v), col_t<decltype(col)>>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, st.maxnb, col, v, qb,
+    hipLaunchKernelGGL((k_cg_mvdir<decltype(v), col_t<decltype(col)>>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, qb.stride, col, v, qb,
                        it, imax, tol, chk);
   });
 }
@@ -697,15 +743,16 @@ void launch_qeq_mvdir_chk(const State& st, QeqBuffers& qb, int it, int imax, dou
 
 void launch_qeq_restart(const State& st, QeqBuffers& qb, int it, int imax, double tol, hipStream_t s) {
   const int n = st.n;
-  hipLaunchKernelGGL(k_check_gate, dim3(kCgBlocks), dim3(kThreads), 0, s, n, qb, it);
-  spmv2<2>(n, st.maxnb, qb, true, qb.x, qb.q, it, s, tol);
+  spmv2<2>(n, qb, true, qb.x, qb.q, s);
   hipLaunchKernelGGL(k_cg_check_fin, dim3(1), dim3(kThreads), 0, s, qb, mv_blocks(n), it, imax, tol);
 }
 
 int qeq_mv_partials(int n) { return mv_blocks(n); }
 
-void launch_qeq_update(const State& st, QeqBuffers& qb, int it, hipStream_t s) {
-  hipLaunchKernelGGL(k_cg_update, dim3(kUpdBlocks), dim3(kUpdThreads), 0, s, st.n, qb, it);
+int qeq_gate_partials() { return kUpdBlocks; }
+
+void launch_qeq_update(const State& st, QeqBuffers& qb, int it, bool gate, hipStream_t s) {
+  hipLaunchKernelGGL(k_cg_update, dim3(kUpdBlocks), dim3(kUpdThreads), 0, s, st.n, qb, it, gate ? 1 : 0);
 }
 
 void launch_qeq_finish(const State& st, QeqBuffers& qb, hipStream_t s) {
@@ -717,7 +764,7 @@ void launch_qeq_finish(const State& st, QeqBuffers& qb, hipStream_t s) {
 void launch_pk_qeq_init(const State& st, QeqBuffers& qb, const PackedQeq& pq, int imax, double tol, int use_hist, hipStream_t s) {
   const int n = st.n;
   hipLaunchKernelGGL(k_cg_guess, dim3(kCgBlocks), dim3(kThreads), 0, s, n, qb, use_hist);
-  spmv2<0>(n, st.maxnb, qb, qb.fp32 && qb.refine, qb.x, qb.q, 0, s);
+  spmv2<0>(n, qb, qb.fp32 && qb.refine, qb.x, qb.q, s);
   hipLaunchKernelGGL(k_pk_cg_init, dim3(pk_blocks(n, 256)), dim3(256), 0, s, n, qb, pq.rowv);
   hipLaunchKernelGGL(k_pk_cg_seg, dim3(pq.S), dim3(kSysThreads), 0, s, 0, pq.S, pq.sys_start, pq.rowv, (const double*)qb.x, pq.pk,
                      pq.pki, 0, imax, tol, pq.any);
@@ -726,7 +773,7 @@ void launch_pk_qeq_init(const State& st, QeqBuffers& qb, const PackedQeq& pq, in
 void launch_pk_qeq_iteration(const State& st, QeqBuffers& qb, const PackedQeq& pq, int it, int imax, double tol, hipStream_t s) {
   const int n = st.n;
   with_matrix(qb, false, [&](auto v, auto col) {
-    hipLaunchKernelGGL((k_pk_cg_mvdir<decltype(v), col_t<decltype(col)>>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, st.maxnb, col, v, qb,
+    hipLaunchKernelGGL((k_pk_cg_mvdir<decltype(v), col_t<decltype(col)>>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, qb.stride, col, v, qb,
                        pq.sysid, (const double*)pq.pk, (const int*)pq.pki, pq.rowv, it);
   });
   hipLaunchKernelGGL(k_pk_cg_step, dim3(pq.S), dim3(kStepThreads), 0, s, qb, pq.S, pq.sys_start, pq.pk, pq.pki, (const double*)pq.rowv, it,
@@ -737,10 +784,10 @@ void launch_pk_qeq_restart(const State& st, QeqBuffers& qb, const PackedQeq& pq,
   const int n = st.n;
   const ValDS v{qb.val32, qb.lo32};
   if (qb.narrow)
-    hipLaunchKernelGGL((k_pk_cg_check<unsigned short>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, st.maxnb, (const unsigned short*)qb.col16, v,
+    hipLaunchKernelGGL((k_pk_cg_check<unsigned short>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, qb.stride, (const unsigned short*)qb.col16, v,
                        qb, pq.sysid, (const int*)pq.pki, pq.rowv);
   else
-    hipLaunchKernelGGL((k_pk_cg_check<int>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, st.maxnb, (const int*)qb.col, v, qb, pq.sysid,
+    hipLaunchKernelGGL((k_pk_cg_check<int>), dim3(mv_grid(n)), dim3(kMvThreads), 0, s, n, qb.stride, (const int*)qb.col, v, qb, pq.sysid,
                        (const int*)pq.pki, pq.rowv);
   hipLaunchKernelGGL(k_pk_cg_seg, dim3(pq.S), dim3(kSysThreads), 0, s, 4, pq.S, pq.sys_start, pq.rowv, (const double*)qb.x, pq.pk,
                      pq.pki, it, imax, tol, pq.any);

@@ -61,21 +61,34 @@ void launch_vatom_ref(const State& st, hipStream_t s);   // per-atom virials of 
 // ---- non-bonded terms and the charge-equilibration matrix (k_nonbonded.hip)
 void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals& g, const Tables& t, hipStream_t s);
 
+// Place of the k-th of a charge-matrix row's c entries in the row's storage. A full group of 64 entries puts side by side the four
+// entries k = l, l + 16, l + 32, l + 48 that lane l of the product's 16 lanes per row adds in turn, so the lane reads them as one
+// vector (8 bytes of 16-bit columns, 16 bytes of FP32 values); the last, partly filled group stays in list order, so that a
+// short row is not spread over lines it does not fill. Rows are a multiple of 64 entries apart and start on 128-byte lines.
+constexpr int kRowGroup = 64;
+__host__ __device__ inline int group_slot(int r) { return ((r & 15) << 2) | ((r >> 4) & 3); }
+__host__ __device__ inline int row_slot(int k, int c) {
+  const int g = k & ~(kRowGroup - 1);
+  return g + kRowGroup <= c ? g | group_slot(k) : k;
+}
+inline int row_stride(int maxnb) { return (maxnb + kRowGroup - 1) / kRowGroup * kRowGroup; }
+
 struct QeqBuffers {
+  int stride = 0;            // entries from row to row (row_stride of the skin list's capacity)
   int* cnt = nullptr;        // n: entries per row
-  // the rows are stored in exactly one column format and one value format:
-  int* col = nullptr;               // n * maxnb: column (owned atom index), when narrow == 0
-  unsigned short* col16 = nullptr;  // n * maxnb: the same in 16 bits, when narrow == 1 (n <= 65535)
-  double* val = nullptr;            // n * maxnb: H_ij in FP64 (FP64 mode)
-  float* val32 = nullptr;           // n * maxnb: H_ij in FP32 (mixed and FP32 modes)
-  // n * maxnb: the FP32 remainder H_ij - (double)val32 (written when refine == 1), so that (double)val32 + (double)lo32
+  // the rows are stored in exactly one column format and one value format, entry k of row i at i * stride + row_slot(k, cnt[i]):
+  int* col = nullptr;               // n * stride: column (owned atom index), when narrow == 0
+  unsigned short* col16 = nullptr;  // n * stride: the same in 16 bits, when narrow == 1 (n <= 65535)
+  double* val = nullptr;            // n * stride: H_ij in FP64 (FP64 mode)
+  float* val32 = nullptr;           // n * stride: H_ij in FP32 (mixed and FP32 modes)
+  // n * stride: the FP32 remainder H_ij - (double)val32 (written when refine == 1), so that (double)val32 + (double)lo32
   // carries H_ij to about 48 bits for the FP64 residuals of the iterative refinement
   float* lo32 = nullptr;
   int narrow = 0;
   // FP64 iterative refinement of the FP32-valued solve: initial and verification residuals with the two-float matrix, CG
   // restarted from the true residual while it exceeds the tolerance (mixed mode; FP32 mode with the fix's 'resident' keyword)
   int refine = 0;
-  // n * maxnb: how the pair of each entry is reached from the row's atom, for the non-bonded pass over the same rows: bit 15 set
+  // n * stride (entries in list order): how the pair of each entry is reached from the row's atom, for the non-bonded pass over the same rows: bit 15 set
   // if the row's atom is the pair's canonical end, bits 0-14 the index in the shift-vector table of the lattice shift applied to
   // the canonical end's partner. Written when keyed == 1 (shift table of at most 32768 vectors).
   unsigned short* key = nullptr;
@@ -89,13 +102,14 @@ struct QeqBuffers {
   double* partial_mv;        // 4 * qeq_mv_partials(n): per-block partials of the matrix-vector product
   double* partial_rs;        // 4 * qeq_mv_partials(n): per-block partials of the refinement's verification residual
   double* partial_qb;        // 4 * qeq_build_blocks(n): per-block partials of the solve's start fused into the matrix build
-  // refinement's bound (k_qeq.hip k_check_gate): the FP32 remainders' row sums sum_j |lo_ij| (n), the CG start x0 (2 n, same
-  // layout as x) and the gate's per-block partials (3 * kCgBlocks)
+  // refinement's bound (k_qeq.hip gate_partials): the FP32 remainders' row sums sum_j |lo_ij| (n), the CG start x0 (2 n, same
+  // layout as x) and the gate's per-block partials (3 * qeq_gate_partials(), pinned host memory)
   double* lorow = nullptr;
   double* x0 = nullptr;
-  double* partial_gate = nullptr;
+  double* gate_host = nullptr;
   int fp32 = 0;              // the matrix values are val32 (mixed and FP32 modes) instead of val
   double* scal;              // device scalars and activity flags per iteration (see k_qeq.hip), own allocation sized by imax
+  double* scal_host = nullptr;   // the same in pinned host memory, written by the kernels that set them
   double *s_hist, *t_hist;   // 4 * n each, [k * n + i], k = 0 most recent
 };
 constexpr int kCgBlocks = 256;
@@ -138,10 +152,11 @@ void launch_nonbonded_rows(Precision p, const State& st, const Globals& g, const
 void launch_qeq_matvec1(const State& st, const QeqBuffers& qb, const double* x, double* y, hipStream_t s);
 void launch_qeq_init(const State& st, QeqBuffers& qb, int imax, double tol, int use_hist, hipStream_t s);
 void launch_qeq_mvdir(const State& st, QeqBuffers& qb, int it, int imax, double tol, hipStream_t s);   // beta, d, q = A d, d.q partials
-void launch_qeq_update(const State& st, QeqBuffers& qb, int it, hipStream_t s);                        // alpha, x, r, p, r.p partials
-// refinement check after update(it): if both systems have stopped, the true residual b - (diag(eta) + H) x with the two-float
-// matrix restarts every system whose residual still exceeds tol (slot `it` of the scalars); otherwise it leaves a marker and
-// the next product continues the iteration (launch_qeq_mvdir with chk = 1)
+// alpha, x, r, p, r.p partials; gate: also, when both systems have stopped, the partials of the refinement's bound
+void launch_qeq_update(const State& st, QeqBuffers& qb, int it, bool gate, hipStream_t s);
+int qeq_gate_partials();
+// refinement check when both systems have stopped before iteration it: the true residual b - (diag(eta) + H) x with the two-float
+// matrix and each system's restart flag (slot `it` of the scalars); the next product takes them up (launch_qeq_mvdir_chk)
 void launch_qeq_restart(const State& st, QeqBuffers& qb, int it, int imax, double tol, hipStream_t s);
 void launch_qeq_mvdir_chk(const State& st, QeqBuffers& qb, int it, int imax, double tol, hipStream_t s);
 int qeq_mv_partials(int n);                                                                             // partials per product
