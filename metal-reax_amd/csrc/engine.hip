@@ -224,6 +224,7 @@ struct Engine {
   DBuf<double> q_scal;       // CG scalars and flags per iteration, sized by the iteration cap alone (never reallocated with the
                              // matrix or the per-atom vectors, so growing it cannot invalidate a built matrix)
   bool qeq_ready = false, qeq_h_valid = false;
+  size_t cg_cap_h = 0;       // entries of cgf_h
   int qeq_imax_cap = 0;      // iteration cap the scalars, the packed flags and the pinned readback buffers are sized for
   int q_fp32_alloc = -1;     // value format the matrix arrays were allocated for (qb.fp32 at the time)
   // FP64 iterative refinement of the charge solve: -1 the precision's default (on in mixed mode), 0 off, 1 on (the fix's
@@ -260,7 +261,7 @@ struct Engine {
   int g_mult = 1;   // lanes per atom of the angle kernels: the group size for the largest bond count times this (1 or 2)
   hipStream_t sb = nullptr;
   hipEvent_t ev_fork = nullptr, ev_bonded = nullptr, ev_cg = nullptr;
-  int* cgf_h = nullptr;      // pinned: packed systems' any-active flags read back per batch
+  int* cgf_h = nullptr;      // pinned: packed systems' any-active flags, set by the kernels
   // pinned: the CG scalars and activity flags (the device layout of QeqBuffers::scal) and the refinement gate's partials, written
   // by the kernels themselves
   double* cgs_h = nullptr;
@@ -285,8 +286,8 @@ struct Engine {
     HIPCHK(hipEventCreateWithFlags(&ev_bonded, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&ev_cg, hipEventDisableTiming));
     timer.s = stream;
-    HIPCHK(hipHostMalloc((void**)&flags_h, 8 * sizeof(int), hipHostMallocDefault));
-    HIPCHK(hipHostMalloc((void**)&disp_h, md_disp_partials() * sizeof(double), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&flags_h, 8 * sizeof(int), hipHostMallocCoherent));
+    HIPCHK(hipHostMalloc((void**)&disp_h, md_disp_partials() * sizeof(double), hipHostMallocCoherent));
     HIPCHK(hipEventCreateWithFlags(&ev_flags, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&ev_disp, hipEventDisableTiming));
   }
@@ -611,12 +612,12 @@ struct Engine {
   std::vector<Cell> cells_h;
   std::vector<int> ext_h;
   bool shv_valid = false;
-  DBuf<int> d_sys_start, d_reb, d_rebany, d_pki, d_cg_any;
+  DBuf<int> d_sys_start, d_reb, d_pki;
   DBuf<Cell> d_cells;
   DBuf<int4> d_ext;
   DBuf<double> d_pk, d_rowv, d_nh_pk, d_disp_pk, d_sys_out;
   PackedQeq pq;
-  int* rebany_h = nullptr;   // pinned
+  int* rebany_h = nullptr;   // pinned, set by the displacement kernel
   int* pki_h = nullptr;      // pinned, 4 S
   double* pk_h = nullptr;    // pinned, 10 S
   size_t pk_cap_h = 0;
@@ -685,7 +686,7 @@ struct Engine {
     qeq_h_valid = false;
     if (qeq_ready) alloc_qeq();
     md_ready = false;
-    d_sys_start.alloc(S + 1); d_cells.alloc(S); d_ext.alloc(S); d_reb.alloc(S); d_rebany.alloc(1);
+    d_sys_start.alloc(S + 1); d_cells.alloc(S); d_ext.alloc(S); d_reb.alloc(S);
     d_pk.alloc(10 * (size_t)S); d_pki.alloc(4 * (size_t)S); d_rowv.alloc(4 * (size_t)n); d_nh_pk.alloc(32 * (size_t)S);
     d_disp_pk.alloc(S); d_sys_out.alloc((size_t)S * (kTerms + 6));
     zero(d_pki.p, 4 * (size_t)S * sizeof(int));
@@ -699,7 +700,7 @@ struct Engine {
       HIPCHK(hipHostMalloc((void**)&pk_h, 10 * (size_t)S * sizeof(double), hipHostMallocDefault));
       pk_cap_h = S;
     }
-    if (!rebany_h) HIPCHK(hipHostMalloc((void**)&rebany_h, sizeof(int), hipHostMallocDefault));
+    if (!rebany_h) HIPCHK(hipHostMalloc((void**)&rebany_h, sizeof(int), hipHostMallocCoherent));
     pq.S = S; pq.sys_start = d_sys_start.p; pq.sysid = st.sysid; pq.pk = d_pk.p; pq.pki = d_pki.p; pq.rowv = d_rowv.p;
     ext_h.clear();
     smx[0] = smx[1] = smx[2] = -1;
@@ -987,7 +988,7 @@ struct Engine {
     t0 = timer.begin(PH_BOCORR);
     launch_bo_correct(prec, st, g, tab, b);
     timer.end(PH_BOCORR, t0);
-    HIPCHK(hipMemcpyAsync(flags_h, st.flags, 8 * sizeof(int), hipMemcpyDeviceToHost, b));
+    launch_flags_out(st.flags, flags_h, b);
     HIPCHK(hipEventRecord(ev_flags, b));
     bonded_pending = true;
     t0 = timer.begin(PH_TERMS);
@@ -1252,12 +1253,11 @@ struct Engine {
       const int cap = std::max(imax + 2, 2048);
       q_scal.alloc(qeq_scal_doubles(cap));
       zero(q_scal.p, q_scal.n * sizeof(double));
-      d_cg_any.alloc((size_t)cap + 2);
       if (cgf_h) HIPCHK(hipHostFree(cgf_h));
       if (cgs_h) HIPCHK(hipHostFree(cgs_h));
       cgf_h = nullptr;
       cgs_h = nullptr;
-      HIPCHK(hipHostMalloc((void**)&cgf_h, ((size_t)cap + 2) * sizeof(int), hipHostMallocDefault));
+      HIPCHK(hipHostMalloc((void**)&cgf_h, ((size_t)cap + 2) * sizeof(int), hipHostMallocCoherent));
       HIPCHK(hipHostMalloc((void**)&cgs_h, qeq_scal_doubles(cap) * sizeof(double), hipHostMallocCoherent));
       std::memset(cgs_h, 0, qeq_scal_doubles(cap) * sizeof(double));
       if (!gate_h) HIPCHK(hipHostMalloc((void**)&gate_h, 3 * qeq_gate_partials() * sizeof(double), hipHostMallocCoherent));
@@ -1266,7 +1266,8 @@ struct Engine {
     qb.scal = q_scal.p;
     qb.scal_host = cgs_h;
     qb.gate_host = gate_h;
-    pq.any = d_cg_any.p;
+    pq.any = cgf_h;
+    cg_cap_h = (size_t)qeq_imax_cap + 2;
   }
   int cg_guess = 8;
   int cg_it = 0, cg_batch = 0;
@@ -1306,7 +1307,6 @@ struct Engine {
         launch_pk_qeq_restart(st, qb, pq, cg_it - 1, imax, cg_tol, stream);
         timer.end(PH_QEQ_CG, t0);
       }
-      HIPCHK(hipMemcpyAsync(cgf_h, d_cg_any.p, (size_t)cg_it * sizeof(int), hipMemcpyDeviceToHost, stream));
       HIPCHK(hipEventRecord(ev_cg, stream));
       return;
     }
@@ -1343,7 +1343,9 @@ struct Engine {
     ensure_cg_cap(imax);
     qeq_matrix(true);
     if (packed) {
-      launch_fill_int(d_cg_any.p, (int)d_cg_any.n, 0, stream);
+      if (pk_flags_busy) HIPCHK(hipStreamSynchronize(stream));   // a solve that was left unfinished by an error may still set them
+      pk_flags_busy = true;
+      std::memset(cgf_h, 0, cg_cap_h * sizeof(int));
       launch_pk_qeq_init(st, qb, pq, imax, tol, hist_count > 0 ? 1 : 0, stream);
       cg_tol = tol;
       cg_it = 1;
@@ -1410,7 +1412,9 @@ struct Engine {
     if (packed) {
       while (true) {
         HIPCHK(hipEventSynchronize(ev_cg));
+        pk_flags_busy = false;
         if (!cgf_h[cg_it - 1] || cg_it >= imax) break;
+        pk_flags_busy = true;
         cg_batch = 2;
         cg_launch_batch(imax);
       }
@@ -1418,13 +1422,10 @@ struct Engine {
       for (int k = 0; k < cg_it; ++k) if (cgf_h[k]) done = k + 1;
       cg_guess = std::max(1, done);
       launch_pk_qeq_finish(st, qb, pq, stream);
-      HIPCHK(hipMemcpyAsync(pki_h, d_pki.p, 4 * (size_t)S * sizeof(int), hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipMemcpyAsync(pk_h, d_pk.p, 10 * (size_t)S * sizeof(double), hipMemcpyDeviceToHost, stream));
       hist_count = std::min(hist_count + 1, 4);
       ++qeq_calls;
       pk_collect_pending = true;
       if (strict) {
-        sync();
         pk_collect();
         for (int q = 0; q < 2; ++q)
           if (!(last_rel[q] <= cg_tol))
@@ -1446,11 +1447,15 @@ struct Engine {
     qeq_begin(imax, tol);
     qeq_end(imax, strict);
   }
-  // packed systems: the largest iteration count and relative residual over the systems of the last solve (after a sync)
+  bool pk_flags_busy = false;   // kernels that set cgf_h may be in flight
+  // packed systems: the largest iteration count and relative residual over the systems of the last solve
   bool pk_collect_pending = false;
   void pk_collect() {
     if (!pk_collect_pending) return;
     pk_collect_pending = false;
+    HIPCHK(hipMemcpyAsync(pki_h, d_pki.p, 4 * (size_t)S * sizeof(int), hipMemcpyDeviceToHost, stream));
+    HIPCHK(hipMemcpyAsync(pk_h, d_pk.p, 10 * (size_t)S * sizeof(double), hipMemcpyDeviceToHost, stream));
+    sync();
     for (int q = 0; q < 2; ++q) {
       int it = 0;
       double rel = 0;
@@ -1654,16 +1659,14 @@ struct Engine {
         launch_pk_thermostat(st, md, d_sys_start.p, S, d_nh_pk.p, stream);
         launch_md_half_kick(st, md, dtf, stream);
         launch_md_drift(st, md, md_dt, stream);
-      } else {   // thermostat, half kick, drift and the displacement partials in fused kernels
-        launch_md_step_start(st, md, dtf, md_dt, !md_nve, v_scale_pending, stream);
+      } else {   // thermostat, half kick, drift in fused kernels; per-block largest squared displacements into pinned memory, reduced
+                 // on the host (exact: a maximum)
+        launch_md_step_start(st, md, dtf, md_dt, !md_nve, v_scale_pending, disp_h, stream);
         v_scale_pending = false;
       }
       if (packed) {   // each system's own displacement decides its own rebuild
-        launch_fill_int(d_rebany.p, 1, 0, stream);
-        launch_pk_disp(st, md, d_sys_start.p, S, 0.5 * skin, d_reb.p, d_rebany.p, d_disp_pk.p, stream);
-        HIPCHK(hipMemcpyAsync(rebany_h, d_rebany.p, sizeof(int), hipMemcpyDeviceToHost, stream));
-      } else {   // the kick-drift kernel's per-block largest squared displacements, reduced on the host (exact: a maximum)
-        HIPCHK(hipMemcpyAsync(disp_h, md.partial, md_disp_partials() * sizeof(double), hipMemcpyDeviceToHost, stream));
+        *rebany_h = 0;   // the previous step's event is behind
+        launch_pk_disp(st, md, d_sys_start.p, S, 0.5 * skin, d_reb.p, rebany_h, d_disp_pk.p, stream);
       }
       timer.end(PH_MD, t0);
       HIPCHK(hipEventRecord(ev_disp, stream));

@@ -162,7 +162,7 @@ __global__ void __launch_bounds__(kRT) k_scale_ke(State st, MdBuffers md, int ap
   if (threadIdx.x == 0) md.partial[blockIdx.x] = v;
 }
 
-__global__ void __launch_bounds__(kRT) k_kick_drift(State st, MdBuffers md, double dtf, double dt, int scale) {
+__global__ void __launch_bounds__(kRT) k_kick_drift(State st, MdBuffers md, double dtf, double dt, int scale, double* disp) {
   __shared__ double sh[kRT];
   const double fs = md.nh[19];
   double m = 0;
@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(kRT) k_kick_drift(State st, MdBuffers md, doub
     if (threadIdx.x < s) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) md.partial[blockIdx.x] = sh[0];
+  if (threadIdx.x == 0) disp[blockIdx.x] = sh[0];   // pinned host memory
 }
 
 // the gather (gather_atom) and the velocity half step in one pass: v -= dtf g / m, then the partials of sum m v^2
@@ -212,14 +212,15 @@ inline int nblk(int n, int per) { return (n + per - 1) / per; }
 }  // namespace
 
 // step start: thermostat half step (the pending end-of-step factor applied first), velocity half step, drift, displacement
-void launch_md_step_start(const State& st, MdBuffers& md, double dtf, double dt, bool thermostat, bool pending, hipStream_t s) {
+void launch_md_step_start(const State& st, MdBuffers& md, double dtf, double dt, bool thermostat, bool pending, double* disp,
+                          hipStream_t s) {
   if (thermostat) {
     hipLaunchKernelGGL(k_scale_ke, dim3(kRBlocks), dim3(kRT), 0, s, st, md, pending ? 1 : 0);
     hipLaunchKernelGGL(k_nhc, dim3(1), dim3(kRT), 0, s, md);
   } else if (pending) {
     hipLaunchKernelGGL(k_scale_v, dim3(nblk(st.n, 256)), dim3(256), 0, s, st, md);
   }
-  hipLaunchKernelGGL(k_kick_drift, dim3(kRBlocks), dim3(kRT), 0, s, st, md, dtf, dt, thermostat ? 1 : 0);
+  hipLaunchKernelGGL(k_kick_drift, dim3(kRBlocks), dim3(kRT), 0, s, st, md, dtf, dt, thermostat ? 1 : 0, disp);
 }
 int md_disp_partials() { return kRBlocks; }
 

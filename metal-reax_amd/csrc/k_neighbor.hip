@@ -69,6 +69,10 @@ __global__ void k_fill_int(int* p, int n, int v) {
   if (i < n) p[i] = v;
 }
 
+__global__ void k_flags_out(const int* flags, int* host) {
+  if (threadIdx.x < 8) host[threadIdx.x] = flags[threadIdx.x];
+}
+
 __global__ void k_cell_ranges(int n, const unsigned* skeys, int* cstart, int* cend, unsigned* atom_key, const int* sidx) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
@@ -378,6 +382,10 @@ void launch_acceptor_rows(const State& st, const Globals& g, const Tables& t, hi
 void launch_fill_int(int* p, int n, int v, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_fill_int, dim3(blocks_for(n, 256)), dim3(256), 0, s, p, n, v);
+}
+
+void launch_flags_out(const int* flags, int* host, hipStream_t s) {
+  hipLaunchKernelGGL(k_flags_out, dim3(1), dim3(64), 0, s, flags, host);
 }
 
 size_t bin_temp_bytes(int n) {

@@ -134,7 +134,7 @@ __device__ inline double sys_block_max(double v, double* sh) {
   return m;
 }
 
-// largest displacement since the system's last rebuild; reb[s] = 1 where it exceeds half the skin (any[0] |= 1)
+// largest displacement since the system's last rebuild; reb[s] = 1 where it exceeds half the skin (any[0] = 1, pinned host memory)
 __global__ void __launch_bounds__(kSysThreads) k_pk_disp(State st, MdBuffers md, const int* sys_start, int S, double lim2, int* reb,
                                                         int* any, double* disp) {
   __shared__ double sh[kSysThreads / 64];
@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(kSysThreads) k_pk_disp(State st, MdBuffers md,
     const int r = m > lim2 ? 1 : 0;
     reb[s] = r;
     disp[s] = sqrt(m);
-    if (r) atomicOr(any, 1);
+    if (r) *any = 1;   // every writer writes 1
   }
 }
 

@@ -535,13 +535,13 @@ __global__ void __launch_bounds__(kSysThreads) k_pk_cg_seg(int kind, int S, cons
       q[3] = 0.0;
       a[0] = (1 < imax && sqrt(v[2 + k]) / q[0] > tol) ? 1 : 0;
       a[1] = 1;
-      if (a[0]) atomicOr(any, 1);
+      if (a[0]) any[0] = 1;
     } else if (a[0] == 0) {   // kind 4
       q[1] = v[2 + k];
       if (a[1] < imax && sqrt(v[2 + k]) / q[0] > tol) {
         a[0] = 1;
         q[3] = 0.0;
-        atomicOr(any + it, 1);
+        any[it] = 1;
       } else {
         a[0] = 2;
       }
@@ -611,10 +611,27 @@ __global__ void __launch_bounds__(kMvThreads) k_pk_cg_check(int n, int stride, c
 
 // One CG iteration's scalar and vector steps after the product (iteration it), one block per system: alpha from the system's
 // d.q (the rows' values from k_pk_cg_mvdir), x += alpha d, r -= alpha q, p = r / eta for the system's rows, then the new r.p,
-// beta and the stock stopping test, in one launch. Thread t takes the system's rows t, t + kStepThreads, ..., and the sums
-// follow block_reduce's fixed order, so a system's solve depends only on its own rows. 1024 threads, since one block updates
-// all the system's rows (a lone 9000-atom system: 0.32 ms of CG per step with 256 threads, 0.20 ms with 1024).
-constexpr int kStepThreads = 1024;
+// beta and the stock stopping test, in one launch. The sums are those of 1024 summands per system, summand v taking the
+// system's rows v, v + 1024, ... in turn, then a butterfly over each 64 of them and the 16 results in order, so a system's solve
+// depends only on its own rows. A block of 256 threads holds four summands per thread (loads of the four in flight together): a
+// block of 1024 threads has to wait until one compute unit has 16 waves free beside the bonded kernels (38 us per launch in
+// a pack of 40 systems of 100 to 3000 atoms, beside them; 16 us with 256).
+constexpr int kStepThreads = 256, kStepEach = 4;
+__device__ inline void step_sum(double (&v)[2][kStepEach], double* sh, double (&out)[2]) {
+  constexpr int kW = kStepThreads / 64, kSums = kW * kStepEach;
+  for (int s = 0; s < 2; ++s)
+    for (int u = 0; u < kStepEach; ++u) v[s][u] = wave_sum(v[s][u]);
+  if (lane_id() == 0)
+    for (int s = 0; s < 2; ++s)
+      for (int u = 0; u < kStepEach; ++u) sh[s * kSums + u * kW + threadIdx.x / 64] = v[s][u];
+  __syncthreads();
+  for (int s = 0; s < 2; ++s) {
+    double a = sh[s * kSums];
+    for (int w = 1; w < kSums; ++w) a += sh[s * kSums + w];
+    out[s] = a;
+  }
+  __syncthreads();
+}
 __global__ void __launch_bounds__(kStepThreads) k_pk_cg_step(QeqBuffers qb, int S, const int* sys_start, double* pk, int* pki,
                                                             const double* rowv, int it, int imax, double tol, int* any) {
   const int sy = blockIdx.x;   // one block per system (grid = S)
@@ -622,38 +639,72 @@ __global__ void __launch_bounds__(kStepThreads) k_pk_cg_step(QeqBuffers qb, int 
   double* P = pk + 10 * (size_t)sy;
   int* A = pki + 4 * (size_t)sy;
   const bool act[2] = {A[0] == 1, A[2] == 1};
-  if (!act[0] && !act[1]) return;   // uniform over the block
-  __shared__ double sh[2 * kStepThreads / 64];
   const int a = sys_start[sy], b = sys_start[sy + 1];
-  double v[2] = {0, 0};
-  for (int i = a + threadIdx.x; i < b; i += kStepThreads) { v[0] += rowv[4 * i]; v[1] += rowv[4 * i + 1]; }
-  block_reduce<2, kStepThreads>(v, sh);
-  const double alpha[2] = {act[0] ? P[1] / v[0] : 0.0, act[1] ? P[4 + 1] / v[1] : 0.0};
-  double w[2] = {0, 0};
-  for (int i = a + threadIdx.x; i < b; i += kStepThreads) {
-    const double hi = qb.hinv[i];
-    for (int s = 0; s < 2; ++s) {
-      if (!act[s]) continue;
-      const int k = 2 * i + s;
-      qb.x[k] += alpha[s] * qb.d[k];
-      qb.r[k] -= alpha[s] * qb.q[k];
-      const double p = qb.r[k] * hi;
-      qb.p[k] = p;
-      w[s] += qb.r[k] * p;
+  if (!act[0] && !act[1]) return;   // uniform over the block
+  __shared__ double sh[2 * kStepEach * kStepThreads / 64];
+  const double2* const rv2 = reinterpret_cast<const double2*>(rowv);
+  const double2* const x2 = reinterpret_cast<const double2*>(qb.x);
+  const double2* const r2 = reinterpret_cast<const double2*>(qb.r);
+  const double2* const d2 = reinterpret_cast<const double2*>(qb.d);
+  const double2* const q2 = reinterpret_cast<const double2*>(qb.q);
+  double v[2][kStepEach], t[2];
+  for (int s = 0; s < 2; ++s)
+    for (int u = 0; u < kStepEach; ++u) v[s][u] = 0.0;
+  for (int i0 = a + threadIdx.x; i0 < b; i0 += kStepEach * kStepThreads) {
+    double2 w[kStepEach];
+#pragma unroll
+    for (int u = 0; u < kStepEach; ++u) w[u] = i0 + u * kStepThreads < b ? rv2[2 * (size_t)(i0 + u * kStepThreads)] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < kStepEach; ++u)
+      if (i0 + u * kStepThreads < b) { v[0][u] += w[u].x; v[1][u] += w[u].y; }
+  }
+  step_sum(v, sh, t);
+  const double alpha[2] = {act[0] ? P[1] / t[0] : 0.0, act[1] ? P[4 + 1] / t[1] : 0.0};
+  for (int s = 0; s < 2; ++s)
+    for (int u = 0; u < kStepEach; ++u) v[s][u] = 0.0;
+  for (int i0 = a + threadIdx.x; i0 < b; i0 += kStepEach * kStepThreads) {
+    double2 x[kStepEach], r[kStepEach], d[kStepEach], q[kStepEach];
+    double hi[kStepEach];
+#pragma unroll
+    for (int u = 0; u < kStepEach; ++u) {
+      const int i = min(i0 + u * kStepThreads, b - 1);   // (past the system's end: loaded, not used)
+      x[u] = x2[i]; r[u] = r2[i]; d[u] = d2[i]; q[u] = q2[i];
+      hi[u] = qb.hinv[i];
+    }
+#pragma unroll
+    for (int u = 0; u < kStepEach; ++u) {
+      const int i = i0 + u * kStepThreads;
+      if (i >= b) continue;
+      if (act[0]) {
+        qb.x[2 * i] = x[u].x + alpha[0] * d[u].x;
+        r[u].x -= alpha[0] * q[u].x;
+        const double p = r[u].x * hi[u];
+        qb.r[2 * i] = r[u].x;
+        qb.p[2 * i] = p;
+        v[0][u] += r[u].x * p;
+      }
+      if (act[1]) {
+        qb.x[2 * i + 1] = x[u].y + alpha[1] * d[u].y;
+        r[u].y -= alpha[1] * q[u].y;
+        const double p = r[u].y * hi[u];
+        qb.r[2 * i + 1] = r[u].y;
+        qb.p[2 * i + 1] = p;
+        v[1][u] += r[u].y * p;
+      }
     }
   }
-  block_reduce<2, kStepThreads>(w, sh);
+  step_sum(v, sh, t);
   if (threadIdx.x != 0) return;
   for (int s = 0; s < 2; ++s) {
     if (!act[s]) continue;
     double* q = P + 4 * s;
     int* as = A + 2 * s;
     q[2] = alpha[s];
-    q[3] = w[s] / q[1];
-    q[1] = w[s];
+    q[3] = t[s] / q[1];
+    q[1] = t[s];
     as[1] += 1;
-    as[0] = (as[1] < imax && sqrt(w[s]) / q[0] > tol) ? 1 : 0;
-    if (as[0]) atomicOr(any + it, 1);
+    as[0] = (as[1] < imax && sqrt(t[s]) / q[0] > tol) ? 1 : 0;
+    if (as[0]) any[it] = 1;
   }
 }
 

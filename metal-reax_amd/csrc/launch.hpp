@@ -22,6 +22,7 @@ struct BinBuffers {
 // ---- neighbour search (k_neighbor.hip)
 void launch_wrap(const State& st, const Cell& c, hipStream_t s);
 void launch_fill_int(int* p, int n, int v, hipStream_t s);
+void launch_flags_out(const int* flags, int* host, hipStream_t s);   // the 8 capacity flags into pinned host memory
 size_t bin_temp_bytes(int n);
 void launch_bin(const State& st, const Cell& c, const BinGrid& g, BinBuffers& b, hipStream_t s);
 // skin list and sub-lists of every atom (radii rs, rb for bond and rh for H-bond candidates). sorted: the atoms are in the order of
@@ -126,7 +127,8 @@ struct PackedQeq {
   int* pki = nullptr;               // 4 S: per solve state (1 active, 0 stopped, 2 stopped and verified by the refinement
                                     // check), stock loop index
   double* rowv = nullptr;           // 4 n: per-row d.q and r.p of both solves
-  int* any = nullptr;               // imax + 2: some system active for iteration it + 1 (set by iteration it; [0] by the start)
+  int* any = nullptr;               // imax + 2, pinned host memory: some system active for iteration it + 1 (set to 1 by iteration
+                                    // it, [0] by the start; cleared by the host)
 };
 void launch_pk_qeq_init(const State& st, QeqBuffers& qb, const PackedQeq& pq, int imax, double tol, int use_hist, hipStream_t s);
 void launch_pk_qeq_iteration(const State& st, QeqBuffers& qb, const PackedQeq& pq, int it, int imax, double tol, hipStream_t s);
@@ -174,13 +176,14 @@ void launch_md_half_kick(const State& st, MdBuffers& md, double dtf, hipStream_t
 void launch_md_drift(const State& st, MdBuffers& md, double dt, hipStream_t s);
 void launch_md_ref_positions(const State& st, MdBuffers& md, hipStream_t s);
 // fused step kernels: see k_md.hip
-void launch_md_step_start(const State& st, MdBuffers& md, double dtf, double dt, bool thermostat, bool pending, hipStream_t s);
-int md_disp_partials();   // per-block partials of the kick-drift kernel's largest squared displacement (in md.partial)
+void launch_md_step_start(const State& st, MdBuffers& md, double dtf, double dt, bool thermostat, bool pending,
+                          double* disp /* pinned: md_disp_partials() */, hipStream_t s);
+int md_disp_partials();   // per-block partials of the kick-drift kernel's largest squared displacement
 void launch_md_gather_step_end(const State& st, MdBuffers& md, double dtf, bool thermostat, hipStream_t s);
 void launch_md_scale(const State& st, MdBuffers& md, hipStream_t s);
 void launch_pk_ref(const State& st, MdBuffers& md, const int* reb, hipStream_t s);
-void launch_pk_disp(const State& st, MdBuffers& md, const int* sys_start, int S, double lim, int* reb, int* any, double* disp,
-                    hipStream_t s);
+void launch_pk_disp(const State& st, MdBuffers& md, const int* sys_start, int S, double lim, int* reb, int* any /* pinned */,
+                    double* disp, hipStream_t s);
 void launch_pk_thermostat(const State& st, MdBuffers& md, const int* sys_start, int S, double* nh_all, hipStream_t s);
 void launch_pk_energy(const State& st, const int* sys_start, int S, double* out, hipStream_t s);
 
