@@ -32,6 +32,7 @@ struct DevPair {
   double D, alpha, r_vdW, gamma_w, rcore, ecore, acore, lgcij, lgre, gamma, v13cor, ovc;
   double ln_rs, ln_rp, ln_rpp;   // log of r_s, r_p, r_pp (0 where the bond kind is absent)
   double pgw, irvdw, ircore, re6;   // (1 / gamma_w)^p_vdW1, 1 / r_vdW, 1 / rcore, lgre^6
+  double bo_far;   // no distance beyond it gives BO' >= bo_cut (infinite where BO' is not a falling function of the distance)
   int tbs, s_ok, pi_ok, pp_ok;
 };
 

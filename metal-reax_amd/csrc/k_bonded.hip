@@ -1,7 +1,7 @@
 // Bond-order chain and the ten bonded ReaxFF terms on the device.
 //
 // Pipeline per step (one launch each, in stream order):
-//   bond_build  (wave per atom)   bond list from the skin list: d <= bond_cut and BO' >= bo_cut, uncorrected BO', dBO'/dx, Delta'
+//   bond_build  (atoms per wave)  bond list from the skin list: d <= bond_cut and BO' >= bo_cut, uncorrected BO', dBO'/dx, Delta'
 //                                 [reference src/cpu/bonded.cpp:109-162, terms.hpp:50-56]; H-bond partner lists [bonded.cpp:120-124]
 //   bo_correct  (thread per atom) corrected BO and its 11 derivative coefficients, always from the pair's canonical end so both ends
 //                                 hold bitwise-identical values [bonded.cpp:164-204, terms.hpp:66-164]; index of the mirror slot of
@@ -26,6 +26,7 @@
 // chain whose values they test: double in FP64 and mixed modes, so they match the FP64 engine outside its rounding, float in
 // FP32 mode. Energies, CdDelta and forces are
 // accumulated in double in every mode.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -118,127 +119,214 @@ __device__ inline void angle_and_dcos(const V3<T>& a, T da, const V3<T>& b, T db
 // ================================================================================================================
 // bond list + uncorrected bond orders
 // ================================================================================================================
-// One wave per atom walks the skin list in chunks of 64. The distance pass runs on every lane; entries within bond_cut are
-// compacted (ballot order = skin-list order) into a per-wave LDS ring and the FP64 BO' evaluation runs on full waves of 64
-// candidates, so the transcendental work is not repeated for the ~90% of skin entries that are out of bond range.
+// A wave takes several consecutive atoms (build_atoms_per_wave). For each, the distance pass walks the bond candidates in chunks of
+// 64 (the next chunk's positions and the entries of the one after in flight, across atoms). Candidates within bond_cut are
+// numbered in list order; those near enough to reach bo_cut (DevPair::bo_far: 2 to 3 A, against a bond_cut of 5 A) go with that
+// number into a per-wave LDS ring shared by the wave's atoms, and the BO' evaluation runs on full waves of 64 of them.
+// Bound by the latency of the position gathers at 24,000 atoms and by vector issue above: one evaluation per atom (52 candidates
+// within bond_cut in water, of which 3.4 become bonds) was two thirds of the instructions. 24,000 atoms 70 -> 56 us, 192,000
+// atoms 489 -> 321 us per step (alone on the device).
+// The sums over an atom's bonds are those of a wave with lane l holding candidates l, l + 64, ... of those within bond_cut
+// in turn: a bond's values go to place (number mod 64) of a zeroed row in LDS and the wave sums the row.
 constexpr int kBuildWaves = 4;
 constexpr int kRing = 128;
 
 template <class TB>
-__device__ inline void bo_prime_batch(const State& st, const Globals& g, const Tables& t, int i, int ti, int m, const int* rj,
-                                      const int* rs, const double* rd, const double* rx, const double* ry, const double* rz,
-                                      int head, int& nb, TB& sum_bo, TB& ddx, TB& ddy, TB& ddz) {
-  const int lane = lane_id(), n = st.n;
-  const TB bo_cut = (TB)g.bo_cut;
-  bool bkeep = false;
-  int j = 0, s = 0;
-  double d = 0, dx = 0, dy = 0, dz = 0;
-  TB bs = 0, bp = 0, bpp = 0, cln = 0, clp = 0, clpp = 0;
-  if (lane < m) {
-    const int e = (head + lane) & (kRing - 1);
-    j = rj[e]; s = rs[e]; d = rd[e]; dx = rx[e]; dy = ry[e]; dz = rz[e];
-    const DevPair& P = t.pair[ti * g.ntypes + st.type[j]];
-    const TB dd = (TB)d;
-    TB C12 = 0, C34 = 0, C56 = 0;
-    if constexpr (std::is_same<TB, double>::value) {
-      // (d / r)^p as exp(p (log d - log r)): one logarithm for the three kinds (log r from the pair table) instead of three
-      // general powers; the exponent's rounding error is a few 1e-16, so BO' moves by about 1e-15 relative
-      const double ld = log(dd);
-      if (P.s_ok) { C12 = P.p_bo1 * exp(P.p_bo2 * (ld - P.ln_rs)); bs = (1.0 + bo_cut) * exp(C12); }
-      if (P.pi_ok) { C34 = P.p_bo3 * exp(P.p_bo4 * (ld - P.ln_rp)); bp = exp(C34); }
-      if (P.pp_ok) { C56 = P.p_bo5 * exp(P.p_bo6 * (ld - P.ln_rpp)); bpp = exp(C56); }
-    } else {
-      if (P.s_ok) { C12 = (TB)P.p_bo1 * rpow<TB>(dd / (TB)P.r_s, (TB)P.p_bo2); bs = (TB(1) + bo_cut) * rexp<TB>(C12); }
-      if (P.pi_ok) { C34 = (TB)P.p_bo3 * rpow<TB>(dd / (TB)P.r_p, (TB)P.p_bo4); bp = rexp<TB>(C34); }
-      if (P.pp_ok) { C56 = (TB)P.p_bo5 * rpow<TB>(dd / (TB)P.r_pp, (TB)P.p_bo6); bpp = rexp<TB>(C56); }
+struct BuildRing {   // LDS of one wave
+  int j[kRing], s[kRing], ta[kRing], no[kRing];   // partner, shift code, its type | atom of the wave << 16, number within bond_cut
+  double d[kRing], x[kRing], y[kRing], z[kRing];
+  TB sum[64][4];
+};
+
+template <class TB>
+struct BondBuild {
+  const State& st;
+  const Globals& g;
+  const Tables& t;
+  BuildRing<TB>& R;
+  const int first, na;   // the wave's atoms
+  int tl;                // lane a: type of atom first + a
+  int head = 0, fill = 0;
+  int open = 0, nb = 0;  // first atom not yet finished, its bonds so far
+
+  // sums of the open atom's bonds; its uncorrected Delta', dDelta' and bond count
+  __device__ void finish() {
+    const int lane = lane_id(), i = first + open, ti = __builtin_amdgcn_readlane(tl, open);
+    TB v[4];
+    for (int c = 0; c < 4; ++c) { v[c] = R.sum[lane][c]; R.sum[lane][c] = TB(0); }
+    const double val = ti >= 0 ? t.sp[ti].valency : 0.0, valv = ti >= 0 ? t.sp[ti].valency_val : 0.0;
+    if (lane == 0) {
+      st.b_cnt[i] = nb;
+      if (nb > st.maxb) atomicMax(&st.flags[1], nb);
     }
-    bkeep = bs + bp + bpp >= bo_cut;
-    const TB rr2 = TB(1) / (dd * dd);
-    cln = (TB)P.p_bo2 * C12 * rr2;
-    clp = (TB)P.p_bo4 * C34 * rr2;
-    clpp = (TB)P.p_bo6 * C56 * rr2;
+    if constexpr (std::is_same<TB, double>::value) {   // row r of 16 lanes holds the r-th sum
+      const double s = wave_sum4_rows(v[0], v[1], v[2], v[3]);
+      if (lane == 0) { st.Dp[i] = s - val; st.Dpb[i] = s - valv; }
+      double* const to = lane < 32 ? st.dDps_x : (lane < 48 ? st.dDps_y : st.dDps_z);
+      if (lane % 16 == 0 && lane > 0) to[i] = s;
+    } else {
+      for (int c = 0; c < 4; ++c) v[c] = wave_sum(v[c]);
+      if (lane == 0) {
+        st.Dp[i] = (double)(v[0] - (TB)val);
+        st.Dpb[i] = (double)(v[0] - (TB)valv);
+        st.dDps_x[i] = (double)v[1]; st.dDps_y[i] = (double)v[2]; st.dDps_z[i] = (double)v[3];
+      }
+    }
+    ++open;
+    nb = 0;
   }
-  const unsigned long long mb = __ballot(bkeep);
-  if (bkeep) {
-    const int p = nb + lanes_below(mb);
-    if (p < st.maxb) {
-      const size_t q = sl(p, i, n);
+
+  // BO' of the ring's first m entries; the atoms below `upto` have all their entries in it (or behind) and are finished
+  __device__ void batch(int m, int upto) {
+    const int lane = lane_id(), n = st.n;
+    const TB bo_cut = (TB)g.bo_cut;
+    bool bkeep = false;
+    int j = 0, s = 0, a = -1, no = 0;
+    double d = 0, dx = 0, dy = 0, dz = 0;
+    TB bs = 0, bp = 0, bpp = 0, cln = 0, clp = 0, clpp = 0;
+    if (lane < m) {
+      const int e = (head + lane) & (kRing - 1);
+      j = R.j[e]; s = R.s[e]; d = R.d[e]; dx = R.x[e]; dy = R.y[e]; dz = R.z[e];
+      a = R.ta[e] >> 16;
+      no = R.no[e];
+    }
+    const int ti = __shfl(tl, a < 0 ? 0 : a, 64);
+    if (lane < m) {
+      const int tj = R.ta[(head + lane) & (kRing - 1)] & 0xFFFF;
+      const DevPair& P = t.pair[ti * g.ntypes + tj];
+      const TB dd = (TB)d;
+      TB C12 = 0, C34 = 0, C56 = 0;
+      if constexpr (std::is_same<TB, double>::value) {
+        // (d / r)^p as exp(p (log d - log r)): one logarithm for the three kinds (log r from the pair table) instead of three
+        // general powers; the exponent's rounding error is a few 1e-16, so BO' moves by about 1e-15 relative
+        const double ld = log(dd);
+        if (P.s_ok) { C12 = P.p_bo1 * exp(P.p_bo2 * (ld - P.ln_rs)); bs = (1.0 + bo_cut) * exp(C12); }
+        if (P.pi_ok) { C34 = P.p_bo3 * exp(P.p_bo4 * (ld - P.ln_rp)); bp = exp(C34); }
+        if (P.pp_ok) { C56 = P.p_bo5 * exp(P.p_bo6 * (ld - P.ln_rpp)); bpp = exp(C56); }
+      } else {
+        if (P.s_ok) { C12 = (TB)P.p_bo1 * rpow<TB>(dd / (TB)P.r_s, (TB)P.p_bo2); bs = (TB(1) + bo_cut) * rexp<TB>(C12); }
+        if (P.pi_ok) { C34 = (TB)P.p_bo3 * rpow<TB>(dd / (TB)P.r_p, (TB)P.p_bo4); bp = rexp<TB>(C34); }
+        if (P.pp_ok) { C56 = (TB)P.p_bo5 * rpow<TB>(dd / (TB)P.r_pp, (TB)P.p_bo6); bpp = rexp<TB>(C56); }
+      }
+      bkeep = bs + bp + bpp >= bo_cut;
+      const TB rr2 = TB(1) / (dd * dd);
+      cln = (TB)P.p_bo2 * C12 * rr2;
+      clp = (TB)P.p_bo4 * C34 * rr2;
+      clpp = (TB)P.p_bo6 * C56 * rr2;
+    }
+    const TB tot = (bs + bp + bpp) - bo_cut;
+    const TB dc = -(bs * cln + bp * clp + bpp * clpp);
+    int p = 0;   // the bond's slot
+    const int last = m > 0 ? __builtin_amdgcn_readlane(a, m - 1) : -1;
+    while (open < upto || open <= last) {
+      const bool mine = bkeep && a == open;
+      const unsigned long long mk = __ballot(mine);
+      if (mine) p = nb + lanes_below(mk);
+      nb += __popcll(mk);
+      int turn = 0;
+      for (unsigned long long left = mk; left; ++turn) {   // numbers that share a place (64 apart) take turns
+        const bool now = mine && no >> 6 == turn;
+        if (now) {
+          TB* q = R.sum[no & 63];
+          q[0] += tot;
+          q[1] += dc * (TB)dx; q[2] += dc * (TB)dy; q[3] += dc * (TB)dz;
+        }
+        left &= ~__ballot(now);
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (open >= upto) break;   // its entries go on in the next batch
+      finish();
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (bkeep && p < st.maxb) {
+      const size_t q = sl(p, first + a, n);
       st.b_j[q] = j; st.b_s[q] = s;
       st.b_d[q] = d; st.b_dx[q] = dx; st.b_dy[q] = dy; st.b_dz[q] = dz;
-      const TB tot = (bs + bp + bpp) - bo_cut;
       st.bop_s[q] = (double)(bs - bo_cut);
       st.bop_pi[q] = (double)bp;
       st.bop_pi2[q] = (double)bpp;
       st.bo[q] = (double)tot;   // uncorrected total until bo_correct overwrites it
-      const TB dc = -(bs * cln + bp * clp + bpp * clpp);
       st.dbop_c[q] = (double)dc;
       st.dlnpi_c[q] = (double)(-bp * clp);
       st.dlnpi2_c[q] = (double)(-bpp * clpp);
-      sum_bo += tot;
-      ddx += dc * (TB)dx; ddy += dc * (TB)dy; ddz += dc * (TB)dz;
     }
+    head = (head + m) & (kRing - 1);
+    fill -= m;
   }
-  nb += __popcll(mb);
-}
+};
 
-// 4 waves per SIMD (108 VGPRs without spills; 129 and 3 waves otherwise)
 template <class TB>
-__global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * kBuildWaves) k_bond_build(State st, Cell c, Globals g, Tables t) {
-  __shared__ int rj_[kBuildWaves][kRing], rs_[kBuildWaves][kRing];
-  __shared__ double rd_[kBuildWaves][kRing], rx_[kBuildWaves][kRing], ry_[kBuildWaves][kRing], rz_[kBuildWaves][kRing];
-  const int w = threadIdx.x >> 6;
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  if (i >= st.n) return;
-  int* rj = rj_[w]; int* rs = rs_[w];
-  double *rd = rd_[w], *rx = rx_[w], *ry = ry_[w], *rz = rz_[w];
+__global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * kBuildWaves) k_bond_build(State st, Globals g, Tables t,
+                                                                                                         int per_wave) {
+  __shared__ BuildRing<TB> rings[kBuildWaves];
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int first = (int)(blockIdx.x * kBuildWaves + w) * per_wave;
+  const int na = min(per_wave, st.n - first);
+  if (na <= 0) return;
   const int lane = lane_id();
-  const int ti = st.type[i];
-  int nb = 0;
-  TB sum_bo = 0, ddx = 0, ddy = 0, ddz = 0;
-  if (ti >= 0) {
-    const double4 pi = st.pos[i];
-    const size_t base = (size_t)i * st.maxbc;
-    const int cnt = min(st.bc_cnt[i], st.maxbc);
-    int head = 0, fill = 0;   // LDS ring of bond candidates (wave-uniform)
-    for (int k0 = 0; k0 < cnt; k0 += 64) {
-      const int k = k0 + lane;
-      bool near = false;
-      int j = 0, s = 0;
-      double dx = 0, dy = 0, dz = 0, d = 0;
-      if (k < cnt) {
-        j = st.bc_j[base + k];
-        const int e = st.bc_s[base + k];
-        s = entry_code(e);
-        d = sqrt(pair_dvec_list(st, pi, j, e, dx, dy, dz));
-        near = d <= g.bond_cut;
-      }
-      const unsigned long long mn = __ballot(near);
-      if (near) {
-        const int e = (head + fill + lanes_below(mn)) & (kRing - 1);
-        rj[e] = j; rs[e] = s; rd[e] = d; rx[e] = dx; ry[e] = dy; rz[e] = dz;
-      }
-      fill += __popcll(mn);
-      __builtin_amdgcn_wave_barrier();
-      if (fill >= 64) {
-        bo_prime_batch<TB>(st, g, t, i, ti, 64, rj, rs, rd, rx, ry, rz, head, nb, sum_bo, ddx, ddy, ddz);
-        head = (head + 64) & (kRing - 1);
-        fill -= 64;
-        __builtin_amdgcn_wave_barrier();
-      }
+  BuildRing<TB>& R = rings[w];
+  for (int c = 0; c < 4; ++c) R.sum[lane][c] = TB(0);
+  int tl = -1, cl = 0;   // lane a: type and candidates of atom first + a
+  if (lane < na) {
+    tl = st.type[first + lane];
+    cl = tl >= 0 ? min(st.bc_cnt[first + lane], st.maxbc) : 0;
+  }
+  BondBuild<TB> B{st, g, t, R, first, na, tl};
+  // the chunk after (a, k0): the atom's next one, or the next atom's first (a = na: none)
+  auto next = [&](int& a, int& k0) {
+    k0 += 64;
+    while (a < na && k0 >= __builtin_amdgcn_readlane(cl, a)) { ++a; k0 = 0; if (a < na && __builtin_amdgcn_readlane(cl, a) > 0) break; }
+  };
+  auto entries = [&](int a, int k0, int& j, int& e) {   // lanes past the row's end carry the wave's first atom, never used
+    j = first; e = 0;
+    if (a < na && k0 + lane < __builtin_amdgcn_readlane(cl, a)) {
+      const size_t o = (size_t)(first + a) * st.maxbc + k0 + lane;
+      j = st.bc_j[o];
+      e = st.bc_s[o];
     }
-    if (fill > 0) bo_prime_batch<TB>(st, g, t, i, ti, fill, rj, rs, rd, rx, ry, rz, head, nb, sum_bo, ddx, ddy, ddz);
+  };
+  int a = 0, k0 = -64;
+  next(a, k0);
+  int aB = a, kB = k0, jC, eC, jB, eB;
+  entries(a, k0, jC, eC);
+  double4 pC = st.pos[jC];
+  next(aB, kB);
+  entries(aB, kB, jB, eB);
+  int near_before = 0;   // candidates of this atom within bond_cut in its earlier chunks
+  while (a < na) {
+    const int j = jC, e = eC, ca = a, ck = k0, i = first + a, ti = __builtin_amdgcn_readlane(tl, a);
+    const double4 pj = pC, pi = st.pos[i];
+    a = aB; k0 = kB; jC = jB; eC = eB;
+    pC = st.pos[jC];
+    if (aB < na) next(aB, kB);
+    entries(aB, kB, jB, eB);
+    bool near = false, keep = false;
+    double dx = 0, dy = 0, dz = 0, d = 0;
+    int tj = 0;
+    if (ck + lane < __builtin_amdgcn_readlane(cl, ca)) {
+      d = sqrt(pair_dvec_pos(st, pi, pj, e, dx, dy, dz));
+      near = d <= g.bond_cut;
+      tj = pos_type(pj.w);
+      keep = near && d <= t.pair[ti * g.ntypes + tj].bo_far;
+    }
+    const unsigned long long mn = __ballot(near), mk = __ballot(keep);
+    if (keep) {
+      const int o = (B.head + B.fill + lanes_below(mk)) & (kRing - 1);
+      R.j[o] = j; R.s[o] = entry_code(e); R.ta[o] = tj | ca << 16; R.no[o] = near_before + lanes_below(mn);
+      R.d[o] = d; R.x[o] = dx; R.y[o] = dy; R.z[o] = dz;
+    }
+    near_before = a == ca ? near_before + __popcll(mn) : 0;
+    B.fill += __popcll(mk);
+    __builtin_amdgcn_wave_barrier();
+    // (entries left over by a batch belong to this atom, which then is not finished)
+    if (B.fill >= 64) B.batch(64, a == ca || B.fill > 64 ? ca : ca + 1);
   }
-  // fixed-order wave reductions
-  sum_bo = wave_sum(sum_bo); ddx = wave_sum(ddx); ddy = wave_sum(ddy); ddz = wave_sum(ddz);
-  if (lane == 0) {
-    st.b_cnt[i] = nb;
-    if (nb > st.maxb) atomicMax(&st.flags[1], nb);
-    const double val = ti >= 0 ? t.sp[ti].valency : 0.0, valv = ti >= 0 ? t.sp[ti].valency_val : 0.0;
-    st.Dp[i] = (double)(sum_bo - (TB)val);
-    st.Dpb[i] = (double)(sum_bo - (TB)valv);
-    st.dDps_x[i] = (double)ddx; st.dDps_y[i] = (double)ddy; st.dDps_z[i] = (double)ddz;
-  }
+  B.batch(B.fill, na);
 }
+// Atoms per wave: below 6000 atoms one (the chain of a wave's chunks is what takes the time: 648 atoms 14 us with one, 33 us with
+// eight), then enough waves to fill the chip, up to 16 atoms, whose bond candidates (4 per atom in water) fill the evaluation.
+// Bond lists per step (HIP events) at 24,000 / 192,000 atoms: one atom 72 / 505 us, two 59 / 396, eight 56 / 333, sixteen - / 321.
+inline int build_atoms_per_wave(int n) { return std::min(16, std::max(1, n / 3000)); }
 
 // ---- atom groups: G lanes per atom (G a power of two >= the largest bond count), lane p owns bond slot p of its atom ----------
 // Sums over a group (group_sum) use lane exchanges with offsets below G, so they stay inside the group and run in a fixed order.
@@ -1405,15 +1493,16 @@ void with_lanes(int lanes, F&& f) {
 }
 
 template <class TB>
-void bond_build_t(const State& st, const Cell& c, const Globals& g, const Tables& t, hipStream_t s) {
-  hipLaunchKernelGGL(k_bond_build<TB>, dim3(nblk(st.n, kBuildWaves)), dim3(64 * kBuildWaves), 0, s, st, c, g, t);
+void bond_build_t(const State& st, const Globals& g, const Tables& t, hipStream_t s) {
+  const int per = build_atoms_per_wave(st.n);
+  hipLaunchKernelGGL(k_bond_build<TB>, dim3(nblk(st.n, kBuildWaves * per)), dim3(64 * kBuildWaves), 0, s, st, g, t, per);
 }
 
 }  // namespace
 
-void launch_bond_build(Precision p, const State& st, const Cell& c, const Globals& g, const Tables& t, hipStream_t s) {
-  if (p == Precision::FP32) bond_build_t<float>(st, c, g, t, s);
-  else bond_build_t<double>(st, c, g, t, s);
+void launch_bond_build(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s) {
+  if (p == Precision::FP32) bond_build_t<float>(st, g, t, s);
+  else bond_build_t<double>(st, g, t, s);
 }
 
 

@@ -1,0 +1,56 @@
+"""Bonded kernels at the edges of their work splits, FP64 and mixed, against the FP64 oracle: dense carbon (diamond with random
+displacements: 94 atoms within bond_cut, so that numbers within bond_cut pass 64 and share places in the sums, 4 to 6 bonds per
+atom, several hundred torsions per wave) at sizes below and above the line where a wave takes several atoms, with the last wave
+partly filled, and atom counts around a wave.
+
+Bars as tests/test_gpu_variants.py: FP64 each term within 1e-9 of max(1, |E|), gradient within 1e-7 kcal/mol/A; mixed 1e-4
+kcal/mol per atom and 4e-3 / 9e-4 kcal/mol/A (largest, RMS). Those hold for forces of the order of 100 kcal/mol/A; rounding grows
+with the terms, so the gradient bars are scaled by the largest reference gradient over 100."""
+import os
+
+import numpy as np
+import pytest
+
+from helpers import new_engine
+from oracle.oracle import Oracle
+
+TERMS = ("e_bond", "e_ov", "e_un", "e_lp", "e_ang", "e_pen", "e_coa", "e_tor", "e_con", "e_vdW")
+BASIS = np.array([[0, 0, 0], [0, 2, 2], [2, 0, 2], [2, 2, 0], [1, 1, 1], [1, 3, 3], [3, 1, 3], [3, 3, 1]]) / 4.0
+
+
+def diamond(cells, drop, seed, a=3.567, sigma=0.08):
+    g = np.stack(np.meshgrid(*[np.arange(c) for c in cells], indexing="ij"), -1).reshape(-1, 3)
+    x = ((g[:, None] + BASIS[None]) * a).reshape(-1, 3)
+    rng = np.random.default_rng(seed)
+    x = x + rng.normal(size=x.shape) * sigma
+    return x[rng.permutation(len(x))[drop:]], np.array(cells) * a
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cells,drop", [((2, 2, 2), 1), ((2, 2, 3), 31), ((3, 3, 3), 0), ((9, 10, 9), 17)])
+def test_dense_carbon(cells, drop):
+    with open(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "ffield.C2013")) as fh:
+        ff = fh.read()
+    x, L = diamond(cells, drop, seed=sum(cells))
+    n = len(x)
+    types, tags, q = np.ones(n, dtype=np.int32), np.arange(1, n + 1), np.zeros(n)
+    box12 = [0, 0, 0, L[0], 0, 0, 0, L[1], 0, 0, 0, L[2]]
+    ref = Oracle(ff).compute(x, types - 1, tags, box12, (True, True, True), q=q)
+    for prec in ("fp64", "mixed"):
+        e = new_engine(ff, ["C"], prec, extra=("checkqeq", "no"))
+        e.set_box(np.zeros(3), L)
+        e.set_atoms(types, tags, x)
+        e.set_charges(q)
+        r = e.compute(rebuild=True, census=True)
+        cen = e.census()
+        e.close()
+        d = (r["grad"] - np.asarray(ref["grad"])) / max(1.0, np.abs(ref["grad"]).max() / 100.0)
+        if prec == "fp64":
+            for k in TERMS:
+                assert abs(r["energy"][k] - ref["energy"][k]) <= 1e-9 * max(1.0, abs(ref["energy"][k])), (n, k)
+            assert np.abs(d).max() <= 1e-7, n
+        else:
+            assert abs(sum(r["energy"].values()) - sum(ref["energy"].values())) / n <= 1e-4, n
+            assert np.abs(d).max() <= 4e-3 and np.sqrt((d ** 2).mean()) <= 9e-4, n
+        for k, name in enumerate(("bonds", "angle_sets", "torsions")):
+            assert np.array_equal(cen[k], np.asarray(ref["census"][name])), (n, prec, name)
