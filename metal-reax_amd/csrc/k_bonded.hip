@@ -7,7 +7,8 @@
 //                                 hold bitwise-identical values [bonded.cpp:164-204, terms.hpp:66-164]; index of the mirror slot of
 //                                 every bond and the step's largest bond count
 //   atom_terms  (thread per atom) bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
-//   valence     (thread per atom) valence angle, penalty, 3-body conjugation at the centre [bonded.cpp:321-474]
+//   valence     (wave per 64 / G atoms, angles spread over its lanes) valence angle, penalty, 3-body conjugation at the centre
+//                                 [bonded.cpp:321-474]
 //   torsion     (thread per atom) torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
 //                                 and derivative contributions of its own half (its own atom, its outer partner, its outer bond) and
 //                                 the end the reference counts (tag order) adds the energy and the central-bond terms [bonded.cpp:476-652]
@@ -75,6 +76,13 @@ template <class T> __device__ inline T safe_exp(T x) {
 // [-ka a - 2 kb b + (ka - kb) a b] inv inv, and a, b from safe_exp, every intermediate stays finite.
 template <class T> __device__ inline T ratio2_deriv(T a, T b, T ka, T kb, T inv) {
   return ((-ka * a - T(2) * kb * b + (ka - kb) * (a * b)) * inv) * inv;
+}
+
+// v as rounded, to any expression it enters: keeps the compiler from contracting the operation that gave it with the next one
+// (where a value used to cross into a loop, and so was rounded, and the same sums are wanted without the loop)
+template <class T> __device__ inline T rounded(T v) {
+  asm("" : "+v"(v));
+  return v;
 }
 
 template <class T> struct V3 { T x, y, z; };
@@ -634,15 +642,127 @@ __global__ void __launch_bounds__(256) k_atom_terms(State st, Globals g, Tables 
 // valence angle, penalty, 3-body conjugation (centre j)
 // ================================================================================================================
 
-// Valence angle, penalty and three-body conjugation at the centre j [reference bonded.cpp:321-474]. Lane p of j's group evaluates
-// the pairs (p, k) with p < k of j's bonds, k running over a wave-uniform loop: the contributions to slot p stay in the lane, the
-// contributions to slot k are summed over the group and kept by lane k, and the centre's are summed over the group at the end.
+// Work items of the angle kernels. A wave's atom groups go through their angles (torsions) in rows, a row holding at most one item
+// per lane: the owner of the item, whose sums it enters. The items that pass the gates are queued over the rows, and once the
+// next row no longer fits, the 64 lanes evaluate the queued items side by side and leave the results in LDS; each owner then
+// adds its items row by row, in the order of a loop over the rows, so the sums do not depend on how the items were spread.
+// Evaluating each row in place instead ran the whole wave for the few lanes with an item in that row (26 % of lanes active in
+// the valence kernel, 10 % in the torsion kernel on water).
+struct ItemRows {
+  int items = 0, rows = 0;   // queued (wave-uniform)
+  int lo = 0, hi = 0, tag = 0, start = 0;   // lane r: row r's lanes with an item (mask), its tag, its first item
+
+  __device__ bool fits(unsigned long long mask) const { return items + __popcll(mask) <= 64 && rows < 64; }
+  // a row with items on the lanes of mask; returns the place of this lane's item
+  __device__ int add(unsigned long long mask, int row_tag) {
+    if (lane_id() == rows) { lo = (int)(unsigned)mask; hi = (int)(unsigned)(mask >> 32); tag = row_tag; start = items; }
+    const int place = items + lanes_below(mask);
+    items += __popcll(mask);
+    ++rows;
+    return place;
+  }
+  __device__ unsigned long long mask_of(int r) const {
+    return (unsigned long long)(unsigned)__builtin_amdgcn_readlane(lo, r) | (unsigned long long)(unsigned)__builtin_amdgcn_readlane(hi, r) << 32;
+  }
+  __device__ int tag_of(int r) const { return __builtin_amdgcn_readlane(tag, r); }
+  __device__ int start_of(int r) const { return __builtin_amdgcn_readlane(start, r); }
+  __device__ void clear() { items = rows = 0; }
+};
+constexpr int kRowClose = 1 << 16;   // tag of a row that ends the rows of slot (tag & 0xFFFF): no items
+constexpr int kAngleWaves = 4;       // waves per block of the angle kernels
+
+// Valence angle, penalty and three-body conjugation at the centre j [reference bonded.cpp:321-474]. Lane p of j's group owns bond
+// slot p and the pairs (p, k) with p < k: the contributions to slot p stay with the lane, those to slot k are summed over the
+// group and kept by lane k, and the centre's are summed over the group at the end. Rows: slot k, then parameter set.
 // PA: also the reference's per-atom virial split (bonded.cpp:462-466): each angle's (x_i - x_j) (x) F_i + (x_k - x_j) (x) F_k,
 // a third to each of i, j and k (the ends through their slots).
+//
+// Bound by the arithmetic of an angle: 11 exponentials, 4 powers (FP64: also the arc cosine), in FP64 some 2000 instructions, run once
+// per 64 angles now. The centre's powers run once each, on the even and the odd lanes of the group. The term kernels of a step
+// (this, torsion, hydrogen bonds) took, before and with this: 648 atoms of water mixed 147 -> 120 us, 24000 269 -> 235 us, 192000 1729 ->
+// 1553 us, FP64 24000 381 -> 325 us, 30000 atoms of disordered carbon mixed 373 -> 336 us. LDS: 6.5 KB per wave in FP32, 13 KB in FP64.
+//
+// Results of an item. A product that the sum takes in by a fused multiply-add is kept as its two factors; a value with other uses,
+// and what rounded() marks, enters rounded. So the sums are those of a loop over the angles in place, bit for bit.
+enum ValResult {
+  V_OWN_CDBO, V_TO_CDBO, V_CDSELF, V_OWN_CDP, V_TO_CDP, V_CE5,
+  V_CE8, V_DCI, V_DCJ = V_DCI + 3, V_DCK = V_DCJ + 3,   // factors of the forces: CE8 and d cos(theta) / d x of i, j, k
+  V_ANG = V_DCK + 3, V_PEN = V_ANG + 2, V_COA, kValResults   // energies (e_ang: two factors)
+};
+template <class TR, class TS>
+struct ValenceLds {   // one wave
+  TS bo[64];                             // lane: its bond
+  TR x[64], y[64], z[64], d[64], tbo[64];
+  int type[64];
+  TS sbo_pi[64], sbo_e[64];              // bo_pi + bo_pi2, exp(-BO^8) (double) or BO^8 (float)
+  TR centre[10][16];                     // group: SBO2 CSBO2 dSBO2 ev6 f9 Cf9 ec2 Dboc p_val3 p_val5
+  int who[64], set[64];                  // item: owner lane | lane of slot k << 8, parameter set
+  TR res[kValResults][64];
+};
+
+// the item's angle (slots of lanes a and b of the same group) with parameter set `set`
+template <class TR, class TS, int G>
+__device__ inline void valence_item(const Globals& g, const Tables& t, ValenceLds<TR, TS>& L, int e) {
+  const int who = L.who[e], a = who & 0xFF, b = who >> 8, c = a / G;
+  const TR thb_cut = (TR)g.thb_cut;
+  const TR p_val6 = (TR)g.p_val6, p_val10 = (TR)g.p_val10;
+  const TR p_pen2 = (TR)g.p_pen2;
+  const TR p_coa2 = (TR)g.p_coa2, p_coa3 = (TR)g.p_coa3, p_coa4 = (TR)g.p_coa4;
+  const TR SBO2 = L.centre[0][c], CSBO2 = L.centre[1][c], dSBO2 = L.centre[2][c], ev6 = L.centre[3][c],
+           f9 = L.centre[4][c], Cf9 = L.centre[5][c], ec2 = L.centre[6][c], Dboc = L.centre[7][c], p_val3 = L.centre[8][c],
+           p_val5 = L.centre[9][c];
+  const TR BOA_ij = (TR)L.bo[a] - thb_cut, BOA_jk = (TR)L.bo[b] - thb_cut, tboi = L.tbo[a], tbok = L.tbo[b];
+  const V3<TR> vij{L.x[a], L.y[a], L.z[a]}, vjk{L.x[b], L.y[b], L.z[b]};
+  TR th, ct, sth;
+  V3<TR> dci, dcj, dck;
+  angle_and_dcos<TR>(vij, L.d[a], vjk, L.d[b], th, ct, sth, dci, dcj, dck);
+  if (sth < TR(1.0e-5)) sth = TR(1.0e-5);
+  if (sizeof(TR) == 8) th = rounded(th);   // acos ends in a product
+  const DevAngle A = t.angle[L.set[e]];
+  const TR p_val1 = (TR)A.p_val1;
+  const TR p_val2 = (TR)A.p_val2, p_val4 = (TR)A.p_val4, p_val7 = (TR)A.p_val7, th00 = (TR)A.theta_00;
+  const TR e3ij = rexp<TR>(-p_val3 * rpow<TR>(BOA_ij, p_val4)), f7ij = TR(1) - e3ij;
+  const TR Cf7ij = p_val3 * p_val4 * rpow<TR>(BOA_ij, p_val4 - TR(1)) * e3ij;
+  const TR e3jk = rexp<TR>(-p_val3 * rpow<TR>(BOA_jk, p_val4)), f7jk = TR(1) - e3jk;
+  const TR Cf7jk = p_val3 * p_val4 * rpow<TR>(BOA_jk, p_val4 - TR(1)) * e3jk;
+  const TR ev7 = safe_exp<TR>(-p_val7 * Dboc), itrm8 = TR(1) / (TR(1) + ev6 + ev7);
+  const TR f8 = p_val5 - (p_val5 - TR(1)) * ((TR(2) + ev6) * itrm8);
+  const TR Cf8 = (TR(1) - p_val5) * ratio2_deriv<TR>(ev6, ev7, p_val6, -p_val7, itrm8);
+  const TR th0 = (TR(180.0) - th00 * (TR(1) - rexp<TR>(-p_val10 * (TR(2) - SBO2)))) * TR(3.14159265) / TR(180.0);
+  const TR e2t = rexp<TR>(-p_val2 * ((th0 - th) * (th0 - th)));
+  const TR e12t = p_val1 >= TR(0) ? p_val1 * (TR(1) - e2t) : p_val1 * -e2t;
+  const TR CE1 = Cf7ij * f7jk * f8 * e12t, CE2 = Cf7jk * f7ij * f8 * e12t, CE3 = Cf8 * f7ij * f7jk * e12t;
+  const TR CE4 = -TR(2) * p_val1 * p_val2 * f7ij * f7jk * f8 * e2t * (th0 - th);
+  const TR Cth0 = p_val10 * (th00 * TR(3.14159265) / TR(180.0)) * rexp<TR>(-p_val10 * (TR(2) - SBO2));
+  const TR CE5 = -CE4 * Cth0 * CSBO2, CE7 = CE5 * dSBO2, CE8 = -CE4 / sth;
+  L.res[V_CE5][e] = CE5;
+  L.res[V_ANG][e] = f7ij * f7jk * f8; L.res[V_ANG + 1][e] = e12t;
+  const TR p_pen1 = (TR)A.p_pen1;
+  const TR ep2ij = rexp<TR>(-p_pen2 * ((BOA_ij - TR(2)) * (BOA_ij - TR(2)))), ep2jk = rexp<TR>(-p_pen2 * ((BOA_jk - TR(2)) * (BOA_jk - TR(2))));
+  const TR epen = p_pen1 * f9 * ep2ij * ep2jk;
+  L.res[V_PEN][e] = epen;
+  const TR CEp1 = epen * Cf9 / f9, tp = -TR(2) * p_pen2 * epen, CEp2 = tp * (BOA_ij - TR(2)), CEp3 = tp * (BOA_jk - TR(2));
+  const TR p_coa1 = (TR)A.p_coa1;
+  const TR dti = tboi - BOA_ij, dtk = tbok - BOA_jk;
+  const TR ecoa = p_coa1 / (TR(1) + ec2) * rexp<TR>(-p_coa3 * (dti * dti)) * rexp<TR>(-p_coa3 * (dtk * dtk)) *
+                  rexp<TR>(-p_coa4 * ((BOA_ij - TR(1.5)) * (BOA_ij - TR(1.5)))) * rexp<TR>(-p_coa4 * ((BOA_jk - TR(1.5)) * (BOA_jk - TR(1.5))));
+  L.res[V_COA][e] = ecoa;
+  const TR CEc1 = -TR(2) * p_coa4 * (BOA_ij - TR(1.5)) * ecoa, CEc2 = -TR(2) * p_coa4 * (BOA_jk - TR(1.5)) * ecoa;
+  const TR CEc3 = -p_coa2 * (ec2 / (TR(1) + ec2)) * ecoa, CEc4 = -TR(2) * p_coa3 * dti * ecoa, CEc5 = -TR(2) * p_coa3 * dtk * ecoa;
+  L.res[V_OWN_CDBO][e] = CE1 + CEp2 + (CEc1 - CEc4);
+  L.res[V_TO_CDBO][e] = CE2 + CEp3 + (CEc2 - CEc5);
+  L.res[V_CDSELF][e] = (CE3 + CE7) + CEp1 + CEc3;
+  L.res[V_OWN_CDP][e] = CEc4; L.res[V_TO_CDP][e] = CEc5;
+  L.res[V_CE8][e] = CE8;
+  L.res[V_DCI][e] = dci.x; L.res[V_DCI + 1][e] = dci.y; L.res[V_DCI + 2][e] = dci.z;
+  L.res[V_DCJ][e] = dcj.x; L.res[V_DCJ + 1][e] = dcj.y; L.res[V_DCJ + 2][e] = dcj.z;
+  L.res[V_DCK][e] = dck.x; L.res[V_DCK + 1][e] = dck.y; L.res[V_DCK + 2][e] = dck.z;
+}
+
 template <class TR, class TS, int G, bool PA>
-__device__ inline void valence_body(const State& st, const Globals& g, const Tables& t) {
+__device__ inline void valence_body(const State& st, const Globals& g, const Tables& t, ValenceLds<TR, TS>& L) {
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = gid / G, p = gid % G, n = st.n;
+  const int j = gid / G, p = gid % G, n = st.n, lane = lane_id(), base = lane - p;
   const bool live = j < n;
   const int tj = live ? st.type[j] : -1;
   const int nb = live ? min(st.b_cnt[j], st.maxb) : 0;
@@ -653,16 +773,39 @@ __device__ inline void valence_body(const State& st, const Globals& g, const Tab
   int n_ang = 0, sbo_region = 0;   // census: bond pairs through the three-body gates, SBO branch
   double e_ang = 0, e_pen = 0, e_coa = 0, cdself = 0, fjx = 0, fjy = 0, fjz = 0, sCE5 = 0, sCE6 = 0;
   double own_cdbo = 0, own_cdp = 0, own_fx = 0, own_fy = 0, own_fz = 0;
-  // centre quantities (every lane of the group computes them)
-  TR SBO2 = 0, CSBO2 = 0, dSBO1 = 0, dSBO2 = 0, ev6 = 0, f9 = 0, Cf9 = 0, ec2 = 0, Dboc = 0, p_val3 = 0, p_val5 = 0;
-  const TR thb_cut = (TR)g.thb_cut;
   const TS thb_cut_s = (TS)g.thb_cut, thb_cutsq_s = (TS)g.thb_cutsq;
-  const TR p_val6 = (TR)g.p_val6, p_val10 = (TR)g.p_val10;
-  const TR p_pen2 = (TR)g.p_pen2, p_pen3 = (TR)g.p_pen3, p_pen4 = (TR)g.p_pen4;
-  const TR p_coa2 = (TR)g.p_coa2, p_coa3 = (TR)g.p_coa3, p_coa4 = (TR)g.p_coa4;
+  // this lane's bond (j, i)
+  const bool mine = act && p < nb;
+  size_t qi = 0;
+  int ti = 0;
+  TR BOij = 0;
+  TS BOij_s = 0, pis = 0, be = sizeof(TS) == 8 ? TS(1) : TS(0);
+  V3<TR> vij{0, 0, 0};
+  if (sbo_on && p < nb) {
+    qi = sl(p, j, n);
+    BOij_s = (TS)st.bo[qi];
+    BOij = (TR)st.bo[qi];
+    pis = (TS)st.bo_pi[qi] + (TS)st.bo_pi2[qi];
+    TS w = BOij_s * BOij_s;
+    w *= w;
+    w *= w;
+    be = sizeof(TS) == 8 ? rexp<TS>(-w) : w;
+  }
+  if (mine) {
+    const int i = st.b_j[qi];
+    ti = st.type[i];
+    vij = V3<TR>{(TR)st.b_dx[qi], (TR)st.b_dy[qi], (TR)st.b_dz[qi]};
+    L.d[lane] = (TR)st.b_d[qi];
+    L.tbo[lane] = (TR)st.tbo[i];
+  }
+  L.bo[lane] = BOij_s; L.x[lane] = vij.x; L.y[lane] = vij.y; L.z[lane] = vij.z; L.type[lane] = ti;
+  L.sbo_pi[lane] = pis; L.sbo_e[lane] = be;
+  __builtin_amdgcn_wave_barrier();
+  // centre quantities (every lane of the group computes them)
+  TR dSBO1 = 0;
   if (sbo_on) {
+    const TR p_val6 = (TR)g.p_val6, p_pen3 = (TR)g.p_pen3, p_pen4 = (TR)g.p_pen4, p_coa2 = (TR)g.p_coa2;
     const DevSpecies& sj = t.sp[tj];
-    p_val3 = (TR)sj.p_val3; p_val5 = (TR)sj.p_val5;
     // SBO and its branch in TS. omp = 1 - prod(exp(-BO^8)): in double the reference's product; in float from expm1 of the
     // exponent sum, since a bond with BO^8 below FP32's epsilon leaves the float product at exactly 1 and would drop out of
     // 1 - prod, which decides the sign of SBO at under-coordinated centres
@@ -670,13 +813,8 @@ __device__ inline void valence_body(const State& st, const Globals& g, const Tab
     {
       TS sw = 0;
       for (int b = 0; b < nb; ++b) {
-        const size_t q = sl(b, j, n);
-        const TS bo = (TS)st.bo[q];
-        SBOp += (TS)st.bo_pi[q] + (TS)st.bo_pi2[q];
-        TS w = bo * bo;
-        w *= w;
-        w *= w;
-        if (sizeof(TS) == 8) prod *= rexp<TS>(-w); else sw += w;
+        SBOp += L.sbo_pi[base + b];
+        if (sizeof(TS) == 8) prod *= L.sbo_e[base + b]; else sw += L.sbo_e[base + b];
       }
       if (sizeof(TS) == 8) omp = TS(1) - prod;
       else { omp = -rexpm1<TS>(-sw); prod = TS(1) - omp; }
@@ -686,121 +824,120 @@ __device__ inline void valence_body(const State& st, const Globals& g, const Tab
     if ((TS)st.vlpex[j] >= TS(0)) { vlpadj = 0; dSBO2s = -omp; }
     else { vlpadj = (TS)st.nlp[j]; dSBO2s = -omp * (TS(1) - p_val8s * dDlp); }
     const TS Dbocs = (TS)st.Delta_boc[j];
-    Dboc = (TR)Dbocs;
+    const TR Dboc = (TR)Dbocs;
     const TS SBO = SBOp + omp * (-Dbocs - p_val8s * vlpadj);
+    const TR dSBO2 = (TR)dSBO2s;
     dSBO1 = (TR)(-TS(8) * prod * (Dbocs + p_val8s * vlpadj));
-    dSBO2 = (TR)dSBO2s;
+    // SBO2 and its derivative from x^p and x^(p - 1) with x = SBO up to 1, 2 - SBO up to 2: the power with exponent p on the
+    // even lanes of the group, the one with p - 1 on the odd lanes
     const TS pv9 = (TS)g.p_val9;
-    if (SBO <= TS(0)) { SBO2 = 0; CSBO2 = 0; sbo_region = 0; }
-    else if (SBO <= TS(1)) { SBO2 = (TR)rpow<TS>(SBO, pv9); CSBO2 = (TR)(pv9 * rpow<TS>(SBO, pv9 - TS(1))); sbo_region = 1; }
-    else if (SBO < TS(2)) { SBO2 = (TR)(TS(2) - rpow<TS>(TS(2) - SBO, pv9)); CSBO2 = (TR)(pv9 * rpow<TS>(TS(2) - SBO, pv9 - TS(1))); sbo_region = 2; }
-    else { SBO2 = 2; CSBO2 = 0; sbo_region = 3; }
-    ev6 = safe_exp<TR>(p_val6 * Dboc);
+    TR SBO2 = 0, CSBO2 = 0;
+    const TS sx = SBO <= TS(1) ? SBO : TS(2) - SBO;
+    const TS pw = SBO > TS(0) && SBO < TS(2) ? rpow<TS>(sx, (p & 1) ? pv9 - TS(1) : pv9) : TS(0);
+    const TS pw0 = dpp<0xA0>(pw), pw1 = dpp<0xF5>(pw);   // quad_perm [0,0,2,2], [1,1,3,3]
+    if (SBO <= TS(0)) { sbo_region = 0; }
+    else if (SBO <= TS(1)) { SBO2 = (TR)pw0; CSBO2 = (TR)(pv9 * pw1); sbo_region = 1; }
+    else if (SBO < TS(2)) { SBO2 = (TR)(TS(2) - pw0); CSBO2 = (TR)(pv9 * pw1); sbo_region = 2; }
+    else { SBO2 = 2; sbo_region = 3; }
     const TR Delta = (TR)st.Delta[j], Dval = (TR)st.Delta_val[j];
     const TR ep3 = safe_exp<TR>(-p_pen3 * Delta), ep4 = safe_exp<TR>(p_pen4 * Delta), itrm = TR(1) / (TR(1) + ep3 + ep4);
-    f9 = (TR(2) + ep3) * itrm;
-    Cf9 = ratio2_deriv<TR>(ep3, ep4, -p_pen3, p_pen4, itrm);
-    ec2 = safe_exp<TR>(p_coa2 * Dval);
-  }
-  // this lane's bond (j, i)
-  const bool mine = act && p < nb;
-  size_t qi = 0;
-  int i = 0, ti = 0;
-  TR BOij = 0, BOA_ij = 0, dij = 1, tboi = 0;
-  TS BOij_s = 0;
-  V3<TR> vij{0, 0, 0};
-  if (mine) {
-    qi = sl(p, j, n);
-    BOij_s = (TS)st.bo[qi];
-    BOij = (TR)st.bo[qi];
-    BOA_ij = BOij - thb_cut;
-    i = st.b_j[qi]; ti = st.type[i];
-    vij = V3<TR>{(TR)st.b_dx[qi], (TR)st.b_dy[qi], (TR)st.b_dz[qi]};
-    dij = (TR)st.b_d[qi];
-    tboi = (TR)st.tbo[i];
+    const TR ev6 = safe_exp<TR>(p_val6 * Dboc), f9 = (TR(2) + ep3) * itrm, Cf9 = ratio2_deriv<TR>(ep3, ep4, -p_pen3, p_pen4, itrm);
+    const TR ec2 = safe_exp<TR>(p_coa2 * Dval);
+    if (p == 0) {
+      const int c = lane / G;
+      L.centre[0][c] = SBO2; L.centre[1][c] = CSBO2; L.centre[2][c] = dSBO2; L.centre[3][c] = ev6; L.centre[4][c] = f9;
+      L.centre[5][c] = Cf9; L.centre[6][c] = ec2; L.centre[7][c] = Dboc; L.centre[8][c] = (TR)sj.p_val3; L.centre[9][c] = (TR)sj.p_val5;
+    }
   }
   double vA[6] = {0, 0, 0, 0, 0, 0}, vC[6] = {0, 0, 0, 0, 0, 0};   // PA: slot p's partner, the centre (this lane's angles)
-  for (int pk = 1; pk < nbw; ++pk) {
-    double to_cdbo = 0, to_cdp = 0, to_fx = 0, to_fy = 0, to_fz = 0;
-    double vto[6] = {0, 0, 0, 0, 0, 0};
+  double to_cdbo = 0, to_cdp = 0, to_fx = 0, to_fy = 0, to_fz = 0;   // this lane's contributions to the row's slot k
+  double vto[6] = {0, 0, 0, 0, 0, 0};
+  ItemRows Q;
+  // rows (slot k, parameter set) until the next one does not fit, then the queue, and on from that row
+  int pk = 1, a = 0;
+  bool any = false;   // slot pk has items
+  int2 ai = make_int2(0, 0);
+  auto gates = [&]() {   // this lane's parameter sets of the pair (p, pk)
+    ai = make_int2(0, 0);
     if (mine && p < pk && pk < nb && BOij_s - thb_cut_s > TS(0)) {
-      const size_t qk = sl(pk, j, n);
-      const TS BOjk_s = (TS)st.bo[qk];
-      const TR BOjk = (TR)st.bo[qk];
-      const TR BOA_jk = BOjk - thb_cut;
-      const int k = st.b_j[qk], tk = st.type[k];
-      const int2 ai = t.angle_idx[(ti * g.ntypes + tj) * g.ntypes + tk];
+      const TS BOjk_s = L.bo[base + pk];
       const bool gate = BOjk_s - thb_cut_s > TS(0) && BOij_s > thb_cut_s && BOjk_s > thb_cut_s && BOij_s * BOjk_s > thb_cutsq_s;
       n_ang += gate ? 1 : 0;
-      if (gate && ai.y != 0) {
-        const V3<TR> vjk{(TR)st.b_dx[qk], (TR)st.b_dy[qk], (TR)st.b_dz[qk]};
-        const TR djk = (TR)st.b_d[qk];
-        TR th, ct, sth;
-        V3<TR> dci, dcj, dck;
-        angle_and_dcos<TR>(vij, dij, vjk, djk, th, ct, sth, dci, dcj, dck);
-        if (sth < TR(1.0e-5)) sth = TR(1.0e-5);
-        const TR tbok = (TR)st.tbo[k];
-        for (int a = 0; a < ai.y; ++a) {
-          const DevAngle A = t.angle[ai.x + a];
-          const TR p_val1 = (TR)A.p_val1;
-          if (!(fabs((double)p_val1) > 0.001)) continue;
-          const TR p_val2 = (TR)A.p_val2, p_val4 = (TR)A.p_val4, p_val7 = (TR)A.p_val7, th00 = (TR)A.theta_00;
-          const TR e3ij = rexp<TR>(-p_val3 * rpow<TR>(BOA_ij, p_val4)), f7ij = TR(1) - e3ij;
-          const TR Cf7ij = p_val3 * p_val4 * rpow<TR>(BOA_ij, p_val4 - TR(1)) * e3ij;
-          const TR e3jk = rexp<TR>(-p_val3 * rpow<TR>(BOA_jk, p_val4)), f7jk = TR(1) - e3jk;
-          const TR Cf7jk = p_val3 * p_val4 * rpow<TR>(BOA_jk, p_val4 - TR(1)) * e3jk;
-          const TR ev7 = safe_exp<TR>(-p_val7 * Dboc), itrm8 = TR(1) / (TR(1) + ev6 + ev7);
-          const TR f8 = p_val5 - (p_val5 - TR(1)) * ((TR(2) + ev6) * itrm8);
-          const TR Cf8 = (TR(1) - p_val5) * ratio2_deriv<TR>(ev6, ev7, p_val6, -p_val7, itrm8);
-          const TR th0 = (TR(180.0) - th00 * (TR(1) - rexp<TR>(-p_val10 * (TR(2) - SBO2)))) * TR(3.14159265) / TR(180.0);
-          const TR e2t = rexp<TR>(-p_val2 * ((th0 - th) * (th0 - th)));
-          const TR e12t = p_val1 >= TR(0) ? p_val1 * (TR(1) - e2t) : p_val1 * -e2t;
-          const TR CE1 = Cf7ij * f7jk * f8 * e12t, CE2 = Cf7jk * f7ij * f8 * e12t, CE3 = Cf8 * f7ij * f7jk * e12t;
-          const TR CE4 = -TR(2) * p_val1 * p_val2 * f7ij * f7jk * f8 * e2t * (th0 - th);
-          const TR Cth0 = p_val10 * (th00 * TR(3.14159265) / TR(180.0)) * rexp<TR>(-p_val10 * (TR(2) - SBO2));
-          const TR CE5 = -CE4 * Cth0 * CSBO2, CE6 = CE5 * dSBO1, CE7 = CE5 * dSBO2, CE8 = -CE4 / sth;
-          e_ang += (double)(f7ij * f7jk * f8 * e12t);
-          const TR p_pen1 = (TR)A.p_pen1;
-          const TR ep2ij = rexp<TR>(-p_pen2 * ((BOA_ij - TR(2)) * (BOA_ij - TR(2)))), ep2jk = rexp<TR>(-p_pen2 * ((BOA_jk - TR(2)) * (BOA_jk - TR(2))));
-          const TR epen = p_pen1 * f9 * ep2ij * ep2jk;
-          e_pen += (double)epen;
-          const TR CEp1 = epen * Cf9 / f9, tp = -TR(2) * p_pen2 * epen, CEp2 = tp * (BOA_ij - TR(2)), CEp3 = tp * (BOA_jk - TR(2));
-          const TR p_coa1 = (TR)A.p_coa1;
-          const TR dti = tboi - BOA_ij, dtk = tbok - BOA_jk;
-          const TR ecoa = p_coa1 / (TR(1) + ec2) * rexp<TR>(-p_coa3 * (dti * dti)) * rexp<TR>(-p_coa3 * (dtk * dtk)) *
-                          rexp<TR>(-p_coa4 * ((BOA_ij - TR(1.5)) * (BOA_ij - TR(1.5)))) * rexp<TR>(-p_coa4 * ((BOA_jk - TR(1.5)) * (BOA_jk - TR(1.5))));
-          e_coa += (double)ecoa;
-          const TR CEc1 = -TR(2) * p_coa4 * (BOA_ij - TR(1.5)) * ecoa, CEc2 = -TR(2) * p_coa4 * (BOA_jk - TR(1.5)) * ecoa;
-          const TR CEc3 = -p_coa2 * (ec2 / (TR(1) + ec2)) * ecoa, CEc4 = -TR(2) * p_coa3 * dti * ecoa, CEc5 = -TR(2) * p_coa3 * dtk * ecoa;
-          own_cdbo += (double)(CE1 + CEp2 + (CEc1 - CEc4));
-          to_cdbo += (double)(CE2 + CEp3 + (CEc2 - CEc5));
-          cdself += (double)((CE3 + CE7) + CEp1 + CEc3);
-          own_cdp += (double)CEc4;
-          to_cdp += (double)CEc5;
-          sCE5 += (double)CE5;
-          sCE6 += (double)CE6;
-          fjx += (double)(CE8 * dcj.x); fjy += (double)(CE8 * dcj.y); fjz += (double)(CE8 * dcj.z);
-          own_fx += (double)(CE8 * dci.x); own_fy += (double)(CE8 * dci.y); own_fz += (double)(CE8 * dci.z);
-          to_fx += (double)(CE8 * dck.x); to_fy += (double)(CE8 * dck.y); to_fz += (double)(CE8 * dck.z);
-          if (PA) {   // F_i = -CE8 dcos/dx_i, F_k = -CE8 dcos/dx_k
-            vir_add(vto, -1.0, (double)vij.x, (double)vij.y, (double)vij.z, (double)(CE8 * dci.x), (double)(CE8 * dci.y),
-                    (double)(CE8 * dci.z));
-            vir_add(vto, -1.0, (double)vjk.x, (double)vjk.y, (double)vjk.z, (double)(CE8 * dck.x), (double)(CE8 * dck.y),
-                    (double)(CE8 * dck.z));
+      if (gate) ai = t.angle_idx[(ti * g.ntypes + tj) * g.ntypes + L.type[base + pk]];
+    }
+  };
+  if (pk < nbw) gates();
+  for (;;) {
+    while (pk < nbw) {
+      if (__any(a < ai.y)) {
+        const bool item = a < ai.y && fabs((double)(TR)t.angle[ai.x + a].p_val1) > 0.001;
+        const unsigned long long mk = __ballot(item);
+        if (mk) {
+          if (!Q.fits(mk)) break;
+          const int e = Q.add(mk, pk);
+          if (item) { L.who[e] = lane | (base + pk) << 8; L.set[e] = ai.x + a; }
+          any = true;
+        }
+        ++a;
+      } else {
+        if (any) {
+          if (!Q.fits(0)) break;
+          Q.add(0, pk | kRowClose);
+        }
+        ++pk;
+        a = 0;
+        any = false;
+        if (pk < nbw) gates();
+      }
+    }
+    if (!Q.rows) break;
+    __builtin_amdgcn_wave_barrier();
+    if (lane < Q.items) valence_item<TR, TS, G>(g, t, L, lane);
+    __builtin_amdgcn_wave_barrier();
+    for (int r = 0; r < Q.rows; ++r) {
+      const int tag = Q.tag_of(r), pk = tag & 0xFFFF;
+      const unsigned long long mask = Q.mask_of(r);
+      if (mask >> lane & 1) {
+        const int e = Q.start_of(r) + lanes_below(mask);
+        auto R = [&](int c) { return L.res[c][e]; };
+        const TR CE5 = R(V_CE5), CE8 = R(V_CE8);
+        e_ang += (double)(R(V_ANG) * R(V_ANG + 1));
+        e_pen += (double)R(V_PEN);
+        e_coa += (double)R(V_COA);
+        own_cdbo += (double)R(V_OWN_CDBO);
+        to_cdbo += (double)R(V_TO_CDBO);
+        cdself += (double)R(V_CDSELF);
+        own_cdp += (double)R(V_OWN_CDP);
+        to_cdp += (double)R(V_TO_CDP);
+        sCE5 += (double)CE5;
+        sCE6 += (double)rounded(CE5 * dSBO1);
+        fjx += (double)(CE8 * R(V_DCJ)); fjy += (double)(CE8 * R(V_DCJ + 1)); fjz += (double)(CE8 * R(V_DCJ + 2));
+        own_fx += (double)(CE8 * R(V_DCI)); own_fy += (double)(CE8 * R(V_DCI + 1)); own_fz += (double)(CE8 * R(V_DCI + 2));
+        to_fx += (double)(CE8 * R(V_DCK)); to_fy += (double)(CE8 * R(V_DCK + 1)); to_fz += (double)(CE8 * R(V_DCK + 2));
+        if (PA) {   // F_i = -CE8 dcos/dx_i, F_k = -CE8 dcos/dx_k
+          vir_add(vto, -1.0, (double)vij.x, (double)vij.y, (double)vij.z, (double)(CE8 * R(V_DCI)), (double)(CE8 * R(V_DCI + 1)),
+                  (double)(CE8 * R(V_DCI + 2)));
+          vir_add(vto, -1.0, (double)L.x[base + pk], (double)L.y[base + pk], (double)L.z[base + pk], (double)(CE8 * R(V_DCK)),
+                  (double)(CE8 * R(V_DCK + 1)), (double)(CE8 * R(V_DCK + 2)));
+        }
+      }
+      if (tag & kRowClose) {
+        to_cdbo = gsum<G>(to_cdbo); to_cdp = gsum<G>(to_cdp); to_fx = gsum<G>(to_fx); to_fy = gsum<G>(to_fy); to_fz = gsum<G>(to_fz);
+        if (p == pk) { own_cdbo += to_cdbo; own_cdp += to_cdp; own_fx += to_fx; own_fy += to_fy; own_fz += to_fz; }
+        to_cdbo = to_cdp = to_fx = to_fy = to_fz = 0;
+        if (PA) {
+          for (int c = 0; c < 6; ++c) {
+            vA[c] += vto[c];
+            vC[c] += vto[c];
+            const double tk = gsum<G>(vto[c]);
+            if (p == pk) vA[c] += tk;
+            vto[c] = 0;
           }
         }
       }
     }
-    to_cdbo = gsum<G>(to_cdbo); to_cdp = gsum<G>(to_cdp); to_fx = gsum<G>(to_fx); to_fy = gsum<G>(to_fy); to_fz = gsum<G>(to_fz);
-    if (p == pk) { own_cdbo += to_cdbo; own_cdp += to_cdp; own_fx += to_fx; own_fy += to_fy; own_fz += to_fz; }
-    if (PA) {
-      for (int c = 0; c < 6; ++c) {
-        vA[c] += vto[c];
-        vC[c] += vto[c];
-        const double tk = gsum<G>(vto[c]);
-        if (p == pk) vA[c] += tk;
-      }
-    }
+    Q.clear();
+    __builtin_amdgcn_wave_barrier();
   }
   e_ang = gsum<G>(e_ang); e_pen = gsum<G>(e_pen); e_coa = gsum<G>(e_coa); cdself = gsum<G>(cdself);
   fjx = gsum<G>(fjx); fjy = gsum<G>(fjy); fjz = gsum<G>(fjz); sCE5 = gsum<G>(sCE5); sCE6 = gsum<G>(sCE6);
@@ -838,16 +975,15 @@ __device__ inline void valence_body(const State& st, const Globals& g, const Tab
   }
 }
 
-// FP32 terms at the compiler's choice of registers; FP64 terms held to 256 VGPRs, 2 waves per SIMD (the compiler's choice, 260
-// VGPRs, leaves one): the bound spills two 8-byte values before the partner loop, reloaded once per partner k outside the
-// angle arithmetic, and gains 2-4% of the FP64 step
 template <class TS, int G, bool PA>
-__global__ void __launch_bounds__(256) k_valence(State st, Globals g, Tables t) {
-  valence_body<float, TS, G, PA>(st, g, t);
+__global__ void __launch_bounds__(64 * kAngleWaves) k_valence(State st, Globals g, Tables t) {
+  __shared__ ValenceLds<float, TS> L[kAngleWaves];
+  valence_body<float, TS, G, PA>(st, g, t, L[threadIdx.x >> 6]);
 }
 template <int G, bool PA>
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256) k_valence_d(State st, Globals g, Tables t) {
-  valence_body<double, double, G, PA>(st, g, t);
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_valence_d(State st, Globals g, Tables t) {
+  __shared__ ValenceLds<double, double> L[kAngleWaves];
+  valence_body<double, double, G, PA>(st, g, t, L[threadIdx.x >> 6]);
 }
 
 template <class TR>
