@@ -9,7 +9,7 @@
 //   atom_terms  (thread per atom) bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
 //   valence     (wave per 64 / G atoms, angles spread over its lanes) valence angle, penalty, 3-body conjugation at the centre
 //                                 [bonded.cpp:321-474]
-//   torsion     (thread per atom) torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
+//   torsion     (as valence)      torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
 //                                 and derivative contributions of its own half (its own atom, its outer partner, its outer bond) and
 //                                 the end the reference counts (tag order) adds the energy and the central-bond terms [bonded.cpp:476-652]
 //   hbond       (wave per atom)   donor hydrogens evaluate their H-bond triples once and leave the acceptor's force in the
@@ -680,7 +680,7 @@ constexpr int kAngleWaves = 4;       // waves per block of the angle kernels
 // Bound by the arithmetic of an angle: 11 exponentials, 4 powers (FP64: also the arc cosine), in FP64 some 2000 instructions, run once
 // per 64 angles now. The centre's powers run once each, on the even and the odd lanes of the group. The term kernels of a step
 // (this, torsion, hydrogen bonds) took, before and with this: 648 atoms of water mixed 147 -> 120 us, 24000 269 -> 235 us, 192000 1729 ->
-// 1553 us, FP64 24000 381 -> 325 us, 30000 atoms of disordered carbon mixed 373 -> 336 us. LDS: 6.5 KB per wave in FP32, 13 KB in FP64.
+// 1553 us, FP64 24000 381 -> 325 us, 30000 atoms of disordered carbon mixed 373 -> 336 us. LDS per wave: FP32 8.4, mixed 9.1, FP64 16 KB.
 //
 // Results of an item. A product that the sum takes in by a fused multiply-add is kept as its two factors; a value with other uses,
 // and what rounded() marks, enters rounded. So the sums are those of a loop over the angles in place, bit for bit.
@@ -995,189 +995,283 @@ __device__ inline TR tan_inv(TR s, TR c) {
 }
 
 // Torsion + four-body conjugation [reference bonded.cpp:476-652], evaluated at BOTH atoms of the central bond: lane p of j's group
-// takes the central bond (j, k) in slot p and walks j's other bonds i (wave-uniform loop) and k's other bonds l. Each end keeps
+// owns the central bond (j, k) in slot p and with it the torsions over j's other bonds i and k's other bonds l. Each end keeps
 // its own half (its atom, its outer partner i and outer bond (j, i)); the end the reference counts (canonical_first) also adds
 // the energy and the central-bond coefficients. The outer-bond contributions of an i are summed over the group and kept by the
 // lane owning slot i.
+// Rows: slot of i, then each owner's next bond of k that passes the gate on the bond orders (found with k's bond orders in LDS);
+// the gates that need l itself are the item's. The outer-bond terms of an i are summed in TR over the owner's bonds of k, as in a
+// loop, and the sums carried over a queue that fills in between.
+// Bound by the arithmetic of a torsion (4 square roots, 15 divisions, 3 exponentials) and, on small systems, by the chain of loads of an
+// item (l, its type, the index, the parameters): 25 us at 648 atoms, where a wave empties its queue a few times. The term kernels of a step (valence,
+// torsion, hydrogen bonds), with the loops in place and with this: 648 atoms of water mixed 120 -> 80 us, 24000 235 -> 187 us, 192000
+// 1553 -> 1235 us, FP64 24000 325 -> 251 us, 30000 atoms of disordered carbon mixed 336 -> 188 us. LDS per wave: FP32 9, mixed 11,
+// FP64 16.6 KB.
 // PA: also the reference's per-atom virial split (bonded.cpp:636-647): each torsion's (x_l - x_i) (x) g_i + (x_l - x_j) (x) g_j +
 // (x_l - x_k) (x) g_k (g the gradients), a quarter to each of its four atoms. Both ends evaluate every torsion, so each end gives
 // the quarters of its own two atoms (j and the outer partner i, through i's slot).
+enum TorResult {
+  R_CDBO, R_FI, R_FJ = R_FI + 3,                       // this end's outer bond, forces on i and j
+  R_CT2 = R_FJ + 3, R_JK,                              // central bond: d / d BOpi (times dfn11: the end's CdDelta), d / d BO
+  R_TOR, R_CON = R_TOR + 2, kTorResults = R_CON + 2    // energies (two factors each)
+};
+constexpr int kFarBonds = 8;   // bond orders of k's bonds kept in LDS per central bond (further ones are read again)
+template <class TR, class TS, bool PA>
+struct TorsionLds {   // one wave
+  TS bo[64];                                           // lane: its bond, as an outer one
+  TR x[64], y[64], z[64], d[64], boa[64], et2[64], ec2[64];
+  int j[64], s[64], type[64], tj[64];
+  TR x11[64];                                          // lane: its bond as a central one: 2 - BO_pi - f11
+  TS far[kFarBonds][64];
+  int who[64];                                         // item: owner lane | lane of i << 6 | slot of l in k's list << 12; -1: no torsion
+  TR res[kTorResults][64];
+  double vir[PA ? 6 : 1][PA ? 64 : 1];
+};
+
+// item e: the torsion i - j - k - l, its gates on l's image and parameter set first
+template <class TR, class TS, bool PA>
+__device__ inline void torsion_item(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L, int e) {
+  const int who = L.who[e], a = who & 63, b = who >> 6 & 63, pl = who >> 12, n = st.n;
+  const int k = L.j[a], sk = L.s[a], i = L.j[b], si = L.s[b];
+  const size_t ql = sl(pl, k, n);
+  const int l = st.b_j[ql], sl_abs = shift_add(sk, st.b_s[ql]), tl = st.type[l];
+  const TR BOkl = (TR)st.bo[ql], rkl = (TR)st.b_d[ql];
+  const V3<TR> dkl{(TR)st.b_dx[ql], (TR)st.b_dy[ql], (TR)st.b_dz[ql]};
+  const int ti4 = t.tors_idx[((L.type[b] * g.ntypes + L.tj[a]) * g.ntypes + L.type[a]) * g.ntypes + tl];
+  if ((l == i && sl_abs == si) || ti4 < 0) {   // i and l are the same image, or no such torsion
+    L.who[e] = -1;
+    return;
+  }
+  const DevTorsion P = t.tors[ti4];
+  const TR thb_cut = (TR)g.thb_cut;
+  const TR p_tor2 = (TR)g.p_tor2, p_cot2 = (TR)g.p_cot2;
+  const TR MINS = TR(1e-10);
+  const TR rij = L.d[b], rjk = L.d[a], BOA_ij = L.boa[b], BOA_jk = L.boa[a], BOA_kl = BOkl - thb_cut;
+  const TR et2ij = L.et2[b], et2jk = L.et2[a], ec2ij = L.ec2[b], ec2jk = L.ec2[a];
+  const V3<TR> dji{L.x[b], L.y[b], L.z[b]}, djk{L.x[a], L.y[a], L.z[a]}, dkj{-djk.x, -djk.y, -djk.z};
+  TR thijk, cijk_, sijk;
+  V3<TR> dci, dcj, dck;   // d cos(theta_ijk) / d x_i, x_j, x_k
+  angle_and_dcos<TR, false>(dji, rij, djk, rjk, thijk, cijk_, sijk, dci, dcj, dck);
+  const TR cijk = cijk_, tijk = tan_inv<TR>(sijk, cijk);
+  TR thjkl, cjkl_, sjkl;
+  V3<TR> ecj, eck, ecl;   // d cos(theta_jkl) / d x_j, x_k, x_l
+  angle_and_dcos<TR, false>(dkj, rjk, dkl, rkl, thjkl, cjkl_, sjkl, ecj, eck, ecl);
+  const TR cjkl = cjkl_, tjkl = tan_inv<TR>(sjkl, cjkl);
+  // x_i - x_l in j's frame
+  const V3<TR> dli{dji.x - djk.x - dkl.x, dji.y - djk.y - dkl.y, dji.z - djk.z - dkl.z};
+  const TR rli = rsqrt_<TR>(dot3(dli, dli));
+  TR s1 = sijk, c1 = cijk, s2 = sjkl, c2 = cjkl;
+  if (s1 >= TR(0) && s1 <= MINS) s1 = MINS; else if (s1 <= TR(0) && s1 >= -MINS) s1 = -MINS;
+  if (s2 >= TR(0) && s2 <= MINS) s2 = MINS; else if (s2 <= TR(0) && s2 >= -MINS) s2 = -MINS;
+  // bond vectors in the reference's orientation: dij (j->i), djk (j->k), dkl (k->l)
+  const V3<TR>& bij = dji;
+  const TR rjk2 = rounded(rjk * rjk), hjk = rjk - rij * c1;
+  const TR ucos = -dot3(bij, djk) * dot3(djk, dkl) + rjk2 * dot3(bij, dkl);
+  const TR usin = -rjk * dot3(bij, cross3(djk, dkl));
+  const TR htra = rij + c1 * (rkl * c2 - rjk), htrb = hjk - rkl * c2;
+  const TR hthd = rij * s1 * (rjk - rkl * c2), hthe = rkl * s2 * hjk;
+  const TR hnra = rkl * s1 * s2, hnhd = rij * rkl * c1 * s2, hnhe = rij * rkl * s1 * c2;
+  const TR tel = rounded(rij * rij + rjk2) + (rkl * rkl) - (rli * rli) -
+                 TR(2) * (rij * rjk * c1 - rij * rkl * c1 * c2 + rjk * rkl * c2);
+  const TR poem = TR(2) * rij * rkl * s1 * s2;
+  TR arg = tel / poem;
+  if (arg > TR(1)) arg = TR(1);
+  if (arg < TR(-1)) arg = TR(-1);
+  const TR ga = (htra - arg * hnra) / rij, gd = -(hthd - arg * hnhd) / s1, ge = -(hthe - arg * hnhe) / s2;
+  const TR sc = TR(2) / poem;
+  // d omega-like derivative vectors of i and j (the reference's dcos_omega_di / _dj)
+  const V3<TR> doi{sc * (ga * bij.x - dli.x + gd * dci.x), sc * (ga * bij.y - dli.y + gd * dci.y), sc * (ga * bij.z - dli.z + gd * dci.z)};
+  const V3<TR> doj{sc * (-ga * bij.x - htrb / rjk * djk.x + gd * dcj.x + ge * ecj.x), sc * (-ga * bij.y - htrb / rjk * djk.y + gd * dcj.y + ge * ecj.y),
+                   sc * (-ga * bij.z - htrb / rjk * djk.z + gd * dcj.z + ge * ecj.z)};
+  // cos(omega) for omega = atan2(usin, ucos), and cos(2 omega), cos(3 omega) by the multiple-angle identities (the
+  // reference's cos(atan2(..)), cos(2 omega), cos(3 omega) to within a few ulp, without the four trigonometric calls;
+  // atan2(0, 0) = 0 gives cos = 1)
+  const TR h2 = ucos * ucos + usin * usin;
+  const TR cw = h2 > TR(0) ? ucos / rsqrt_<TR>(h2) : TR(1);
+  const TR c2w = TR(2) * (cw * cw) - TR(1), c3w = (TR(4) * (cw * cw) - TR(3)) * cw;
+  const TR x = L.x11[a];
+  const TR et1 = rexp<TR>((TR)P.p_tor1 * (x * x));
+  const TR et2kl = rexp<TR>(-p_tor2 * BOA_kl), ec2kl = rexp<TR>(-p_cot2 * ((BOA_kl - TR(1.5)) * (BOA_kl - TR(1.5))));
+  const TR fn10 = (TR(1) - et2ij) * (TR(1) - et2jk) * (TR(1) - et2kl);
+  const TR V1 = (TR)P.V1, V2 = (TR)P.V2, V3_ = (TR)P.V3, p_tor1 = (TR)P.p_tor1, p_cot1 = (TR)P.p_cot1;
+  const TR CV = TR(0.5) * (V1 * (TR(1) + cw) + V2 * et1 * (TR(1) - c2w) + V3_ * (TR(1) + c3w));
+  const TR CT1 = sijk * sjkl * CV;
+  const TR CT2 = -fn10 * TR(2) * p_tor1 * V2 * et1 * x * (TR(1) - (cw * cw)) * sijk * sjkl;
+  const TR CT4 = CT1 * p_tor2 * et2ij * (TR(1) - et2jk) * (TR(1) - et2kl);
+  const TR CT5 = CT1 * p_tor2 * (TR(1) - et2ij) * et2jk * (TR(1) - et2kl);
+  const TR cmn = -fn10 * CV, CT7 = cmn * sjkl * tijk, CT8 = cmn * sijk * tjkl;
+  const TR CT9 = fn10 * sijk * sjkl * (TR(0.5) * V1 - TR(2) * V2 * et1 * cw + TR(1.5) * V3_ * (c2w + TR(2) * (cw * cw)));
+  const TR fn12 = ec2ij * ec2jk * ec2kl;
+  const TR gg = TR(1) + ((cw * cw) - TR(1)) * sijk * sjkl;
+  const TR Cc = -TR(2) * fn12 * p_cot1 * p_cot2 * gg;
+  const TR CC1 = Cc * (BOA_ij - TR(1.5)), CC2 = Cc * (BOA_jk - TR(1.5));
+  const TR CC4 = -p_cot1 * fn12 * ((cw * cw) - TR(1)) * sjkl * tijk;
+  const TR CC5 = -p_cot1 * fn12 * ((cw * cw) - TR(1)) * sijk * tjkl;
+  const TR CC6 = TR(2) * p_cot1 * fn12 * cw * sijk * sjkl;
+  const TR a7 = CT7 + CC4, a8 = CT8 + CC5, a9 = CT9 + CC6;
+  const TR gix = a7 * dci.x + a9 * doi.x, giy = a7 * dci.y + a9 * doi.y, giz = a7 * dci.z + a9 * doi.z;
+  const TR gjx = a7 * dcj.x + a8 * ecj.x + a9 * doj.x, gjy = a7 * dcj.y + a8 * ecj.y + a9 * doj.y, gjz = a7 * dcj.z + a8 * ecj.z + a9 * doj.z;
+  L.res[R_CDBO][e] = CT4 + CC1;
+  L.res[R_FI][e] = gix; L.res[R_FI + 1][e] = giy; L.res[R_FI + 2][e] = giz;
+  L.res[R_FJ][e] = gjx; L.res[R_FJ + 1][e] = gjy; L.res[R_FJ + 2][e] = gjz;
+  L.res[R_CT2][e] = CT2; L.res[R_JK][e] = CT5 + CC2;
+  L.res[R_TOR][e] = fn10 * sijk * sjkl; L.res[R_TOR + 1][e] = CV;
+  L.res[R_CON][e] = p_cot1 * fn12; L.res[R_CON + 1][e] = gg;
+  if (PA) {   // g_k with the reference's dcos(omega)/dx_k; positions relative to l: x_l - x_i = -dli, x_l - x_j = djk + dkl
+    const TR htrc = rkl - c2 * hjk, hnrc = rij * s1 * s2, gcl = (htrc - arg * hnrc) / rkl;
+    const V3<TR> dok{sc * (-gcl * dkl.x + htrb / rjk * djk.x + gd * dck.x + ge * eck.x),
+                     sc * (-gcl * dkl.y + htrb / rjk * djk.y + gd * dck.y + ge * eck.y),
+                     sc * (-gcl * dkl.z + htrb / rjk * djk.z + gd * dck.z + ge * eck.z)};
+    const double gkx = (double)(a7 * dck.x + a8 * eck.x + a9 * dok.x), gky = (double)(a7 * dck.y + a8 * eck.y + a9 * dok.y),
+                 gkz = (double)(a7 * dck.z + a8 * eck.z + a9 * dok.z);
+    double v[6] = {0, 0, 0, 0, 0, 0};
+    vir_add(v, -1.0, (double)dli.x, (double)dli.y, (double)dli.z, (double)gix, (double)giy, (double)giz);
+    vir_add(v, 1.0, (double)(djk.x + dkl.x), (double)(djk.y + dkl.y), (double)(djk.z + dkl.z), (double)gjx, (double)gjy, (double)gjz);
+    vir_add(v, 1.0, (double)dkl.x, (double)dkl.y, (double)dkl.z, gkx, gky, gkz);
+    for (int c = 0; c < 6; ++c) L.vir[c][e] = v[c];
+  }
+}
+
 template <class TR, class TS, int G, bool kCen, bool PA>
-__device__ __forceinline__ void torsion_body(State st, Globals g, Tables t) {
+__device__ inline void torsion_body(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L) {
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = gid / G, pk = gid % G, n = st.n;
+  const int j = gid / G, pk = gid % G, n = st.n, lane = lane_id(), base = lane - pk;
   const bool live = j < n;
   const int tj = live ? st.type[j] : -1;
   const int nbj = live ? min(st.b_cnt[j], st.maxb) : 0;
   const int nbw = wave_max(nbj);
   double e_tor = 0, e_con = 0, cdself = 0, fjx = 0, fjy = 0, fjz = 0;
-  double own_fx = 0, own_fy = 0, own_fz = 0;
+  double own_c = 0, own_fx = 0, own_fy = 0, own_fz = 0;
   double fIx = 0, fIy = 0, fIz = 0;   // this lane's forces on the outer partners i, summed (for the virial)
   const TR thb_cut = (TR)g.thb_cut;
   const TS thb_cut_s = (TS)g.thb_cut;
   const TR p_tor2 = (TR)g.p_tor2, p_tor3 = (TR)g.p_tor3, p_tor4 = (TR)g.p_tor4, p_cot2 = (TR)g.p_cot2;
-  const TR MINS = TR(1e-10);
-  // this lane's central bond (j, k)
-  bool cen = live && tj >= 0 && nbj >= 2 && pk < nbj;
-  size_t qk = 0;
-  int k = 0, sk = 0, tk = 0, nbk = 0, symk = 0;
-  bool counted = false;
-  TR BOjk = 0, BOA_jk = 0, rjk = 1, et2jk = 0, ec2jk = 0, f11 = 0, dfn11 = 0, BOpijk = 0;
-  V3<TR> djk{0, 0, 0}, dkj{0, 0, 0};
-  if (cen) {
-    qk = sl(pk, j, n);
-    BOjk = (TR)st.bo[qk];
-    k = st.b_j[qk]; sk = st.b_s[qk]; tk = st.type[k];
-    nbk = min(st.b_cnt[k], st.maxb);
-    cen = (TS)st.bo[qk] > thb_cut_s && nbk >= 2;
-  }
-  if (cen) {
-    counted = canonical_first(j, k, sk, st.tag);
-    symk = st.b_sym[qk];   // slot of j in k's list
-    BOA_jk = BOjk - thb_cut;
-    rjk = (TR)st.b_d[qk];
+  // this lane's bond (j, k): an outer one of the other lanes' torsions, and the central one of its own
+  const bool bond = live && tj >= 0 && nbj >= 2 && pk < nbj;
+  const size_t qk = bond ? sl(pk, j, n) : 0;
+  bool cen = false, counted = false;
+  int k = 0, symk = 0;
+  TS BOjk_s = 0;
+  TR dfn11 = 0;
+  V3<TR> djk{0, 0, 0};
+  unsigned long long far = 0;   // slots of k's bonds (k, l) that can be outer ones
+  if (bond) {
+    BOjk_s = (TS)st.bo[qk];
+    k = st.b_j[qk];
+    const int sk = st.b_s[qk], nbk = min(st.b_cnt[k], st.maxb);
+    const TR BOjk = (TR)st.bo[qk], BOA_jk = BOjk - thb_cut;
     djk = V3<TR>{(TR)st.b_dx[qk], (TR)st.b_dy[qk], (TR)st.b_dz[qk]};
-    dkj = V3<TR>{-djk.x, -djk.y, -djk.z};
-    const TR Dj = (TR)st.Delta_boc[j], Dk = (TR)st.Delta_boc[k];
-    et2jk = rexp<TR>(-p_tor2 * BOA_jk);
-    ec2jk = rexp<TR>(-p_cot2 * ((BOA_jk - TR(1.5)) * (BOA_jk - TR(1.5))));
-    const TR et3 = safe_exp<TR>(-p_tor3 * (Dj + Dk)), et4 = safe_exp<TR>(p_tor4 * (Dj + Dk)), it34 = TR(1) / (TR(1) + et3 + et4);
-    f11 = (TR(2) + et3) * it34;
-    BOpijk = (TR)st.bo_pi[qk];
-    dfn11 = ratio2_deriv<TR>(et3, et4, -p_tor3, p_tor4, it34);
+    L.x[lane] = djk.x; L.y[lane] = djk.y; L.z[lane] = djk.z; L.d[lane] = (TR)st.b_d[qk];
+    L.boa[lane] = BOA_jk;
+    L.et2[lane] = rexp<TR>(-p_tor2 * BOA_jk);
+    L.ec2[lane] = rexp<TR>(-p_cot2 * ((BOA_jk - TR(1.5)) * (BOA_jk - TR(1.5))));
+    L.j[lane] = k; L.s[lane] = sk; L.type[lane] = st.type[k]; L.tj[lane] = tj;
+    cen = BOjk_s > thb_cut_s && nbk >= 2;
+    if (cen) {
+      counted = canonical_first(j, k, sk, st.tag);
+      symk = st.b_sym[qk];   // slot of j in k's list
+      const TR Dj = (TR)st.Delta_boc[j], Dk = (TR)st.Delta_boc[k];
+      const TR et3 = safe_exp<TR>(-p_tor3 * (Dj + Dk)), et4 = safe_exp<TR>(p_tor4 * (Dj + Dk)), it34 = TR(1) / (TR(1) + et3 + et4);
+      const TR f11 = (TR(2) + et3) * it34, BOpijk = (TR)st.bo_pi[qk];
+      dfn11 = ratio2_deriv<TR>(et3, et4, -p_tor3, p_tor4, it34);
+      L.x11[lane] = TR(2) - BOpijk - f11;
+      int c = 0;
+      for (int p0 = 0; p0 < nbk; p0 += 4) {
+        TS v[4];
+        for (int u = 0; u < 4; ++u) v[u] = (TS)st.bo[sl(min(p0 + u, nbk - 1), k, n)];
+        for (int u = 0; u < 4; ++u)
+          if (p0 + u < nbk && p0 + u != symk && v[u] > thb_cut_s) {
+            far |= 1ull << (p0 + u);
+            if (c < kFarBonds) L.far[c][lane] = v[u];
+            ++c;
+          }
+      }
+    }
   }
+  L.bo[lane] = BOjk_s;
+  __builtin_amdgcn_wave_barrier();
   double cdbo_jk = 0, cdbopi_jk = 0;
   int n_tor = 0;   // census: torsions through the four-body gates that this lane's central bond counts
   double vJ[6] = {0, 0, 0, 0, 0, 0}, vIown[6] = {0, 0, 0, 0, 0, 0};   // PA: j's quarters, this lane's slot partner's quarters
-  for (int pi = 0; pi < nbw; ++pi) {
-    TR cdbo_ij = 0, fix = 0, fiy = 0, fiz = 0;   // this lane's terms of partner i: at most one per bond of k
-    double vI[6] = {0, 0, 0, 0, 0, 0};
-    if (cen && pi != pk && pi < nbj) {
-      const size_t qi = sl(pi, j, n);
-      const TS BOij_s = (TS)st.bo[qi];
-      const TR BOij = (TR)st.bo[qi];
-      if (BOij_s > thb_cut_s) {
-        // the four-body gate's product, left to right as the reference (FP64 gates: the first two factors formed here)
-        const TS BOijk_s = sizeof(TS) == 8 ? BOij_s * (TS)st.bo[qk] : TS(0);
-        const int i = st.b_j[qi], si_ = st.b_s[qi], ti = st.type[i];
-        const TR rij = (TR)st.b_d[qi], BOA_ij = BOij - thb_cut;
-        const V3<TR> dji{(TR)st.b_dx[qi], (TR)st.b_dy[qi], (TR)st.b_dz[qi]};
-        TR thijk, cijk_, sijk;
-        V3<TR> dci, dcj, dck;   // d cos(theta_ijk) / d x_i, x_j, x_k
-        angle_and_dcos<TR, false>(dji, rij, djk, rjk, thijk, cijk_, sijk, dci, dcj, dck);
-        const TR cijk = cijk_, tijk = tan_inv<TR>(sijk, cijk);
-        const TR et2ij = rexp<TR>(-p_tor2 * BOA_ij), ec2ij = rexp<TR>(-p_cot2 * ((BOA_ij - TR(1.5)) * (BOA_ij - TR(1.5))));
-        for (int pl = 0; pl < nbk; ++pl) {
-          if (pl == symk) continue;
-          const size_t ql = sl(pl, k, n);
-          const TS BOkl_s = (TS)st.bo[ql];
-          if (!(BOkl_s > thb_cut_s)) continue;
-          const TR BOkl = (TR)st.bo[ql];
-          const int l = st.b_j[ql], sl_abs = shift_add(sk, st.b_s[ql]), tl = st.type[l];
-          if (l == i && sl_abs == si_) continue;   // i and l are the same image
-          const int ti4 = t.tors_idx[((ti * g.ntypes + tj) * g.ntypes + tk) * g.ntypes + tl];
-          if (ti4 < 0) continue;
-          if (sizeof(TS) == 8 ? !(BOijk_s * BOkl_s > thb_cut_s) : !(BOij * BOjk * BOkl > thb_cut)) continue;
-          if (kCen) n_tor += counted ? 1 : 0;
-          const DevTorsion P = t.tors[ti4];
-          const TR rkl = (TR)st.b_d[ql], BOA_kl = BOkl - thb_cut;
-          const V3<TR> dkl{(TR)st.b_dx[ql], (TR)st.b_dy[ql], (TR)st.b_dz[ql]};
-          TR thjkl, cjkl_, sjkl;
-          V3<TR> ecj, eck, ecl;   // d cos(theta_jkl) / d x_j, x_k, x_l
-          angle_and_dcos<TR, false>(dkj, rjk, dkl, rkl, thjkl, cjkl_, sjkl, ecj, eck, ecl);
-          const TR cjkl = cjkl_, tjkl = tan_inv<TR>(sjkl, cjkl);
-          // x_i - x_l in j's frame
-          const V3<TR> dli{dji.x - djk.x - dkl.x, dji.y - djk.y - dkl.y, dji.z - djk.z - dkl.z};
-          const TR rli = rsqrt_<TR>(dot3(dli, dli));
-          TR s1 = sijk, c1 = cijk, s2 = sjkl, c2 = cjkl;
-          if (s1 >= TR(0) && s1 <= MINS) s1 = MINS; else if (s1 <= TR(0) && s1 >= -MINS) s1 = -MINS;
-          if (s2 >= TR(0) && s2 <= MINS) s2 = MINS; else if (s2 <= TR(0) && s2 >= -MINS) s2 = -MINS;
-          // bond vectors in the reference's orientation: dij (j->i), djk (j->k), dkl (k->l)
-          const V3<TR>& bij = dji;
-          const TR ucos = -dot3(bij, djk) * dot3(djk, dkl) + (rjk * rjk) * dot3(bij, dkl);
-          const TR usin = -rjk * dot3(bij, cross3(djk, dkl));
-          const TR htra = rij + c1 * (rkl * c2 - rjk), htrb = rjk - rij * c1 - rkl * c2;
-          const TR hthd = rij * s1 * (rjk - rkl * c2), hthe = rkl * s2 * (rjk - rij * c1);
-          const TR hnra = rkl * s1 * s2, hnhd = rij * rkl * c1 * s2, hnhe = rij * rkl * s1 * c2;
-          const TR tel = (rij * rij) + (rjk * rjk) + (rkl * rkl) - (rli * rli) - TR(2) * (rij * rjk * c1 - rij * rkl * c1 * c2 + rjk * rkl * c2);
-          const TR poem = TR(2) * rij * rkl * s1 * s2;
-          TR arg = tel / poem;
-          if (arg > TR(1)) arg = TR(1);
-          if (arg < TR(-1)) arg = TR(-1);
-          const TR ga = (htra - arg * hnra) / rij, gd = -(hthd - arg * hnhd) / s1, ge = -(hthe - arg * hnhe) / s2;
-          const TR sc = TR(2) / poem;
-          // d omega-like derivative vectors of i and j (the reference's dcos_omega_di / _dj)
-          const V3<TR> doi{sc * (ga * bij.x - dli.x + gd * dci.x), sc * (ga * bij.y - dli.y + gd * dci.y), sc * (ga * bij.z - dli.z + gd * dci.z)};
-          const V3<TR> doj{sc * (-ga * bij.x - htrb / rjk * djk.x + gd * dcj.x + ge * ecj.x), sc * (-ga * bij.y - htrb / rjk * djk.y + gd * dcj.y + ge * ecj.y),
-                           sc * (-ga * bij.z - htrb / rjk * djk.z + gd * dcj.z + ge * ecj.z)};
-          // cos(omega) for omega = atan2(usin, ucos), and cos(2 omega), cos(3 omega) by the multiple-angle identities (the
-          // reference's cos(atan2(..)), cos(2 omega), cos(3 omega) to within a few ulp, without the four trigonometric calls;
-          // atan2(0, 0) = 0 gives cos = 1)
-          const TR h2 = ucos * ucos + usin * usin;
-          const TR cw = h2 > TR(0) ? ucos / rsqrt_<TR>(h2) : TR(1);
-          const TR c2w = TR(2) * (cw * cw) - TR(1), c3w = (TR(4) * (cw * cw) - TR(3)) * cw;
-          const TR x = TR(2) - BOpijk - f11;
-          const TR et1 = rexp<TR>((TR)P.p_tor1 * (x * x));
-          const TR et2kl = rexp<TR>(-p_tor2 * BOA_kl), ec2kl = rexp<TR>(-p_cot2 * ((BOA_kl - TR(1.5)) * (BOA_kl - TR(1.5))));
-          const TR fn10 = (TR(1) - et2ij) * (TR(1) - et2jk) * (TR(1) - et2kl);
-          const TR V1 = (TR)P.V1, V2 = (TR)P.V2, V3_ = (TR)P.V3, p_tor1 = (TR)P.p_tor1, p_cot1 = (TR)P.p_cot1;
-          const TR CV = TR(0.5) * (V1 * (TR(1) + cw) + V2 * et1 * (TR(1) - c2w) + V3_ * (TR(1) + c3w));
-          const TR CT1 = sijk * sjkl * CV;
-          const TR CT2 = -fn10 * TR(2) * p_tor1 * V2 * et1 * x * (TR(1) - (cw * cw)) * sijk * sjkl;
-          const TR CT3 = CT2 * dfn11;
-          const TR CT4 = CT1 * p_tor2 * et2ij * (TR(1) - et2jk) * (TR(1) - et2kl);
-          const TR CT5 = CT1 * p_tor2 * (TR(1) - et2ij) * et2jk * (TR(1) - et2kl);
-          const TR cmn = -fn10 * CV, CT7 = cmn * sjkl * tijk, CT8 = cmn * sijk * tjkl;
-          const TR CT9 = fn10 * sijk * sjkl * (TR(0.5) * V1 - TR(2) * V2 * et1 * cw + TR(1.5) * V3_ * (c2w + TR(2) * (cw * cw)));
-          const TR fn12 = ec2ij * ec2jk * ec2kl;
-          const TR gg = TR(1) + ((cw * cw) - TR(1)) * sijk * sjkl;
-          const TR Cc = -TR(2) * fn12 * p_cot1 * p_cot2 * gg;
-          const TR CC1 = Cc * (BOA_ij - TR(1.5)), CC2 = Cc * (BOA_jk - TR(1.5));
-          const TR CC4 = -p_cot1 * fn12 * ((cw * cw) - TR(1)) * sjkl * tijk;
-          const TR CC5 = -p_cot1 * fn12 * ((cw * cw) - TR(1)) * sijk * tjkl;
-          const TR CC6 = TR(2) * p_cot1 * fn12 * cw * sijk * sjkl;
-          // this end's half: j itself, its outer partner i, its outer bond ij, its CdDelta
-          cdself += (double)CT3;
-          cdbo_ij += CT4 + CC1;
-          const TR a7 = CT7 + CC4, a8 = CT8 + CC5, a9 = CT9 + CC6;
-          const TR gix = a7 * dci.x + a9 * doi.x, giy = a7 * dci.y + a9 * doi.y, giz = a7 * dci.z + a9 * doi.z;
-          const double gjx = (double)(a7 * dcj.x + a8 * ecj.x + a9 * doj.x), gjy = (double)(a7 * dcj.y + a8 * ecj.y + a9 * doj.y),
-                       gjz = (double)(a7 * dcj.z + a8 * ecj.z + a9 * doj.z);
-          fix += gix; fiy += giy; fiz += giz;
-          fjx += gjx; fjy += gjy; fjz += gjz;
-          if (PA) {   // g_k with the reference's dcos(omega)/dx_k; positions relative to l: x_l - x_i = -dli, x_l - x_j = djk + dkl
-            const TR htrc = rkl + c2 * (rij * c1 - rjk), hnrc = rij * s1 * s2, gcl = (htrc - arg * hnrc) / rkl;
-            const V3<TR> dok{sc * (-gcl * dkl.x + htrb / rjk * djk.x + gd * dck.x + ge * eck.x),
-                             sc * (-gcl * dkl.y + htrb / rjk * djk.y + gd * dck.y + ge * eck.y),
-                             sc * (-gcl * dkl.z + htrb / rjk * djk.z + gd * dck.z + ge * eck.z)};
-            const double gkx = (double)(a7 * dck.x + a8 * eck.x + a9 * dok.x), gky = (double)(a7 * dck.y + a8 * eck.y + a9 * dok.y),
-                         gkz = (double)(a7 * dck.z + a8 * eck.z + a9 * dok.z);
-            double v[6] = {0, 0, 0, 0, 0, 0};
-            vir_add(v, -1.0, (double)dli.x, (double)dli.y, (double)dli.z, (double)gix, (double)giy, (double)giz);
-            vir_add(v, 1.0, (double)(djk.x + dkl.x), (double)(djk.y + dkl.y), (double)(djk.z + dkl.z), gjx, gjy, gjz);
-            vir_add(v, 1.0, (double)dkl.x, (double)dkl.y, (double)dkl.z, gkx, gky, gkz);
-            for (int c = 0; c < 6; ++c) { vJ[c] += v[c]; vI[c] += v[c]; }
-          }
-          if (counted) {   // energy and the central bond once per torsion
-            e_tor += (double)(fn10 * sijk * sjkl * CV);
-            e_con += (double)(p_cot1 * fn12 * gg);
-            cdbopi_jk += (double)CT2;
-            cdbo_jk += (double)(CT5 + CC2);
-          }
+  TR cdbo_ij = 0, fix = 0, fiy = 0, fiz = 0;   // this lane's terms of the partner in the row's slot: at most one per bond of k
+  double vI[6] = {0, 0, 0, 0, 0, 0};
+  ItemRows Q;
+  // rows (slot pi of i, r-th bond of k that passes) until the next one does not fit, then the queue, and on from that row
+  int pi = 0;
+  bool any = false;              // slot pi has items
+  unsigned long long pass = 0;   // slots of l still to come for pi
+  auto gates = [&]() {
+    pass = 0;
+    if (!cen || pi == pk || pi >= nbj || !(L.bo[base + pi] > thb_cut_s)) return;
+    // the four-body gate's product, left to right as the reference
+    const TS BOijk_s = L.bo[base + pi] * BOjk_s;
+    int c = 0;
+    for (unsigned long long m = far; m; m &= m - 1, ++c) {
+      const int pl = __ffsll(m) - 1;
+      TS BOkl_s = rounded(L.far[min(c, kFarBonds - 1)][lane]);   // loaded here: else the compiler merges the two loads into a flat one
+      if (c >= kFarBonds) BOkl_s = (TS)st.bo[sl(pl, k, n)];
+      if (BOijk_s * BOkl_s > thb_cut_s) pass |= 1ull << pl;
+    }
+  };
+  if (nbw > 0) gates();
+  for (;;) {
+    while (pi < nbw) {
+      const unsigned long long mk = __ballot(pass != 0);
+      if (mk) {
+        if (!Q.fits(mk)) break;
+        const int e = Q.add(mk, pi);
+        if (pass) { L.who[e] = lane | (base + pi) << 6 | (__ffsll(pass) - 1) << 12; pass &= pass - 1; }
+        any = true;
+      } else {
+        if (any) {
+          if (!Q.fits(0)) break;
+          Q.add(0, pi | kRowClose);
+        }
+        ++pi;
+        any = false;
+        if (pi < nbw) gates();
+      }
+    }
+    if (!Q.rows) break;
+    __builtin_amdgcn_wave_barrier();
+    if (lane < Q.items) torsion_item<TR, TS, PA>(st, g, t, L, lane);
+    __builtin_amdgcn_wave_barrier();
+    for (int r = 0; r < Q.rows; ++r) {
+      const int tag = Q.tag_of(r), slot = tag & 0xFFFF;
+      const unsigned long long mask = Q.mask_of(r);
+      const int e = Q.start_of(r) + lanes_below(mask);
+      if ((mask >> lane & 1) && L.who[e] >= 0) {
+        auto R = [&](int c) { return L.res[c][e]; };
+        if (kCen) n_tor += counted ? 1 : 0;
+        // this end's half: j itself, its outer partner i, its outer bond ij, its CdDelta
+        cdself += (double)rounded(R(R_CT2) * dfn11);
+        cdbo_ij += R(R_CDBO);
+        fix += R(R_FI); fiy += R(R_FI + 1); fiz += R(R_FI + 2);
+        fjx += (double)R(R_FJ); fjy += (double)R(R_FJ + 1); fjz += (double)R(R_FJ + 2);
+        if (PA)
+          for (int c = 0; c < 6; ++c) { vJ[c] += L.vir[c][e]; vI[c] += L.vir[c][e]; }
+        if (counted) {   // energy and the central bond once per torsion
+          e_tor += (double)(R(R_TOR) * R(R_TOR + 1));
+          e_con += (double)(R(R_CON) * R(R_CON + 1));
+          cdbopi_jk += (double)R(R_CT2);
+          cdbo_jk += (double)R(R_JK);
         }
       }
-    }
-    fIx += (double)fix; fIy += (double)fiy; fIz += (double)fiz;
-    const double gc = gsum<G>((double)cdbo_ij), gx = gsum<G>((double)fix), gy = gsum<G>((double)fiy), gz = gsum<G>((double)fiz);
-    if (pk == pi) {   // the lane owning slot i: its BO coefficient now, its force for the virial and the end
-      if (live && tj >= 0) st.Cdbo[sl(pk, j, n)] += gc;
-      own_fx += gx; own_fy += gy; own_fz += gz;
-    }
-    if (PA)
-      for (int c = 0; c < 6; ++c) {
-        const double vs = gsum<G>(vI[c]);
-        if (pk == pi) vIown[c] += vs;
+      if (tag & kRowClose) {
+        fIx += (double)fix; fIy += (double)fiy; fIz += (double)fiz;
+        const double gc = gsum<G>((double)cdbo_ij), gx = gsum<G>((double)fix), gy = gsum<G>((double)fiy), gz = gsum<G>((double)fiz);
+        if (pk == slot) { own_c = gc; own_fx += gx; own_fy += gy; own_fz += gz; }   // the lane owning slot i
+        cdbo_ij = fix = fiy = fiz = 0;
+        if (PA)
+          for (int c = 0; c < 6; ++c) {
+            const double vs = gsum<G>(vI[c]);
+            if (pk == slot) vIown[c] += vs;
+            vI[c] = 0;
+          }
       }
+    }
+    Q.clear();
+    __builtin_amdgcn_wave_barrier();
   }
   // This end's half of the torsion virial about the midpoint m of each central bond: with x_i - m = d_ji - d_jk / 2 and
   // x_j - m = -d_jk / 2, - sum (x_i - m) (x) g_i - sum (x_j - m) (x) g_j = - sum_p d_jp (x) F_p + sum_lanes (d_jk / 2) (x) (F_I + F_j),
@@ -1194,7 +1288,7 @@ __device__ __forceinline__ void torsion_body(State st, Globals g, Tables t) {
   for (int c = 0; c < 6; ++c) w[c] = gsum<G>(w[c]);
   if (live && tj >= 0 && pk < nbj) {
     const size_t q = sl(pk, j, n);
-    st.Cdbo[q] += cdbo_jk;
+    st.Cdbo[q] = (st.Cdbo[q] + own_c) + cdbo_jk;
     st.Cdbopi[q] += cdbopi_jk;
     st.fpx[q] += own_fx; st.fpy[q] += own_fy; st.fpz[q] += own_fz;
   }
@@ -1224,12 +1318,14 @@ __device__ __forceinline__ void torsion_body(State st, Globals g, Tables t) {
 // bound spills two 8-byte values, reloaded once per outer partner i, outside the loop over l). kCen: the variant that also
 // records the torsion census (launched only for a force call that asks for it, so the counter costs the ordinary step nothing)
 template <class TS, int G, bool kCen, bool PA>
-__global__ void __attribute__((amdgpu_waves_per_eu(3))) __launch_bounds__(256) k_torsion_f(State st, Globals g, Tables t) {
-  torsion_body<float, TS, G, kCen, PA>(st, g, t);
+__global__ void __launch_bounds__(64 * kAngleWaves) k_torsion_f(State st, Globals g, Tables t) {
+  __shared__ TorsionLds<float, TS, PA> L[kAngleWaves];
+  torsion_body<float, TS, G, kCen, PA>(st, g, t, L[threadIdx.x >> 6]);
 }
 template <int G, bool kCen, bool PA>
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(256) k_torsion_d(State st, Globals g, Tables t) {
-  torsion_body<double, double, G, kCen, PA>(st, g, t);
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_torsion_d(State st, Globals g, Tables t) {
+  __shared__ TorsionLds<double, double, PA> L[kAngleWaves];
+  torsion_body<double, double, G, kCen, PA>(st, g, t, L[threadIdx.x >> 6]);
 }
 
 // ================================================================================================================

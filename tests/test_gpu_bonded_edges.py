@@ -54,3 +54,44 @@ def test_dense_carbon(cells, drop):
             assert np.abs(d).max() <= 4e-3 and np.sqrt((d ** 2).mean()) <= 9e-4, n
         for k, name in enumerate(("bonds", "angle_sets", "torsions")):
             assert np.array_equal(cen[k], np.asarray(ref["census"][name])), (n, prec, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("a,cells,drop", [(3.2, (2, 3, 3), 0), (3.0, (2, 2, 3), 5)])
+def test_many_bonds(a, cells, drop):
+    """Bond orders without the overcoordination corrections (ovc and 13corr 0) in compressed diamond: 14 to 23 bonds per atom above
+    the three-body cutoff, so that an angle row and a torsion row fill the queue several times per slot, and the far bonds of a
+    central bond exceed those kept in LDS. Bars as above, the energy bar also scaled: 1e-4 kcal/mol per atom for terms that sum to
+    100 kcal/mol per atom."""
+    with open(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "ffield.C2013")) as fh:
+        t = fh.read().split("\n")
+    b = next(k for k, line in enumerate(t) if "Nr of bonds" in line) + 2
+    for line, field in ((b, 7), (b + 1, 6)):
+        f = t[line].split()
+        f[field] = "0.0"
+        t[line] = " ".join(f)
+    ff = "\n".join(t)
+    x, L = diamond(cells, drop, seed=9, a=a, sigma=0.05)
+    n = len(x)
+    types, tags, q = np.ones(n, dtype=np.int32), np.arange(1, n + 1), np.zeros(n)
+    ref = Oracle(ff).compute(x, types - 1, tags, [0, 0, 0, L[0], 0, 0, 0, L[1], 0, 0, 0, L[2]], (True, True, True), q=q)
+    scale = max(1.0, np.abs(ref["grad"]).max() / 100.0)
+    e_scale = max(1.0, sum(abs(v) for v in ref["energy"].values()) / n / 100.0)
+    for prec in ("fp64", "mixed"):
+        e = new_engine(ff, ["C"], prec, extra=("checkqeq", "no"))
+        e.set_box(np.zeros(3), L)
+        e.set_atoms(types, tags, x)
+        e.set_charges(q)
+        r = e.compute(rebuild=True, census=True)
+        cen = e.census()
+        e.close()
+        d = (r["grad"] - np.asarray(ref["grad"])) / scale
+        if prec == "fp64":
+            for k in TERMS:
+                assert abs(r["energy"][k] - ref["energy"][k]) <= 1e-9 * max(1.0, abs(ref["energy"][k])), (n, k)
+            assert np.abs(d).max() <= 1e-7, n
+        else:
+            assert abs(sum(r["energy"].values()) - sum(ref["energy"].values())) / n <= 1e-4 * e_scale, n
+            assert np.abs(d).max() <= 4e-3 and np.sqrt((d ** 2).mean()) <= 9e-4, n
+        for k, name in enumerate(("bonds", "angle_sets", "torsions")):
+            assert np.array_equal(cen[k], np.asarray(ref["census"][name])), (n, prec, name)
