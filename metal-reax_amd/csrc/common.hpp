@@ -404,6 +404,16 @@ __device__ inline double read_lane(double v, int lane) {   // lane uniform over 
   b.i[0] = __builtin_amdgcn_readlane(b.i[0], lane); b.i[1] = __builtin_amdgcn_readlane(b.i[1], lane);
   return b.d;
 }
+__device__ inline float read_lane(float v, int lane) {
+  Bits32 b;
+  b.f = v;
+  b.i = __builtin_amdgcn_readlane(b.i, lane);
+  return b.f;
+}
+__device__ inline long long read_lane(long long v, int lane) {
+  const unsigned lo = __builtin_amdgcn_readlane((int)v, lane), hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return (long long)((unsigned long long)hi << 32 | lo);
+}
 // wave sums of K values in place (every lane gets all of them), four at a time
 template <int K>
 __device__ inline void wave_sums(double (&v)[K]) {

@@ -1314,8 +1314,7 @@ __device__ inline void torsion_body(const State& st, const Globals& g, const Tab
   }
 }
 
-// FP32 terms at 3 waves per SIMD (at most 168 VGPRs, no spill); FP64 at 2 (the compiler's choice, 258 VGPRs, leaves one; the
-// bound spills two 8-byte values, reloaded once per outer partner i, outside the loop over l). kCen: the variant that also
+// FP32 terms: 156 VGPRs and 45 KB of LDS per block, 3 waves per SIMD; FP64 held to 2 (216 VGPRs, 67 KB). kCen: the variant that also
 // records the torsion census (launched only for a force call that asks for it, so the counter costs the ordinary step nothing)
 template <class TS, int G, bool kCen, bool PA>
 __global__ void __launch_bounds__(64 * kAngleWaves) k_torsion_f(State st, Globals g, Tables t) {
@@ -1367,6 +1366,11 @@ __device__ inline void hbond_term(const DevHBond& P, TR eh2, const V3<TR>& dji, 
 // of its candidate: energy and the force on j stay in the lane, the BO derivative coefficient and the force on i are reduced over
 // the wave into the bond slot, and the force on the acceptor k is written to the candidate's slot of hf for the acceptor to
 // collect. Non-donors only clear their H-bond energy.
+// Bound by the latency of a wave's chain of loads (23 % of the vector issue slots used at 24,000 atoms; 126 VGPRs, 4 waves per SIMD, and
+// held to 102 it spills: 170 -> 194 us for the three term kernels). So the entries run two chunks ahead and the positions one, the bonds
+// are read once, a slot per lane, and handed round by lane reads, and a slot's sums are read before its triples are evaluated.
+// Terms of a step (valence, torsion, H-bonds) without and with that: 24,000 atoms 187 -> 169 us, 192,000 1237 -> 1109 us, FP64 24,000
+// 250 -> 228 us.
 // PA (per-atom calls): also the reference's per-atom virial split (bonded.cpp:703-710): each triple's (x_j - x_i) (x) g_i +
 // (x_j - x_k) (x) g_k, a third to the donor, to i (through the bond slot) and to the acceptor (through the candidate slot).
 constexpr int kHbWaves = 4;
@@ -1377,9 +1381,11 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
   __shared__ int rk_[kHbWaves][kHbRing], rh_[kHbWaves][kHbRing], rt_[kHbWaves][kHbRing];
   __shared__ double rx_[kHbWaves][kHbRing], ry_[kHbWaves][kHbRing], rz_[kHbWaves][kHbRing], rr_[kHbWaves][kHbRing];
   const int wv = threadIdx.x >> 6;
-  const int j = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int j = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   if (j >= st.n) return;
   const int lane = lane_id(), n = st.n, tj = st.type[j];
+  const int nc = min(st.hc_cnt[j], st.maxhc), nb = min(st.b_cnt[j], st.maxb);
+  const double4 pj = st.pos[j];
   const int role = (tj >= 0 && g.hbond_cut > 0) ? t.sp[tj].p_hbond : 0;
   if (role != 1) {
     if (lane == 0) {
@@ -1391,26 +1397,35 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
   }
   int* rk = rk_[wv]; int* rh = rh_[wv]; int* rt = rt_[wv];
   double *rx = rx_[wv], *ry = ry_[wv], *rz = rz_[wv], *rr = rr_[wv];
-  const int nc = min(st.hc_cnt[j], st.maxhc);
   const size_t hbase = (size_t)j * st.maxhc;
-  const double4 pj = st.pos[j];
+  const int* __restrict__ lj = st.hc_j + hbase;
+  const int* __restrict__ ls = st.hc_s + hbase;
+  // candidates: this chunk's positions and the next chunk's entries in flight
+  int kB = j, eB = 0, kC = j, eC = 0;
+  if (lane < nc) { kC = lj[lane]; eC = ls[lane]; }
+  if (64 + lane < nc) { kB = lj[64 + lane]; eB = ls[64 + lane]; }
+  // slot `lane` of j's bonds (nb <= 64)
+  int bi = 0, bt = 0;
+  long long btag = 0;
+  TR bx = 0, by = 0, bz = 0, bd = 1, bbo = 0;
+  bool bok = false;
+  if (lane < nb) {
+    const size_t q = sl(lane, j, n);
+    bi = st.b_j[q]; bx = (TR)st.b_dx[q]; by = (TR)st.b_dy[q]; bz = (TR)st.b_dz[q]; bd = (TR)st.b_d[q];
+    const double o = st.bo[q];
+    bbo = (TR)o;
+    bok = (TS)o >= TS(1e-2);
+    bt = st.type[bi]; btag = st.tag[bi];
+  }
+  double4 pC = st.pos[kC];
   const double hcut = g.hbond_cut;
-  const int nb = min(st.b_cnt[j], st.maxb);
   TR* hf = reinterpret_cast<TR*>(st.hf);
   double e_hb = 0, fjx = 0, fjy = 0, fjz = 0;
   double w[6] = {0, 0, 0, 0, 0, 0};   // virial of the triples about the donor
   int head = 0, fill = 0, inrange = 0;
   int n_hb = 0;   // census: triples evaluated (bond BO >= 0.01 to an acceptor type, parameters set, i and k not one atom)
-  // the bonds (j, i) that can carry an H-bond (acceptor-type partner, BO >= 0.01), tested by the lanes at once (nb <= 64)
-  unsigned long long hbonds;
-  {
-    bool ok = false;
-    if (lane < nb) {
-      const size_t q = sl(lane, j, n);
-      ok = t.sp[st.type[st.b_j[q]]].p_hbond == 2 && (TS)st.bo[q] >= TS(1e-2);
-    }
-    hbonds = __ballot(ok);
-  }
+  // the bonds (j, i) that can carry an H-bond (acceptor-type partner, BO >= 0.01), tested by the lanes at once
+  const unsigned long long hbonds = __ballot(bok && t.sp[bt].p_hbond == 2);
   // the triples of the m ring entries from head on
   auto batch = [&](int m) {
     const bool has = lane < m;
@@ -1429,16 +1444,18 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
       double vt[6] = {0, 0, 0, 0, 0, 0};
       const int p = __ffsll((long long)left) - 1;
       const size_t q = sl(p, j, n);
-      const int i = st.b_j[q], ti = st.type[i];
-      const V3<TR> dji{(TR)st.b_dx[q], (TR)st.b_dy[q], (TR)st.b_dz[q]};
-      const TR rij = (TR)st.b_d[q];
+      double* const to = lane < 32 ? (lane < 16 ? st.Cdbo : st.fpx) : (lane < 48 ? st.fpy : st.fpz);
+      const double old = lane % 16 == 0 ? to[q] : 0.0;   // the sums' target: read before the triples
+      const int ti = __builtin_amdgcn_readlane(bt, p);
+      const V3<TR> dji{read_lane(bx, p), read_lane(by, p), read_lane(bz, p)};
+      const TR rij = read_lane(bd, p), BOij = read_lane(bbo, p);
       double c1 = 0, fx = 0, fy = 0, fz = 0, et = 0;
       // the same atom as i, possibly another image, is not an acceptor of this triple (reference quirk Q-32)
-      if (has && tagk != st.tag[i]) {
+      if (has && tagk != read_lane(btag, p)) {
         const DevHBond P = t.hb[(ti * g.ntypes + tj) * g.ntypes + tk];
         if (P.r0 > 0.0) {
           ++n_hb;
-          const TR e2 = rexp<TR>(-(TR)P.p2 * (TR)st.bo[q]);
+          const TR e2 = rexp<TR>(-(TR)P.p2 * BOij);
           TR e, CH1, CH2, c3;
           V3<TR> dti, dtj, dtk;
           hbond_term<TR>(P, e2, dji, rij, djk, rjk, e, CH1, CH2, c3, dti, dtj, dtk);
@@ -1462,8 +1479,7 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
       }
       {   // row r of 16 lanes holds the r-th sum: its first lane adds it to the bond's slot
         const double s = wave_sum4_rows(c1, fx, fy, fz);
-        double* const to = lane < 32 ? (lane < 16 ? st.Cdbo : st.fpx) : (lane < 48 ? st.fpy : st.fpz);
-        if (lane % 16 == 0) to[q] += s;
+        if (lane % 16 == 0) to[q] = old + s;
       }
       if (PA) {
         const size_t nsl = (size_t)st.maxb * n;
@@ -1488,13 +1504,18 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
     }
   };
   for (int h0 = 0; h0 < nc; h0 += 64) {
-    const int h = h0 + lane;
-    int k = 0, tk = -1;
+    const int h = h0 + lane, k = kC, en = eC;
+    const double4 pk = pC;
+    kC = kB; eC = eB;
+    if (h0 + 64 < nc) pC = st.pos[kC];
+    kB = j; eB = 0;
+    if (h + 128 < nc) { kB = lj[h + 128]; eB = ls[h + 128]; }
+    int tk = -1;
     bool ok = false;
     double dx = 0, dy = 0, dz = 0, r = 0;
     if (h < nc) {
-      k = st.hc_j[hbase + h];
-      r = sqrt(pair_dvec_list(st, pj, k, st.hc_s[hbase + h], dx, dy, dz, tk));
+      tk = pos_type(pk.w);
+      r = sqrt(pair_dvec_pos(st, pj, pk, en, dx, dy, dz));
       ok = r <= hcut;
       if (!ok) {   // beyond hbond_cut this step: no force on the acceptor from this slot
         const size_t o = 3 * (hbase + h);
