@@ -258,19 +258,28 @@ __device__ inline int entry_shift_index(const State& st, int e) {
 
 #pragma clang fp contract(off)
 // pair_dvec for a list entry e = code | flag of neighbour j (position pj) of the atom at pi, without tags or branches: the same
-// operands in the same order as pair_dvec (the table holds shift_vec of every code), so the result is bitwise identical
+// operands in the same order as pair_dvec (the table holds shift_vec of every code), so the result is bitwise identical: the
+// shift goes to x_j seen from the canonical end, to x_i from the other, and a difference changes its sign exactly.
 // (pi and pj by value: selecting between a reference into global memory and one to a local would put the local on the stack)
 __device__ inline double pair_dvec_shift(const double4 pi, const double4 pj, bool canon, const double4 S, double& dx, double& dy,
                                          double& dz) {
-  const double ax = canon ? pj.x : pi.x, ay = canon ? pj.y : pi.y, az = canon ? pj.z : pi.z;
-  const double bx = canon ? pi.x : pj.x, by = canon ? pi.y : pj.y, bz = canon ? pi.z : pj.z;
-  const double ex = (ax + S.x) - bx, ey = (ay + S.y) - by, ez = (az + S.z) - bz;
-  dx = canon ? ex : -ex;
-  dy = canon ? ey : -ey;
-  dz = canon ? ez : -ez;
+  const double jx = canon ? S.x : 0.0, jy = canon ? S.y : 0.0, jz = canon ? S.z : 0.0;
+  const double ix = canon ? 0.0 : S.x, iy = canon ? 0.0 : S.y, iz = canon ? 0.0 : S.z;
+  dx = (pj.x + jx) - (pi.x + ix);
+  dy = (pj.y + jy) - (pi.y + iy);
+  dz = (pj.z + jz) - (pi.z + iz);
+  return dx * dx + dy * dy + dz * dz;
+}
+// the same where no lane has a shift (most chunks of 64 entries: the entries of an atom come cell by cell): the shift vector of
+// code 0 is zero
+__device__ inline double pair_dvec_plain(const double4 pi, const double4 pj, double& dx, double& dy, double& dz) {
+  dx = pj.x - pi.x;
+  dy = pj.y - pi.y;
+  dz = pj.z - pi.z;
   return dx * dx + dy * dy + dz * dz;
 }
 __device__ inline double pair_dvec_pos(const State& st, const double4 pi, const double4 pj, int e, double& dx, double& dy, double& dz) {
+  if (!__any(entry_code(e) != 0)) return pair_dvec_plain(pi, pj, dx, dy, dz);
   return pair_dvec_shift(pi, pj, (e & kCanon) != 0, st.shv[pos_sys(pi.w) * st.shv_stride + entry_shift_index(st, e)], dx, dy, dz);
 }
 __device__ inline double pair_dvec_list(const State& st, const double4& pi, int j, int e, double& dx, double& dy, double& dz) {
@@ -288,6 +297,9 @@ __device__ inline double pair_dvec_list(const State& st, const double4& pi, int 
 // the LDS permutes behind __shfl (two per double and step, each a trip through the LDS pipe: a wave's eleven non-bonded sums
 // were 132 of them). Every sum adds the same pairs in the same order as the xor butterfly (offsets 32, 16, 8, 4, 2, 1).
 __device__ inline int lane_id() { return threadIdx.x & 63; }
+// the wave's number in the grid (of a wave per atom: the atom), known to the compiler as one value per wave: the atom's own data, base
+// addresses and loop bounds live in scalar registers
+__device__ inline int wave_atom() { return (int)(blockIdx.x * (blockDim.x >> 6)) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;                    // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int kDppShl4 = 0x104, kDppShr4 = 0x114;                  // row_shl:4 (lane i reads i + 4), row_shr:4 (reads i - 4)

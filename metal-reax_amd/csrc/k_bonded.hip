@@ -1400,7 +1400,7 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
   __shared__ int rk_[kHbWaves][kHbRing], rh_[kHbWaves][kHbRing], rt_[kHbWaves][kHbRing];
   __shared__ double rx_[kHbWaves][kHbRing], ry_[kHbWaves][kHbRing], rz_[kHbWaves][kHbRing], rr_[kHbWaves][kHbRing];
   const int wv = threadIdx.x >> 6;
-  const int j = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  const int j = wave_atom();
   if (j >= st.n) return;
   const int lane = lane_id(), n = st.n, tj = st.type[j];
   const int nc = min(st.hc_cnt[j], st.maxhc), nb = min(st.b_cnt[j], st.maxb);
@@ -1587,7 +1587,7 @@ __global__ void __launch_bounds__(64 * kHbWaves) k_hbond_donor(State st, Globals
 // lists those slots in ascending order; fixed between neighbour rebuilds).
 template <class TR>
 __global__ void __launch_bounds__(256) k_hbond_acceptor(State st, Globals g, Tables t) {
-  const int k = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int k = wave_atom();
   if (k >= st.n) return;
   const int lane = lane_id(), tk = st.type[k];
   const int role = (tk >= 0 && g.hbond_cut > 0) ? t.sp[tk].p_hbond : 0;

@@ -100,7 +100,7 @@ constexpr double kGapSlack = 1e-6;   // subtracted from every gap (Angstrom): fa
 // (sidx: atoms in the order of their cells; null when the atoms themselves are in that order)
 __global__ void __launch_bounds__(256) k_nbr_cells(State st, Globals g, Tables t, Cell c, int nc0, int nc1, int nc2, const int* sidx,
                                                    const int* cstart, const int* cend, const unsigned* atom_key, double rs2, SubCut cut) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   const int lane = lane_id();
   const double4 pi = st.pos[i];
@@ -167,7 +167,7 @@ constexpr int kBruteWaves = 4;
 __global__ void __launch_bounds__(64 * kBruteWaves) k_nbr_brute(State st, Globals g, Tables t, Cell c, int sm0, int sm1, int sm2, double rs2,
                                                                 SubCut cut) {
   __shared__ int codes_[kBruteWaves][64];
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   const int lane = lane_id(), n = st.n;
   int* codes = codes_[threadIdx.x >> 6];
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(64 * kBruteWaves) k_nbr_brute(State st, Global
 // fill them along with the skin list; this pass lists them from it with packed systems, and again when a sub-list's capacity has
 // grown. Entries two chunks ahead and positions one chunk ahead are loaded while a chunk is tested (the walk is latency-bound).
 __global__ void __launch_bounds__(256) k_sublists(State st, Globals g, Tables t, SubCut cut) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   const int lane = lane_id();
   ListRow row = list_row(st, g, t, i);
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(256) k_sublists(State st, Globals g, Tables t,
 // acceptor's row in arrival order (an integer atomic claims the position), then each row is put in ascending slot order by
 // rank counting (the slot indices are distinct), so the acceptor's later force gather runs in a fixed order.
 __global__ void __launch_bounds__(256) k_hc_transpose(State st, Globals g, Tables t) {
-  const int j = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int j = wave_atom();
   if (j >= st.n) return;
   const int tj = st.type[j];
   if (tj < 0 || t.sp[tj].p_hbond != 1) return;
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(256) k_hc_transpose(State st, Globals g, Table
 template <bool kLds>
 __global__ void __launch_bounds__(256) k_hc_sort(State st, Globals g, Tables t) {
   extern __shared__ int hc_keys[];
-  const int k = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int k = wave_atom();
   if (k >= st.n) return;
   const int tk = st.type[k];
   if (tk < 0 || t.sp[tk].p_hbond != 2) return;

@@ -34,9 +34,10 @@ __device__ inline void nb_acc(NbAcc& a, double ce, double evdw, double eel, doub
 // Horner taper in r and its exponents (0.33333333333333 for the shielded Coulomb's cube root as written), pow(x, y) evaluated
 // as exp(y log x) (a few ulp), the type pair's (1 / gamma_w)^p_vdW1 and the reciprocals of r_vdW and rcore from the table,
 // e1 = e2^2 for the two Morse exponentials, and one division for 1 / r
-__device__ inline void nb_pair_d(const Globals& g, const DevPair* __restrict__ row, double qi, double qj, int tj, double r,
+template <class Row>
+__device__ inline void nb_pair_d(const Globals& g, const Row* __restrict__ row, double qi, double qj, int tj, double r,
                                  double dx, double dy, double dz, NbAcc& a) {
-  const DevPair& P = row[tj];
+  const Row& P = row[tj];
   const double p_vdW1 = g.p_vdW1, p1i = 1.0 / g.p_vdW1;
   const int vt = g.vdw_type;
   const double ir = 1.0 / r;
@@ -144,6 +145,8 @@ template <bool D> struct NbPrec;
 template <> struct NbPrec<false> {
   using Q = float;
   using Row = NbPairF;
+  using Tab = NbPairF;
+  static __device__ Tab tab(const Row& P) { return P; }
   static __device__ const NbPairF* row(const Globals& g, const Tables& t, int ti) { return t.nbf + ti * g.ntypes; }
   static __device__ void pair(const Globals& g, const NbPairF* row, float qi, float qj, int tj, double rd, double dx, double dy,
                               double dz, NbAcc& a) {
@@ -154,11 +157,16 @@ template <> struct NbPrec<false> {
     return (double)(23.02f * ((float)sp.chi * q + ((float)sp.eta / 2.0f) * (q * q)));
   }
 };
+// the non-bonded part of DevPair
+struct NbPairD { double D, alpha, irvdw, pgw, ecore, acore, ircore, gamma, lgcij, re6; };
 template <> struct NbPrec<true> {
   using Q = double;
   using Row = DevPair;
+  using Tab = NbPairD;
+  static __device__ Tab tab(const Row& P) { return {P.D, P.alpha, P.irvdw, P.pgw, P.ecore, P.acore, P.ircore, P.gamma, P.lgcij, P.re6}; }
   static __device__ const DevPair* row(const Globals& g, const Tables& t, int ti) { return t.pair + ti * g.ntypes; }
-  static __device__ void pair(const Globals& g, const DevPair* row, double qi, double qj, int tj, double rd, double dx, double dy,
+  template <class R>
+  static __device__ void pair(const Globals& g, const R* row, double qi, double qj, int tj, double rd, double dx, double dy,
                               double dz, NbAcc& a) {
     nb_pair_d(g, row, qi, qj, tj, rd, dx, dy, dz, a);
   }
@@ -246,7 +254,7 @@ __global__ void __launch_bounds__(64 * kNbWaves) k_nonbonded_f(State st, Globals
   __shared__ int rj_[kNbWaves][kNbRing], rt_[kNbWaves][kNbRing];
   __shared__ double rx_[kNbWaves][kNbRing], ry_[kNbWaves][kNbRing], rz_[kNbWaves][kNbRing], rr_[kNbWaves][kNbRing];
   const int w = threadIdx.x >> 6;
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   nb_list_wave<false>(st, g, t, i, rj_[w], rt_[w], rx_[w], ry_[w], rz_[w], rr_[w]);
 }
@@ -255,44 +263,69 @@ __global__ void __launch_bounds__(64 * kNbWaves) k_nonbonded_d(State st, Globals
   __shared__ int rj_[kNbWaves][kNbRing], rt_[kNbWaves][kNbRing];
   __shared__ double rx_[kNbWaves][kNbRing], ry_[kNbWaves][kNbRing], rz_[kNbWaves][kNbRing], rr_[kNbWaves][kNbRing];
   const int w = threadIdx.x >> 6;
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);   // not wave_atom: it spills here
   if (i >= st.n) return;
   nb_list_wave<true>(st, g, t, i, rj_[w], rt_[w], rx_[w], ry_[w], rz_[w], rr_[w]);
 }
 
-// pair_dvec_list for a charge-matrix entry: the same operands in the same order, the shift vector found through the entry's key
-#pragma clang fp contract(off)
-__device__ inline double pair_dvec_key(const State& st, const double4 pi, const double4 pj, int key, double& dx, double& dy, double& dz) {
-  const bool canon = (key & 0x8000) != 0;
-  const double4 S = st.shv[pos_sys(pi.w) * st.shv_stride + (key & 0x7FFF)];
-  const double ax = canon ? pj.x : pi.x, ay = canon ? pj.y : pi.y, az = canon ? pj.z : pi.z;
-  const double bx = canon ? pi.x : pj.x, by = canon ? pi.y : pj.y, bz = canon ? pi.z : pj.z;
-  const double ex = (ax + S.x) - bx, ey = (ay + S.y) - by, ez = (az + S.z) - bz;
-  dx = canon ? ex : -ex;
-  dy = canon ? ey : -ey;
-  dz = canon ? ez : -ez;
-  return dx * dx + dy * dy + dz * dz;
+// What every pair of a row looks up, in LDS (one wave): the shift vectors and the row type's parameters. Read from memory in the
+// pair loop they cost as much address traffic as the positions, and, loads returning in order, a wait for all that is in flight for the
+// next pairs. The non-bonded pass over the rows took 81 us at 24,000 atoms and 661 us at 192,000; with chunks that have no shift taken
+// without one 76 and 588, with these tables 62 and 466, with the row's own data in scalar registers (wave_atom) 58 and 411. Cells with
+// more shifts (thin ones: 64 take 1.5 KB per wave, and leave the matrix build its 6 blocks per CU) or force fields with more types read
+// them from memory.
+constexpr int kTabShifts = 64, kTabTypes = 16;
+inline bool row_tables_fit(const State& st, const Globals& g) {
+  return (long long)(2 * st.smx0 + 1) * (2 * st.smx1 + 1) * (2 * st.smx2 + 1) <= kTabShifts && g.ntypes <= kTabTypes;
 }
-#pragma clang fp contract(on)
+template <class P>
+struct RowTables {
+  double x[kTabShifts], y[kTabShifts], z[kTabShifts];
+  P par[kTabTypes];
+  __device__ void fill_shifts(const State& st, const double4* __restrict__ shv) {
+    const int ns = 2 * shift_index(st, 0) + 1;
+    for (int k = lane_id(); k < ns; k += 64) {
+      const double4 S = shv[k];
+      x[k] = S.x; y[k] = S.y; z[k] = S.z;
+    }
+  }
+  __device__ double4 shift(int k) const { return make_double4(x[k], y[k], z[k], 0.0); }
+};
+
+// pair_dvec_list for a charge-matrix entry: the same operands in the same order, the shift vector found through the entry's key
+// (zero: the key's index of the zero shift)
+template <class F>
+__device__ inline double pair_dvec_key(F&& shift, const double4 pi, const double4 pj, int key, int zero, double& dx, double& dy, double& dz) {
+  const int k = key & 0x7FFF;
+  if (!__any(k != zero)) return pair_dvec_plain(pi, pj, dx, dy, dz);
+  return pair_dvec_shift(pi, pj, (key & 0x8000) != 0, shift(k), dx, dy, dz);
+}
 
 // The non-bonded terms over the charge-matrix rows: the rows hold, in skin-list order, exactly the pairs within the matrix
 // cutoff, so every lane carries a pair (no distance pre-pass, no compaction) and a row costs its column and key (4 bytes per
 // pair with 16-bit columns) instead of the 8-byte skin entries of all pairs out to the list radius. Lane l takes entries l,
 // l + 64, ..., the assignment of the skin-list kernel's compacted batches, so the sums are the same.
-template <bool D, class TC>
+template <bool D, bool kTab, class TC>
 __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tables& t, const TC* __restrict__ col,
-                                    const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride, int i) {
+                                    const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride, int i,
+                                    RowTables<typename NbPrec<D>::Tab>& L) {
   using Q = typename NbPrec<D>::Q;
   const int lane = lane_id();
   const int ti = st.type[i];
   NbAcc a;
   if (ti >= 0) {
     const size_t base = (size_t)i * stride;   // keys in list order, columns as row_slot puts them
-    const int cnt = rcnt[i];
+    const int cnt = rcnt[i], zero = shift_index(st, 0);
     const Q qi = (Q)st.q[i];
     const double4 pi = st.pos[i];
     const double cut = g.nonb_cut, cut2 = cut * cut * (1.0 + 1e-12);
     const typename NbPrec<D>::Row* __restrict__ row = NbPrec<D>::row(g, t, ti);
+    const double4* __restrict__ shv = st.shv + pos_sys(pi.w) * st.shv_stride;
+    if (kTab) {
+      L.fill_shifts(st, shv);
+      if (lane < g.ntypes) L.par[lane] = NbPrec<D>::tab(row[lane]);
+      __builtin_amdgcn_wave_barrier();
+    }
     // two-deep software pipeline as in the matrix build: columns/keys two strides ahead, positions and charges one ahead
     // (lanes past the row's end carry the row atom itself and key 0, valid indices never used)
     int jB = i, kyB = 0, jC = i, kyC = 0;
@@ -310,10 +343,13 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
       jB = i; kyB = 0;
       if (k + 128 < cnt) { jB = (int)col[base + row_slot(k + 128, cnt)]; kyB = key[base + k + 128]; }
       double dx, dy, dz;
-      const double r2 = pair_dvec_key(st, pi, pj, ky, dx, dy, dz);
+      const double r2 = pair_dvec_key([&](int s) { return kTab ? L.shift(s) : shv[s]; }, pi, pj, ky, zero, dx, dy, dz);
       if (r2 <= cut2) {
         const double rd = sqrt(r2);
-        if (rd <= cut) NbPrec<D>::pair(g, row, qi, qj, pos_type(pj.w), rd, dx, dy, dz, a);
+        if (rd <= cut) {
+          if constexpr (kTab) NbPrec<D>::pair(g, L.par, qi, qj, pos_type(pj.w), rd, dx, dy, dz, a);
+          else NbPrec<D>::pair(g, row, qi, qj, pos_type(pj.w), rd, dx, dy, dz, a);
+        }
       }
     }
   }
@@ -321,34 +357,40 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
 }
 
 // (5 waves per SIMD: 96 VGPRs without spills; the compiler's choice, 106 VGPRs and 4 waves, is slower)
-template <class TC>
+template <class TC, bool kTab>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_nonbonded_rows(State st, Globals g, Tables t, const TC* __restrict__ col,
                                                         const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  __shared__ RowTables<NbPairF> L[kTab ? 4 : 1];
+  const int i = wave_atom();
   if (i >= st.n) return;
-  nb_rows_wave<false, TC>(st, g, t, col, key, rcnt, stride, i);
+  nb_rows_wave<false, kTab, TC>(st, g, t, col, key, rcnt, stride, i, L[kTab ? threadIdx.x >> 6 : 0]);
 }
-
-template <class TC>
+template <class TC, bool kTab>
 __global__ void __launch_bounds__(256) k_nonbonded_rows_d(State st, Globals g, Tables t, const TC* __restrict__ col,
                                                           const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  __shared__ RowTables<NbPairD> L[kTab ? 4 : 1];
+  const int i = wave_atom();
   if (i >= st.n) return;
-  nb_rows_wave<true, TC>(st, g, t, col, key, rcnt, stride, i);
+  nb_rows_wave<true, kTab, TC>(st, g, t, col, key, rcnt, stride, i, L[kTab ? threadIdx.x >> 6 : 0]);
 }
 
-constexpr int kQbWaves = 4, kQbRing = 128;
+constexpr int kQbWaves = 4, kQbRing = 256;
 
-// One wave per row atom over its skin list: a filter pass (distance only, list entries two chunks ahead and positions one chunk
-// ahead in flight) pushes the pairs within the matrix cutoff, in list order, into a per-wave LDS ring; every 64 of them are
-// finished together (taper, shielded 1/r, stores), so the costly part runs on full waves. Row entries are kept in skin-list
+// One wave per row atom over its skin list, 128 entries at a time: a filter pass (distance only) pushes the pairs within the matrix
+// cutoff, in list order, into a per-wave LDS ring; every 64 of them are finished together (taper, shielded 1/r, stores), so the
+// costly part runs on full waves. Bound by the latency of a wave's chain of loads: doing the arithmetic, the position gathers or the
+// stores twice adds 0 to 5 %. So two chunks go through the chain at once, each round's loads go out in the order in which they are
+// waited for (the guess gathers of the batches, the next positions, the entries after those), and the row's own data sit in scalar
+// registers (79 VGPRs, 6 waves per SIMD). 24,000 / 192,000 atoms of water: 138 / 1064 us a chunk at a time with the tables in memory,
+// 137 / 1075 with the tables in LDS, 123 / 945 two chunks at a time, 117 / 915 us with the row's data in scalar registers. Row entries are kept in skin-list
 // order: slot m of the row is the m-th pair of the list within the cutoff. The 16-bit key is the canonical flag and the
 // shift-table index the distance used.
 // fuse: the row also forms the charge solve's start from the guess in x (k_cg_guess ran before): y = H x with the values as
 // built (FP64, or the FP32 values a non-refined FP32 solve iterates with), r = b - (y + eta x), p = r / eta, and the row's
 // b.b and r.p for the block partials; this replaces a separate product pass over the rows.
+template <bool kTab>
 __device__ inline void qeq_build_row(const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, int i, int fuse,
-                                     int* rj, int* rk, double* rr, double (&acc)[4]) {
+                                     int* rj, int* rk, double* rr, RowTables<double>& L, double (&acc)[4]) {
   const int lane = lane_id();
   const int ti = st.type[i];
   const size_t base = (size_t)i * st.maxnb, rbase = (size_t)i * qb.stride;
@@ -358,85 +400,132 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
   const double4 pi = st.pos[i];
   const double4* __restrict__ shv = st.shv + pos_sys(pi.w) * st.shv_stride;
   const double* __restrict__ shld = t.qeq_shld + max(ti, 0) * g.ntypes;
+  const double eta = ti >= 0 ? t.qeq_eta[ti] : 1.0, chi = ti >= 0 ? t.qeq_chi[ti] : 0.0;
+  const double2* __restrict__ x2 = reinterpret_cast<const double2*>(qb.x);
+  const double2 xi = fuse ? x2[i] : make_double2(0.0, 0.0);
+  const int zero = shift_index(st, 0);
+  const int* __restrict__ lj = st.nb_j + base;
+  const int* __restrict__ ls = st.nb_s + base;
+  // entry k of the list (past its end the last one, which no lane uses)
+  const int last = max(cnt - 1, 0);
+  auto entry = [&](int k, int& j, int& e) { const int q = min(k, last); j = cnt ? lj[q] : i; e = cnt ? ls[q] : 0; };
+  int jn[2], en[2], jc[2], ec[2];   // the next two chunks' entries, this pair's
+  double4 pc[2];
+  for (int u = 0; u < 2; ++u) {   // with the count in flight (entries past it are cleared)
+    const int q = min(64 * u + lane, st.maxnb - 1);
+    jc[u] = lj[q]; ec[u] = ls[q];
+  }
+  for (int u = 0; u < 2; ++u)
+    if (64 * u + lane >= cnt) { jc[u] = i; ec[u] = 0; }
+  for (int u = 0; u < 2; ++u) entry(64 * (2 + u) + lane, jn[u], en[u]);
+  if (kTab) {
+    L.fill_shifts(st, shv);
+    if (lane < g.ntypes) L.par[lane] = shld[lane];
+    __builtin_amdgcn_wave_barrier();
+  }
+  for (int u = 0; u < 2; ++u) pc[u] = st.pos[jc[u]];
   int m = 0, head = 0, fill = 0;
   double lo_sum = 0.0;   // this lane's part of sum_j |lo_ij| (refinement)
   double y0 = 0.0, y1 = 0.0;   // fuse: this lane's part of (H x) of both systems
-  const double2* __restrict__ x2 = reinterpret_cast<const double2*>(qb.x);
-  auto batch = [&](int count) {
+  // the lane's entry of a batch taken from the ring: column, key | type, squared distance, then the matrix entry
+  struct Batch { int j, k; double h; double2 x; };
+  auto take = [&](int count, Batch& b) {
+    const int e = (head + lane) & (kQbRing - 1);
+    b.j = i;
+    if (lane < count) { b.j = rj[e]; b.k = rk[e]; b.h = rr[e]; }
+    if (fuse) b.x = x2[b.j];
+    head = (head + count) & (kQbRing - 1);
+    fill -= count;
+  };
+  // h - (float)h is exact in FP64; rounded to FP32 it leaves the two parts within about 2^-48 (relative) of h
+  auto low = [](double h) { return (float)(h - (double)(float)h); };
+  auto evaluate = [&](int count, Batch& b) {
     if (lane < count) {
-      const int e = (head + lane) & (kQbRing - 1);
-      const int j = rj[e], kt = rk[e];
-      const double r = sqrt(rr[e]);
+      const double r = sqrt(b.h);
       double Tap = T[7] * r + T[6];
       Tap = Tap * r + T[5]; Tap = Tap * r + T[4]; Tap = Tap * r + T[3]; Tap = Tap * r + T[2]; Tap = Tap * r + T[1]; Tap = Tap * r + T[0];
-      const double h = (Tap * 14.4) * rcbrt_f64(r * r * r + shld[kt >> 16]);
-      const size_t o = rbase + m + (count == kRowGroup ? group_slot(lane) : lane);   // row_slot: m counts full groups
-      if (qb.narrow) qb.col16[o] = (unsigned short)j; else qb.col[o] = j;
-      double hv = h;   // the value the start's product uses
+      double sh;
+      if constexpr (kTab) sh = L.par[b.k >> 16]; else sh = shld[b.k >> 16];
+      b.h = (Tap * 14.4) * rcbrt_f64(r * r * r + sh);
+      double hv = b.h;   // the value the start's product uses
       if (qb.fp32) {
-        const float hf = (float)h;
-        qb.val32[o] = hf;
-        // h - hf is exact in FP64; rounded to FP32 it leaves hf + lo within about 2^-48 (relative) of h
-        if (qb.refine) {
-          const float lo = (float)(h - (double)hf);
-          qb.lo32[o] = lo;
-          lo_sum += fabs((double)lo);
-        } else {
-          hv = (double)hf;
-        }
-      } else {
-        qb.val[o] = h;
+        if (qb.refine) lo_sum += fabs((double)low(b.h));
+        else hv = (double)(float)b.h;
       }
       if (fuse) {
-        const double2 xj = x2[j];
-        y0 += hv * xj.x;
-        y1 += hv * xj.y;
+        y0 += hv * b.x.x;
+        y1 += hv * b.x.y;
       }
-      if (qb.keyed) qb.key[rbase + m + lane] = (unsigned short)(kt & 0xFFFF);
+    }
+  };
+  auto store = [&](int count, const Batch& b) {
+    if (lane < count) {
+      const size_t o = rbase + m + (count == kRowGroup ? group_slot(lane) : lane);   // row_slot: m counts full groups
+      if (qb.narrow) qb.col16[o] = (unsigned short)b.j; else qb.col[o] = b.j;
+      if (qb.fp32) {
+        qb.val32[o] = (float)b.h;
+        if (qb.refine) qb.lo32[o] = low(b.h);
+      } else {
+        qb.val[o] = b.h;
+      }
+      if (qb.keyed) qb.key[rbase + m + lane] = (unsigned short)(b.k & 0xFFFF);
     }
     m += count;
   };
-  const int* __restrict__ lj = st.nb_j + base;
-  const int* __restrict__ ls = st.nb_s + base;
-  int jB = i, eB = 0, jC = i, eC = 0;
-  if (lane < cnt) { jC = lj[lane]; eC = ls[lane]; }
-  double4 pC = st.pos[jC];
-  if (64 + lane < cnt) { jB = lj[64 + lane]; eB = ls[64 + lane]; }
-  for (int k0 = 0; k0 < cnt; k0 += 64) {
-    const int k = k0 + lane;
-    const int j = jC, e = eC;
-    const double4 pj = pC;
-    jC = jB; eC = eB;
-    if (k0 + 64 < cnt) pC = st.pos[jC];
-    jB = i; eB = 0;
-    if (k + 128 < cnt) { jB = lj[k + 128]; eB = ls[k + 128]; }
-    bool keep = false;
-    double r2 = 0;
-    int kt = 0;
-    if (k < cnt) {
-      const bool canon = (e & kCanon) != 0;
-      const int sidx = entry_shift_index(st, e);
-      double dx, dy, dz;
-      r2 = pair_dvec_shift(pi, pj, canon, shv[sidx], dx, dy, dz);
-      const int tj = pos_type(pj.w);
-      keep = tj >= 0 && r2 <= swb2;
-      kt = (qb.keyed ? (canon ? 0x8000 : 0) | sidx : 0) | (tj << 16);   // a keyed table has at most 32768 entries
+  for (int k0 = 0; k0 < cnt; k0 += 128) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k = k0 + 64 * u + lane, j = jc[u], e = ec[u];
+      const double4 pj = pc[u];
+      bool keep = false;
+      double r2 = 0;
+      int kt = 0;
+      if (k < cnt) {
+        const bool canon = (e & kCanon) != 0;
+        int sidx = zero;
+        double dx, dy, dz;
+        if (!__any(entry_code(e) != 0)) {
+          r2 = pair_dvec_plain(pi, pj, dx, dy, dz);
+        } else {
+          sidx = entry_shift_index(st, e);
+          r2 = pair_dvec_shift(pi, pj, canon, kTab ? L.shift(sidx) : shv[sidx], dx, dy, dz);
+        }
+        const int tj = pos_type(pj.w);
+        keep = tj >= 0 && r2 <= swb2;
+        kt = (qb.keyed ? (canon ? 0x8000 : 0) | sidx : 0) | (tj << 16);   // a keyed table has at most 32768 entries
+      }
+      const unsigned long long msk = __ballot(keep);
+      if (keep) {
+        const int e2 = (head + fill + lanes_below(msk)) & (kQbRing - 1);
+        rj[e2] = j; rk[e2] = kt; rr[e2] = r2;
+      }
+      fill += __popcll(msk);
     }
-    const unsigned long long msk = __ballot(keep);
-    if (keep) {
-      const int e2 = (head + fill + lanes_below(msk)) & (kQbRing - 1);
-      rj[e2] = j; rk[e2] = kt; rr[e2] = r2;
-    }
-    fill += __popcll(msk);
     __builtin_amdgcn_wave_barrier();
-    if (fill >= 64) {
-      batch(64);
-      head = (head + 64) & (kQbRing - 1);
-      fill -= 64;
-      __builtin_amdgcn_wave_barrier();
-    }
+    // the full batches leave the ring; their guess values, then the next chunks' positions, then the entries after those go out
+    Batch b0, b1;
+    const int nfull = fill >> 6;
+    if (nfull > 0) take(64, b0);
+    if (nfull > 1) take(64, b1);
+    __builtin_amdgcn_wave_barrier();
+    for (int u = 0; u < 2; ++u) { jc[u] = jn[u]; ec[u] = en[u]; pc[u] = st.pos[jc[u]]; }
+    for (int u = 0; u < 2; ++u) entry(k0 + 64 * (4 + u) + lane, jn[u], en[u]);
+    if (nfull > 0) evaluate(64, b0);
+    if (nfull > 1) evaluate(64, b1);
+    // what was loaded has come back here, before the stores go out: loads and stores are waited for in order, so a wait at the
+    // top of the loop would be one for the stores
+    for (int u = 0; u < 2; ++u)
+      asm volatile("" : "+v"(pc[u].x), "+v"(pc[u].y), "+v"(pc[u].z), "+v"(pc[u].w), "+v"(jn[u]), "+v"(en[u]));
+    if (nfull > 0) store(64, b0);
+    if (nfull > 1) store(64, b1);
   }
-  if (fill > 0) batch(fill);
+  if (fill > 0) {
+    Batch b;
+    const int count = fill;
+    take(count, b);
+    evaluate(count, b);
+    store(count, b);
+  }
   {
     double s[3] = {lo_sum, y0, y1};
     wave_sums<3>(s);
@@ -445,14 +534,11 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
   if (lane == 0) {
     qb.cnt[i] = m;
     if (qb.refine) qb.lorow[i] = lo_sum;
-    const double eta = ti >= 0 ? t.qeq_eta[ti] : 1.0;
     const double hinv = 1.0 / eta;
-    const double chi = ti >= 0 ? t.qeq_chi[ti] : 0.0;
     qb.eta[i] = eta;
     qb.hinv[i] = hinv;
     qb.chi[i] = chi;
     if (fuse) {   // the start of k_spmv2's kMode 1 for this row (b from this build's chi: the guess kernel ran before it)
-      const double2 xi = x2[i];
       const double wv[2] = {y0 + eta * xi.x, y1 + eta * xi.y};
       for (int s = 0; s < 2; ++s) {
         const double b = s == 0 ? -chi : -1.0;
@@ -468,15 +554,17 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
   }
 }
 
+template <bool kTab>
 __global__ void __launch_bounds__(256) k_qeq_build(State st, Globals g, Tables t, QeqBuffers qb, int fuse) {
+  __shared__ RowTables<double> L[kTab ? kQbWaves : 1];
   __shared__ int ring_j[kQbWaves][kQbRing];
   __shared__ int ring_k[kQbWaves][kQbRing];   // key | neighbour type << 16
   __shared__ double ring_r2[kQbWaves][kQbRing];
   __shared__ double sh[4 * kQbWaves];
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int wv = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = wave_atom();
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (i < st.n) qeq_build_row(st, g, t, qb, i, fuse, ring_j[wv], ring_k[wv], ring_r2[wv], acc);
+  if (i < st.n) qeq_build_row<kTab>(st, g, t, qb, i, fuse, ring_j[wv], ring_k[wv], ring_r2[wv], L[kTab ? wv : 0], acc);
   if (fuse) {   // the block's partials of b.b and r.p, its rows in wave order (a fixed order)
     if (lane_id() == 0)
       for (int k = 0; k < 4; ++k) sh[k * kQbWaves + wv] = acc[k];
@@ -494,7 +582,7 @@ __global__ void __launch_bounds__(256) k_qeq_build(State st, Globals g, Tables t
 // nonb_cut. The test is the one every non-bonded kernel takes (the FP64 square root of the canonical squared distance <=
 // nonb_cut, in all precisions), on the same list entries, so the count is the number of pairs those kernels evaluate there.
 __global__ void __launch_bounds__(256) k_census_nb(State st, Globals g) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   const int lane = lane_id();
   const int ti = st.type[i];
@@ -531,20 +619,27 @@ void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals
   else hipLaunchKernelGGL(k_nonbonded_f, grid, blk, 0, s, st, g, t);
 }
 
-void launch_nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
+template <bool kTab>
+static void nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
   const dim3 grid(nblk((long long)st.n * 64, 256)), blk(256);
   if (p == Precision::FP64) {
-    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows_d<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
-    else hipLaunchKernelGGL(k_nonbonded_rows_d<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
+    if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows_d<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+    else hipLaunchKernelGGL((k_nonbonded_rows_d<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
   } else {
-    if (qb.narrow) hipLaunchKernelGGL(k_nonbonded_rows<unsigned short>, grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
-    else hipLaunchKernelGGL(k_nonbonded_rows<int>, grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
+    if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+    else hipLaunchKernelGGL((k_nonbonded_rows<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
   }
+}
+void launch_nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
+  if (row_tables_fit(st, g)) nonbonded_rows<true>(p, st, g, t, qb, s);
+  else nonbonded_rows<false>(p, st, g, t, qb, s);
 }
 
 void launch_qeq_build(const State& st, const Cell& c, const Globals& g, const Tables& t, QeqBuffers& qb, int fuse, hipStream_t s) {
   (void)c;
-  hipLaunchKernelGGL(k_qeq_build, dim3(qeq_build_blocks(st.n)), dim3(256), 0, s, st, g, t, qb, fuse);
+  const dim3 grid(qeq_build_blocks(st.n)), blk(256);
+  if (row_tables_fit(st, g)) hipLaunchKernelGGL(k_qeq_build<true>, grid, blk, 0, s, st, g, t, qb, fuse);
+  else hipLaunchKernelGGL(k_qeq_build<false>, grid, blk, 0, s, st, g, t, qb, fuse);
 }
 
 }  // namespace rxa

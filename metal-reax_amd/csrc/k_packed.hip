@@ -58,7 +58,7 @@ __global__ void k_pk_wrap(State st, const Cell* cells, const int* reb) {
 // (the image is taken from the listing atom's side, as in the single-system searches; only kept entries need the tags)
 __global__ void __launch_bounds__(256) k_pk_nbr(State st, const Cell* cells, const int* sys_start, const int4* ext, const int* reb,
                                                double rs2) {
-  const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int i = wave_atom();
   if (i >= st.n) return;
   const int s = st.sysid[i];
   if (!reb[s]) return;
