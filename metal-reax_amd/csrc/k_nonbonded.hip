@@ -329,10 +329,10 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
     // two-deep software pipeline as in the matrix build: columns/keys two strides ahead, positions and charges one ahead
     // (lanes past the row's end carry the row atom itself and key 0, valid indices never used)
     int jB = i, kyB = 0, jC = i, kyC = 0;
-    if (lane < cnt) { jC = (int)col[base + row_slot(lane, cnt)]; kyC = key[base + lane]; }
+    if (lane < cnt) { jC = (int)col[base + row_slot(lane)]; kyC = key[base + lane]; }
     double4 pC = st.pos[jC];
     Q qC = (Q)st.q[jC];
-    if (lane + 64 < cnt) { jB = (int)col[base + row_slot(lane + 64, cnt)]; kyB = key[base + lane + 64]; }
+    if (lane + 64 < cnt) { jB = (int)col[base + row_slot(lane + 64)]; kyB = key[base + lane + 64]; }
     for (int k = lane; k < cnt; k += 64) {
       const double4 pj = pC;
       const Q qj = qC;
@@ -341,7 +341,7 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
       pC = st.pos[jC];
       qC = (Q)st.q[jC];
       jB = i; kyB = 0;
-      if (k + 128 < cnt) { jB = (int)col[base + row_slot(k + 128, cnt)]; kyB = key[base + k + 128]; }
+      if (k + 128 < cnt) { jB = (int)col[base + row_slot(k + 128)]; kyB = key[base + k + 128]; }
       double dx, dy, dz;
       const double r2 = pair_dvec_key([&](int s) { return kTab ? L.shift(s) : shv[s]; }, pi, pj, ky, zero, dx, dy, dz);
       if (r2 <= cut2) {
@@ -458,18 +458,17 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
       }
     }
   };
-  auto store = [&](int count, const Batch& b) {
-    if (lane < count) {
-      const size_t o = rbase + m + (count == kRowGroup ? group_slot(lane) : lane);   // row_slot: m counts full groups
-      if (qb.narrow) qb.col16[o] = (unsigned short)b.j; else qb.col[o] = b.j;
-      if (qb.fp32) {
-        qb.val32[o] = (float)b.h;
-        if (qb.refine) qb.lo32[o] = low(b.h);
-      } else {
-        qb.val[o] = b.h;
-      }
-      if (qb.keyed) qb.key[rbase + m + lane] = (unsigned short)(b.k & 0xFFFF);
+  auto store = [&](int count, const Batch& b) {   // places past the row's end: the row's own column (take) and zero
+    const size_t o = rbase + m + group_slot(lane);   // row_slot: m counts full groups
+    const double h = lane < count ? b.h : 0.0;
+    if (qb.narrow) qb.col16[o] = (unsigned short)b.j; else qb.col[o] = b.j;
+    if (qb.fp32) {
+      qb.val32[o] = (float)h;
+      if (qb.refine) qb.lo32[o] = low(h);
+    } else {
+      qb.val[o] = h;
     }
+    if (qb.keyed && lane < count) qb.key[rbase + m + lane] = (unsigned short)(b.k & 0xFFFF);
     m += count;
   };
   for (int k0 = 0; k0 < cnt; k0 += 128) {

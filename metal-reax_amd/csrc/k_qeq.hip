@@ -114,101 +114,118 @@ __global__ void __launch_bounds__(kThreads) k_cg_guess(int n, QeqBuffers qb, int
 }
 
 // Product layout: kRowLanes lanes per row (64 / kRowLanes rows per wave side by side); lane l adds the entries l, l + 16, ... of its
-// row in turn, four of them from one vector load of columns and one of values (row_slot), two such groups in flight; the row sum
-// is a xor butterfly inside the lane group.
+// row in turn, four of them from one vector load of columns and one of values (row_slot); the row sum is a xor butterfly inside
+// the lane group.
 constexpr int kRowLanes = 16;
-constexpr int kRowGroups = 2;   // groups of 64 entries in flight
 
 // Matrix value accessors: FP64 values, FP32 values, or the two-float pair hi + lo (FP64 to about 48 bits) of the refinement's
-// residuals. Raw: a value as stored, kept in that form until it is used; four: a lane's four values of a full group, side by
-// side. Products and sums are FP64 in every case.
+// residuals. Four: a lane's four values of a group as loaded, widened when they are used. Products and sums are FP64 in every case.
 struct ValD {
-  using Raw = double;
+  struct Four { double2 a, b; };
   const double* v;
-  __device__ Raw one(size_t o) const { return v[o]; }
-  __device__ void four(size_t o, Raw (&h)[4]) const {
+  __device__ double one(size_t o) const { return v[o]; }
+  __device__ ValD from(size_t o) const { return {v + o}; }
+  __device__ Four four(unsigned o) const {
     const double2* p = reinterpret_cast<const double2*>(v + o);
-    const double2 a = p[0], b = p[1];
-    h[0] = a.x; h[1] = a.y; h[2] = b.x; h[3] = b.y;
+    return {p[0], p[1]};
   }
-  static __device__ Raw zero() { return 0.0; }
-  static __device__ double wide(Raw r) { return r; }
+  static __device__ double wide(const Four& f, int u, bool in) { const double h = u == 0 ? f.a.x : u == 1 ? f.a.y : u == 2 ? f.b.x : f.b.y; return in ? h : 0.0; }
 };
 struct ValF {
-  using Raw = float;
+  struct Four { float4 a; };
   const float* v;
-  __device__ Raw one(size_t o) const { return v[o]; }
-  __device__ void four(size_t o, Raw (&h)[4]) const {
-    const float4 a = *reinterpret_cast<const float4*>(v + o);
-    h[0] = a.x; h[1] = a.y; h[2] = a.z; h[3] = a.w;
-  }
-  static __device__ Raw zero() { return 0.0f; }
-  static __device__ double wide(Raw r) { return (double)r; }
+  __device__ double one(size_t o) const { return (double)v[o]; }
+  __device__ ValF from(size_t o) const { return {v + o}; }
+  __device__ Four four(unsigned o) const { return {*reinterpret_cast<const float4*>(v + o)}; }
+  static __device__ double wide(const Four& f, int u, bool in) { const float h = u == 0 ? f.a.x : u == 1 ? f.a.y : u == 2 ? f.a.z : f.a.w; return (double)(in ? h : 0.0f); }
 };
 struct ValDS {
-  struct Raw { float hi, lo; };
+  struct Four { float4 hi, lo; };
   const float* hi;
   const float* lo;
-  __device__ Raw one(size_t o) const { return {hi[o], lo[o]}; }
-  __device__ void four(size_t o, Raw (&h)[4]) const {
-    const float4 a = *reinterpret_cast<const float4*>(hi + o), b = *reinterpret_cast<const float4*>(lo + o);
-    h[0] = {a.x, b.x}; h[1] = {a.y, b.y}; h[2] = {a.z, b.z}; h[3] = {a.w, b.w};
+  __device__ double one(size_t o) const { return (double)hi[o] + (double)lo[o]; }
+  __device__ ValDS from(size_t o) const { return {hi + o, lo + o}; }
+  __device__ Four four(unsigned o) const { return {*reinterpret_cast<const float4*>(hi + o), *reinterpret_cast<const float4*>(lo + o)}; }
+  static __device__ double wide(const Four& f, int u, bool in) {
+    const double h = u == 0 ? (double)f.hi.x + (double)f.lo.x : u == 1 ? (double)f.hi.y + (double)f.lo.y
+                   : u == 2 ? (double)f.hi.z + (double)f.lo.z : (double)f.hi.w + (double)f.lo.w;
+    return in ? h : 0.0;
   }
-  static __device__ Raw zero() { return {0.0f, 0.0f}; }
-  static __device__ double wide(Raw r) { return (double)r.hi + (double)r.lo; }
 };
-__device__ inline void four_columns(const unsigned short* p, int (&j)[4]) {
-  const ushort4 c = *reinterpret_cast<const ushort4*>(p);
-  j[0] = c.x; j[1] = c.y; j[2] = c.z; j[3] = c.w;
-}
-__device__ inline void four_columns(const int* p, int (&j)[4]) {
-  const int4 c = *reinterpret_cast<const int4*>(p);
-  j[0] = c.x; j[1] = c.y; j[2] = c.z; j[3] = c.w;
-}
+template <class TC> struct FourCols;
+template <> struct FourCols<unsigned short> { using T = ushort4; };
+template <> struct FourCols<int> { using T = int4; };
 
 // (H v)_row for both systems (v interleaved), off-diagonal part, summed over the row's lane group (all its lanes get the sum);
-// rows >= n give zero. Columns 32 or 16 bits (TC). Places past the row's end take the row's own column and value 0: they add
-// exact zeros. Bound by the gathers of v (16 bytes per entry through the L1) and the matrix stream: per product launch (HIP
-// events) 24,000 water rows of 422 entries 19.1 us, 192,000 rows with 32-bit columns 164 us (4.0 TB/s of matrix); with one
-// entry per load 20.3 and 172 us. Groups in flight: 1 gives 19.9 and 179 us, 4 gives 22.2 and 174 us (occupancy).
+// rows >= n give zero. Columns 32 or 16 bits (TC). The constructor sends the loads of the row's count and first two groups of 64
+// entries out (the CG kernel reduces the last launch's partials meanwhile), finish() does the rest, two groups at a time. A row that
+// ends before the longest of its wave reads its last group again with weights zero: the loads have no branches, whose waits would be
+// for everything in flight.
+// Bound by the gathers of v (16 bytes per entry through the L1) and the matrix stream (192,000 rows: 3 TB/s). The products of an MD step
+// (about ten) on water, rows of 422 entries: 24,000 rows 175 us, 192,000 rows with 32-bit columns 1458 us, FP64 24,000 rows 216 us; with
+// the last group in list order, read entry by entry, and the first loads after the reduction 179, 1490 and 227 us. The next two
+// groups' entries in flight during a pair's gathers took 186, 1470 and 216 us (90 VGPRs, 5 waves per SIMD: 24,000 rows no longer fit
+// the chip at once; at 80 they just do, which is why the launch's flags and beta are held in scalar registers).
+template <class VA, class TC>
+struct RowProduct {
+  struct Pair { typename FourCols<TC>::T c[2]; typename VA::Four h[2]; };   // two groups
+  const TC* __restrict__ col;   // from the wave's first row on (a scalar address and 32-bit offsets per lane)
+  VA val;
+  const double2* __restrict__ v2;
+  unsigned off;
+  int ng;   // groups of the row
+  Pair A;
+  double y0 = 0, y1 = 0;
+
+  __device__ void load(Pair& p, int f, int g) const {
+    const unsigned o = off + (unsigned)(g * kRowGroup);
+    p.c[f] = *reinterpret_cast<const typename FourCols<TC>::T*>(col + o);
+    p.h[f] = val.four(o);
+  }
+  __device__ RowProduct(int row, int n, int stride, const int* __restrict__ cnt, const TC* __restrict__ col_, const VA val_,
+                        const double2* __restrict__ v2_) : v2(v2_) {
+    const int at = min(row, n - 1), first = __builtin_amdgcn_readfirstlane(at);
+    const size_t base = (size_t)first * stride;
+    col = col_ + base;
+    val = val_.from(base);
+    off = (unsigned)((at - first) * stride + 4 * (lane_id() % kRowLanes));
+    const int c = cnt[at];
+    load(A, 0, 0);
+    load(A, 1, stride > kRowGroup ? 1 : 0);
+    ng = row < n ? (c + kRowGroup - 1) / kRowGroup : 0;
+    if (ng < 1) { A.c[0].x = A.c[0].y = A.c[0].z = A.c[0].w = at; }   // nothing stored there
+    if (ng < 2) A.c[1] = A.c[0];
+  }
+  __device__ double2 at(unsigned j) const { return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(v2) + (j << 4)); }
+  __device__ void gather(const typename FourCols<TC>::T& c, double2 (&x)[4]) const { x[0] = at(c.x); x[1] = at(c.y); x[2] = at(c.z); x[3] = at(c.w); }
+  __device__ void add(const typename VA::Four& h, bool in, const double2 (&x)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const double w = VA::wide(h, u, in);
+      y0 += w * x[u].x;
+      y1 += w * x[u].y;
+    }
+  }
+  __device__ double2 finish() {
+    for (int g = 0;; ) {
+      double2 x[2][4];
+      gather(A.c[0], x[0]);
+      gather(A.c[1], x[1]);
+      add(A.h[0], g < ng, x[0]);
+      add(A.h[1], g + 1 < ng, x[1]);
+      g += 2;
+      if (!__any(g < ng)) break;
+      load(A, 0, max(min(g, ng - 1), 0));   // past the row's end its last group, not used
+      load(A, 1, max(min(g + 1, ng - 1), 0));
+    }
+    return make_double2(group_sum<kRowLanes>(y0), group_sum<kRowLanes>(y1));
+  }
+};
 template <class VA, class TC>
 __device__ inline double2 row_product(int row, int n, int stride, const int* __restrict__ cnt, const TC* __restrict__ col,
                                       const VA val, const double2* __restrict__ v2) {
-  double y0 = 0, y1 = 0;
-  if (row < n) {
-    const int li = lane_id() % kRowLanes, c = cnt[row];
-    const size_t base = (size_t)row * stride;
-    for (int k0 = 0; k0 < c; k0 += kRowGroups * kRowGroup) {
-      int j[kRowGroups][4];
-      typename VA::Raw h[kRowGroups][4];
-      double2 x[kRowGroups][4];
-#pragma unroll
-      for (int f = 0; f < kRowGroups; ++f) {
-        const int g = k0 + f * kRowGroup;
-        if (g + kRowGroup <= c) {
-          four_columns(col + base + g + 4 * li, j[f]);
-          val.four(base + g + 4 * li, h[f]);
-        } else {   // the row's last entries, in list order
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int k = g + u * kRowLanes + li;
-            j[f][u] = row;
-            h[f][u] = VA::zero();
-            if (k < c) { j[f][u] = (int)col[base + k]; h[f][u] = val.one(base + k); }
-          }
-        }
-      }
-#pragma unroll
-      for (int f = 0; f < kRowGroups; ++f)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) x[f][u] = v2[j[f][u]];
-#pragma unroll
-      for (int f = 0; f < kRowGroups; ++f)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) { y0 += VA::wide(h[f][u]) * x[f][u].x; y1 += VA::wide(h[f][u]) * x[f][u].y; }
-    }
-  }
-  return make_double2(group_sum<kRowLanes>(y0), group_sum<kRowLanes>(y1));
+  RowProduct<VA, TC> P(row, n, stride, cnt, col, val, v2);
+  return P.finish();
 }
 
 // Grid of the product kernels: a multiple of the 8 XCDs. Workgroup b is dispatched to XCD b % 8, so it takes the virtual block
@@ -303,6 +320,7 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
                                                         int it, int imax, double tol, int chk) {
   __shared__ double sh[2 * kMvThreads / 64];
   const int i = product_row();
+  RowProduct<VA, TC> P(i, n, stride, qb.cnt, col, val, reinterpret_cast<const double2*>(qb.p));
   int act[2];
   double beta[2] = {0.0, 0.0};
   bool fresh = it == 1;
@@ -334,6 +352,7 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
         put_act(qb, it - 1, s, act[s]);
       }
   }
+  for (int s = 0; s < 2; ++s) { act[s] = __builtin_amdgcn_readfirstlane(act[s]); beta[s] = read_lane(beta[s], 0); }   // one value per launch
   if (!act[0] && !act[1]) return;
   const int li = lane_id() % kRowLanes, s = li / (kRowLanes / 2), k = 2 * i + s;   // this lane's system
   const bool mine = i < n && li % (kRowLanes / 2) == 0 && act[s];
@@ -343,7 +362,7 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
     e = qb.eta[i];
     if (!fresh) { d = qb.d[k]; q = qb.q[k]; }
   }
-  const double2 y = row_product<VA, TC>(i, n, stride, qb.cnt, col, val, reinterpret_cast<const double2*>(qb.p));
+  const double2 y = P.finish();
   double dq[2] = {0.0, 0.0};
   if (mine) {
     const double w = (s ? y.y : y.x) + e * p;
@@ -370,8 +389,8 @@ __global__ void __launch_bounds__(kThreads) k_spmv1(int n, int stride, const int
   const int c = cnt[i];
   double y = 0;
   for (int k = lane; k < c; k += 64) {
-    const size_t o = base + row_slot(k, c);
-    y += VA::wide(val.one(o)) * v[col[o]];
+    const size_t o = base + row_slot(k);
+    y += val.one(o) * v[col[o]];
   }
   y = wave_sum(y);
   if (lane == 0) w[i] = y + eta[i] * v[i];

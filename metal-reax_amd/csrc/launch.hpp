@@ -62,22 +62,19 @@ void launch_vatom_ref(const State& st, hipStream_t s);   // per-atom virials of 
 // ---- non-bonded terms and the charge-equilibration matrix (k_nonbonded.hip)
 void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals& g, const Tables& t, hipStream_t s);
 
-// Place of the k-th of a charge-matrix row's c entries in the row's storage. A full group of 64 entries puts side by side the four
-// entries k = l, l + 16, l + 32, l + 48 that lane l of the product's 16 lanes per row adds in turn, so the lane reads them as one
-// vector (8 bytes of 16-bit columns, 16 bytes of FP32 values); the last, partly filled group stays in list order, so that a
-// short row is not spread over lines it does not fill. Rows are a multiple of 64 entries apart and start on 128-byte lines.
+// Place of the k-th entry of a charge-matrix row in the row's storage: a group of 64 entries puts side by side the four entries
+// k = l, l + 16, l + 32, l + 48 that lane l of the product's 16 lanes per row adds in turn, so the lane reads them as one vector (8
+// bytes of 16-bit columns, 16 bytes of FP32 values). The last group's places past the row's end hold the row's own column and zero.
+// Rows are a multiple of 64 entries apart and start on 128-byte lines.
 constexpr int kRowGroup = 64;
 __host__ __device__ inline int group_slot(int r) { return ((r & 15) << 2) | ((r >> 4) & 3); }
-__host__ __device__ inline int row_slot(int k, int c) {
-  const int g = k & ~(kRowGroup - 1);
-  return g + kRowGroup <= c ? g | group_slot(k) : k;
-}
+__host__ __device__ inline int row_slot(int k) { return (k & ~(kRowGroup - 1)) | group_slot(k); }
 inline int row_stride(int maxnb) { return (maxnb + kRowGroup - 1) / kRowGroup * kRowGroup; }
 
 struct QeqBuffers {
   int stride = 0;            // entries from row to row (row_stride of the skin list's capacity)
   int* cnt = nullptr;        // n: entries per row
-  // the rows are stored in exactly one column format and one value format, entry k of row i at i * stride + row_slot(k, cnt[i]):
+  // the rows are stored in exactly one column format and one value format, entry k of row i at i * stride + row_slot(k):
   int* col = nullptr;               // n * stride: column (owned atom index), when narrow == 0
   unsigned short* col16 = nullptr;  // n * stride: the same in 16 bits, when narrow == 1 (n <= 65535)
   double* val = nullptr;            // n * stride: H_ij in FP64 (FP64 mode)

@@ -61,3 +61,22 @@ def test_rows_with_and_without_tables(ffield_text, shape):
         assert np.array_equal(qa, qb), (shape, prec)
         assert ra["energy"] == rb["energy"], (shape, prec)
         assert np.array_equal(ra["grad"], rb["grad"]) and np.array_equal(ra["virial"], rb["virial"]), (shape, prec)
+
+
+@pytest.mark.gpu
+def test_rows_from_empty_to_several_groups(ffield_text):
+    """A cluster of n atoms in a wide cell, n - 1 entries per row: rows without an entry beside rows of 1, 63, 64, 65 and 129, where a
+    product's groups of 64 begin, end and run past each other in one wave."""
+    rng = np.random.default_rng(11)
+    centres = np.array([[20.0, 20, 20], [60, 20, 20], [20, 60, 20], [60, 60, 20], [20, 20, 60], [60, 20, 60]])
+    x = np.concatenate([c + rng.uniform(-2.5, 2.5, (n, 3)) for c, n in zip(centres, (1, 2, 64, 65, 66, 130))])
+    order = rng.permutation(len(x))
+    x = x[order]
+    types, tags, L = np.full(len(x), 3, dtype=np.int32), np.arange(1, len(x) + 1), np.full(3, 80.0)
+    v = rng.normal(size=len(x))
+    for prec, bar in (("fp64", 1e-12), ("mixed", 1e-6)):   # mixed: FP32 values, 6e-8 each
+        e, species = _engine(ffield_text, (x, types, tags, L), prec, True)
+        y = e.qeq_matvec(v)
+        e.close()
+        yo = Oracle(ffield_text).qeq_matvec(x, species[types - 1], tags, [0, 0, 0, 80, 0, 0, 0, 80, 0, 0, 0, 80], (True, True, True), v)
+        assert np.abs(y - yo).max() <= bar * max(1.0, np.abs(yo).max()), prec
