@@ -13,6 +13,8 @@
 // H (stock fix qeq/reaxff compute_H / calculate_H, LAMMPS fix_qeq_reaxff.cpp): H_ij = 14.4 Tap_q(r) / (r^3 + (g_i g_j)^-1.5)^(1/3) for
 // r^2 <= swb^2, stored as full rows (both directions, every image): FP64 values in FP64 mode, FP32 values otherwise; 16-bit
 // column indices when the system has at most 65535 atoms.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -271,16 +273,28 @@ __global__ void __launch_bounds__(64 * kNbWaves) k_nonbonded_d(State st, Globals
 // What every pair of a row looks up, in LDS (one wave): the shift vectors and the row type's parameters. Read from memory in the
 // pair loop they cost as much address traffic as the positions, and, loads returning in order, a wait for all that is in flight for the
 // next pairs. The non-bonded pass over the rows took 81 us at 24,000 atoms and 661 us at 192,000; with chunks that have no shift taken
-// without one 76 and 588, with these tables 62 and 466, with the row's own data in scalar registers (wave_atom) 58 and 411. Cells with
-// more shifts (thin ones: 64 take 1.5 KB per wave, and leave the matrix build its 6 blocks per CU) or force fields with more types read
-// them from memory.
-constexpr int kTabShifts = 64, kTabTypes = 16;
-inline bool row_tables_fit(const State& st, const Globals& g) {
-  return (long long)(2 * st.smx0 + 1) * (2 * st.smx1 + 1) * (2 * st.smx2 + 1) <= kTabShifts && g.ntypes <= kTabTypes;
+// without one 76 and 588, with these tables 62 and 466, with the row's own data in scalar registers (wave_atom) 58 and 411. Two
+// capacities, since the matrix build's ring leaves room for 8 blocks per CU with 32 shifts (cells wider than the list radius have 27)
+// and for 5 with 128 (125 where one more image is in reach): 40 packed systems with 125 shifts, one capacity of 64 (tables in memory)
+// 23.2 ms for 20 steps, with 128 22.7 ms. Cells with more shifts (thin ones) or force fields with more types read them from memory.
+constexpr int kTabTypes = 16;
+// the tables' capacity in shift vectors (0: no tables)
+inline int row_table_shifts(const State& st, const Globals& g) {
+  const long long ns = (long long)(2 * st.smx0 + 1) * (2 * st.smx1 + 1) * (2 * st.smx2 + 1);
+  return g.ntypes > kTabTypes || ns > 128 ? 0 : ns > 32 ? 128 : 32;
 }
-template <class P>
+// calls f(integral_constant c) for the capacity
+template <class F>
+inline void with_row_tables(const State& st, const Globals& g, F&& f) {
+  switch (row_table_shifts(st, g)) {
+    case 32: f(std::integral_constant<int, 32>{}); break;
+    case 128: f(std::integral_constant<int, 128>{}); break;
+    default: f(std::integral_constant<int, 0>{}); break;
+  }
+}
+template <class P, int kTab>
 struct RowTables {
-  double x[kTabShifts], y[kTabShifts], z[kTabShifts];
+  double x[kTab ? kTab : 1], y[kTab ? kTab : 1], z[kTab ? kTab : 1];
   P par[kTabTypes];
   __device__ void fill_shifts(const State& st, const double4* __restrict__ shv) {
     const int ns = 2 * shift_index(st, 0) + 1;
@@ -305,10 +319,10 @@ __device__ inline double pair_dvec_key(F&& shift, const double4 pi, const double
 // cutoff, so every lane carries a pair (no distance pre-pass, no compaction) and a row costs its column and key (4 bytes per
 // pair with 16-bit columns) instead of the 8-byte skin entries of all pairs out to the list radius. Lane l takes entries l,
 // l + 64, ..., the assignment of the skin-list kernel's compacted batches, so the sums are the same.
-template <bool D, bool kTab, class TC>
+template <bool D, int kTab, class TC>
 __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tables& t, const TC* __restrict__ col,
                                     const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride, int i,
-                                    RowTables<typename NbPrec<D>::Tab>& L) {
+                                    RowTables<typename NbPrec<D>::Tab, kTab>& L) {
   using Q = typename NbPrec<D>::Q;
   const int lane = lane_id();
   const int ti = st.type[i];
@@ -357,18 +371,18 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
 }
 
 // (5 waves per SIMD: 96 VGPRs without spills; the compiler's choice, 106 VGPRs and 4 waves, is slower)
-template <class TC, bool kTab>
+template <class TC, int kTab>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_nonbonded_rows(State st, Globals g, Tables t, const TC* __restrict__ col,
                                                         const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
-  __shared__ RowTables<NbPairF> L[kTab ? 4 : 1];
+  __shared__ RowTables<NbPairF, kTab> L[kTab ? 4 : 1];
   const int i = wave_atom();
   if (i >= st.n) return;
   nb_rows_wave<false, kTab, TC>(st, g, t, col, key, rcnt, stride, i, L[kTab ? threadIdx.x >> 6 : 0]);
 }
-template <class TC, bool kTab>
+template <class TC, int kTab>
 __global__ void __launch_bounds__(256) k_nonbonded_rows_d(State st, Globals g, Tables t, const TC* __restrict__ col,
                                                           const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
-  __shared__ RowTables<NbPairD> L[kTab ? 4 : 1];
+  __shared__ RowTables<NbPairD, kTab> L[kTab ? 4 : 1];
   const int i = wave_atom();
   if (i >= st.n) return;
   nb_rows_wave<true, kTab, TC>(st, g, t, col, key, rcnt, stride, i, L[kTab ? threadIdx.x >> 6 : 0]);
@@ -388,9 +402,9 @@ constexpr int kQbWaves = 4, kQbRing = 256;
 // fuse: the row also forms the charge solve's start from the guess in x (k_cg_guess ran before): y = H x with the values as
 // built (FP64, or the FP32 values a non-refined FP32 solve iterates with), r = b - (y + eta x), p = r / eta, and the row's
 // b.b and r.p for the block partials; this replaces a separate product pass over the rows.
-template <bool kTab>
+template <int kTab>
 __device__ inline void qeq_build_row(const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, int i, int fuse,
-                                     int* rj, int* rk, double* rr, RowTables<double>& L, double (&acc)[4]) {
+                                     int* rj, int* rk, double* rr, RowTables<double, kTab>& L, double (&acc)[4]) {
   const int lane = lane_id();
   const int ti = st.type[i];
   const size_t base = (size_t)i * st.maxnb, rbase = (size_t)i * qb.stride;
@@ -553,9 +567,9 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
   }
 }
 
-template <bool kTab>
+template <int kTab>
 __global__ void __launch_bounds__(256) k_qeq_build(State st, Globals g, Tables t, QeqBuffers qb, int fuse) {
-  __shared__ RowTables<double> L[kTab ? kQbWaves : 1];
+  __shared__ RowTables<double, kTab> L[kTab ? kQbWaves : 1];
   __shared__ int ring_j[kQbWaves][kQbRing];
   __shared__ int ring_k[kQbWaves][kQbRing];   // key | neighbour type << 16
   __shared__ double ring_r2[kQbWaves][kQbRing];
@@ -618,27 +632,26 @@ void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals
   else hipLaunchKernelGGL(k_nonbonded_f, grid, blk, 0, s, st, g, t);
 }
 
-template <bool kTab>
-static void nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
-  const dim3 grid(nblk((long long)st.n * 64, 256)), blk(256);
-  if (p == Precision::FP64) {
-    if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows_d<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
-    else hipLaunchKernelGGL((k_nonbonded_rows_d<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
-  } else {
-    if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
-    else hipLaunchKernelGGL((k_nonbonded_rows<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
-  }
-}
 void launch_nonbonded_rows(Precision p, const State& st, const Globals& g, const Tables& t, const QeqBuffers& qb, hipStream_t s) {
-  if (row_tables_fit(st, g)) nonbonded_rows<true>(p, st, g, t, qb, s);
-  else nonbonded_rows<false>(p, st, g, t, qb, s);
+  const dim3 grid(nblk((long long)st.n * 64, 256)), blk(256);
+  with_row_tables(st, g, [&](auto tab) {
+    constexpr int kTab = decltype(tab)::value;
+    if (p == Precision::FP64) {
+      if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows_d<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+      else hipLaunchKernelGGL((k_nonbonded_rows_d<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
+    } else {
+      if (qb.narrow) hipLaunchKernelGGL((k_nonbonded_rows<unsigned short, kTab>), grid, blk, 0, s, st, g, t, qb.col16, qb.key, qb.cnt, qb.stride);
+      else hipLaunchKernelGGL((k_nonbonded_rows<int, kTab>), grid, blk, 0, s, st, g, t, qb.col, qb.key, qb.cnt, qb.stride);
+    }
+  });
 }
 
 void launch_qeq_build(const State& st, const Cell& c, const Globals& g, const Tables& t, QeqBuffers& qb, int fuse, hipStream_t s) {
   (void)c;
   const dim3 grid(qeq_build_blocks(st.n)), blk(256);
-  if (row_tables_fit(st, g)) hipLaunchKernelGGL(k_qeq_build<true>, grid, blk, 0, s, st, g, t, qb, fuse);
-  else hipLaunchKernelGGL(k_qeq_build<false>, grid, blk, 0, s, st, g, t, qb, fuse);
+  with_row_tables(st, g, [&](auto tab) {
+    hipLaunchKernelGGL(k_qeq_build<decltype(tab)::value>, grid, blk, 0, s, st, g, t, qb, fuse);
+  });
 }
 
 }  // namespace rxa
