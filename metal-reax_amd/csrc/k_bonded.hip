@@ -134,10 +134,13 @@ __device__ inline void angle_and_dcos(const V3<T>& a, T da, const V3<T>& b, T db
 // Bound by the latency of the position gathers at 24,000 atoms and by vector issue above: one evaluation per atom (52 candidates
 // within bond_cut in water, of which 3.4 become bonds) was two thirds of the instructions. 24,000 atoms 70 -> 56 us, 192,000
 // atoms 489 -> 321 us per step (alone on the device).
+// bo_far is looked up in LDS, and the entries are loaded without branches: a lookup in memory came behind the loads for the next chunks
+// and waited for them. 24,000 / 192,000 atoms 55 -> 51 / 293 -> 265 us, 30,000 atoms of disordered carbon 46 -> 42 us.
 // The sums over an atom's bonds are those of a wave with lane l holding candidates l, l + 64, ... of those within bond_cut
 // in turn: a bond's values go to place (number mod 64) of a zeroed row in LDS and the wave sums the row.
 constexpr int kBuildWaves = 4;
 constexpr int kRing = 128;
+constexpr int kFarTypes = 8;   // force fields with more types read bo_far from the pair table
 
 template <class TB>
 struct BuildRing {   // LDS of one wave
@@ -263,10 +266,15 @@ struct BondBuild {
   }
 };
 
-template <class TB>
+template <class TB, bool kTab>
 __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * kBuildWaves) k_bond_build(State st, Globals g, Tables t,
                                                                                                          int per_wave) {
   __shared__ BuildRing<TB> rings[kBuildWaves];
+  __shared__ double far[kTab ? kFarTypes * kFarTypes : 1];
+  if (kTab) {
+    for (int k = threadIdx.x; k < g.ntypes * g.ntypes; k += 64 * kBuildWaves) far[k] = t.pair[k].bo_far;
+    __syncthreads();
+  }
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int first = (int)(blockIdx.x * kBuildWaves + w) * per_wave;
   const int na = min(per_wave, st.n - first);
@@ -285,18 +293,21 @@ __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * k
     k0 += 64;
     while (a < na && k0 >= __builtin_amdgcn_readlane(cl, a)) { ++a; k0 = 0; if (a < na && __builtin_amdgcn_readlane(cl, a) > 0) break; }
   };
-  auto entries = [&](int a, int k0, int& j, int& e) {   // lanes past the row's end carry the wave's first atom, never used
-    j = first; e = 0;
-    if (a < na && k0 + lane < __builtin_amdgcn_readlane(cl, a)) {
-      const size_t o = (size_t)(first + a) * st.maxbc + k0 + lane;
-      j = st.bc_j[o];
-      e = st.bc_s[o];
-    }
+  // a chunk's entries; lanes past the row's end carry its last one, never used (without a chunk, the first atom's: see valid)
+  auto entries = [&](int a, int k0, int& j, int& e) {
+    const int row = min(a, na - 1), last = max(__builtin_amdgcn_readlane(cl, row) - 1, 0);
+    const size_t o = (size_t)(first + row) * st.maxbc;
+    const int q = min(k0 + lane, last);
+    j = st.bc_j[o + q];
+    e = st.bc_s[o + q];
   };
+  // the partner of a chunk's entry, or the first atom where there is no chunk (a row without candidates holds no entries)
+  auto partner = [&](int a, int j) { return a < na ? j : first; };
   int a = 0, k0 = -64;
   next(a, k0);
   int aB = a, kB = k0, jC, eC, jB, eB;
   entries(a, k0, jC, eC);
+  jC = partner(a, jC);
   double4 pC = st.pos[jC];
   next(aB, kB);
   entries(aB, kB, jB, eB);
@@ -304,7 +315,7 @@ __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * k
   while (a < na) {
     const int j = jC, e = eC, ca = a, ck = k0, i = first + a, ti = __builtin_amdgcn_readlane(tl, a);
     const double4 pj = pC, pi = st.pos[i];
-    a = aB; k0 = kB; jC = jB; eC = eB;
+    a = aB; k0 = kB; jC = partner(aB, jB); eC = eB;
     pC = st.pos[jC];
     if (aB < na) next(aB, kB);
     entries(aB, kB, jB, eB);
@@ -315,7 +326,8 @@ __global__ void __attribute__((amdgpu_waves_per_eu(4))) __launch_bounds__(64 * k
       d = sqrt(pair_dvec_pos(st, pi, pj, e, dx, dy, dz));
       near = d <= g.bond_cut;
       tj = pos_type(pj.w);
-      keep = near && d <= t.pair[ti * g.ntypes + tj].bo_far;
+      if constexpr (kTab) keep = near && d <= far[ti * g.ntypes + tj];
+      else keep = near && d <= t.pair[ti * g.ntypes + tj].bo_far;
     }
     const unsigned long long mn = __ballot(near), mk = __ballot(keep);
     if (keep) {
@@ -1767,7 +1779,9 @@ void with_lanes(int lanes, F&& f) {
 template <class TB>
 void bond_build_t(const State& st, const Globals& g, const Tables& t, hipStream_t s) {
   const int per = build_atoms_per_wave(st.n);
-  hipLaunchKernelGGL(k_bond_build<TB>, dim3(nblk(st.n, kBuildWaves * per)), dim3(64 * kBuildWaves), 0, s, st, g, t, per);
+  const dim3 grid(nblk(st.n, kBuildWaves * per)), blk(64 * kBuildWaves);
+  if (g.ntypes <= kFarTypes) hipLaunchKernelGGL((k_bond_build<TB, true>), grid, blk, 0, s, st, g, t, per);
+  else hipLaunchKernelGGL((k_bond_build<TB, false>), grid, blk, 0, s, st, g, t, per);
 }
 
 }  // namespace
