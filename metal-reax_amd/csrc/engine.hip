@@ -1048,7 +1048,7 @@ struct Engine {
     }
     const hipStream_t b = bstream();
     hipEvent_t t0 = timer.begin(PH_TERMS);
-    launch_angle_terms(prec, st, g, tab, std::min(64, bmax * g_mult), b);
+    launch_angle_terms(prec, st, g, tab, std::min(64, bmax * g_mult), g_mult == 1 && both_group_sizes(st.n, flags_h[6]), b);
     timer.end(PH_TERMS, t0);
     t0 = timer.begin(PH_DBOND);
     launch_bond_derivatives(st, b);

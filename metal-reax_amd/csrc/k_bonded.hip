@@ -7,7 +7,7 @@
 //                                 hold bitwise-identical values [bonded.cpp:164-204, terms.hpp:66-164]; index of the mirror slot of
 //                                 every bond and the step's largest bond count
 //   atom_terms  (thread per atom) bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
-//   valence     (wave per 64 / G atoms, angles spread over its lanes) valence angle, penalty, 3-body conjugation at the centre
+//   valence     (wave per 64 / G atoms, angles spread over its lanes; G: both_group_sizes, with_group) valence angle, penalty, 3-body conjugation at the centre
 //                                 [bonded.cpp:321-474]
 //   torsion     (as valence)      torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
 //                                 and derivative contributions of its own half (its own atom, its outer partner, its outer bond) and
@@ -366,7 +366,8 @@ __device__ inline void each_lane(F&& f) {
 // ================================================================================================================
 // corrected bond orders (always from the canonical end) and atom quantities
 // ================================================================================================================
-// Also finds each slot's mirror on the other atom (b_sym) and the step's largest bond count (flags[7]); a slot without a mirror
+// Also finds each slot's mirror on the other atom (b_sym), the step's largest bond count (flags[7]) and the number of atoms with more
+// than 8 bonds (flags[6]); a slot without a mirror
 // sets flags[3]. L lanes per atom, lane p taking slots p, p + L, ...: the slots are independent (the correction reads the
 // uncorrected sums of both ends), so a lane's chain of dependent loads is one slot's instead of the atom's; the total bond order
 // is summed in slot order through the group (the order of a serial loop, so the sums are bitwise those of one thread per atom).
@@ -467,12 +468,15 @@ __global__ void __launch_bounds__(256) k_bo_correct(State st, Globals g, Tables 
   const int nbw = wave_max(nb);
   {   // the largest bond count of this step (flags[7]): one atomic per block, and none where the flag is as large already (atomics
       // on one address follow one another, about 14 ns each)
-    __shared__ int most[4];
-    const int c = wave_max(live && p0 == 0 ? st.b_cnt[i] : 0);
+    __shared__ int most[4], many[4];
+    const int bc = live && p0 == 0 ? st.b_cnt[i] : 0, c = wave_max(bc);
     if (lane_id() == 0) most[threadIdx.x >> 6] = c;
+    const int over = __popcll(__ballot(bc > 8));   // atoms with more than 8 bonds: flags[6]
+    if (lane_id() == 0) many[threadIdx.x >> 6] = over;
     __syncthreads();
     if (threadIdx.x == 0) {
-      const int m = max(max(most[0], most[1]), max(most[2], most[3]));
+      const int m = max(max(most[0], most[1]), max(most[2], most[3])), k = many[0] + many[1] + many[2] + many[3];
+      if (k > 0) atomicAdd(&st.flags[6], k);
       if (m > __hip_atomic_load(&st.flags[7], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&st.flags[7], m);
     }
   }
@@ -702,6 +706,27 @@ struct ItemRows {
 constexpr int kRowClose = 1 << 16;   // tag of a row that ends the rows of slot (tag & 0xFFFF): no items
 constexpr int kAngleWaves = 4;       // waves per block of the angle kernels
 
+// Group sizes of the angle kernels. The sums of an atom are the same with any number of lanes that holds its bonds, so where only a few
+// atoms have 9 to 16 bonds, a launch gives 16 lanes per atom to the aligned groups of 8 atoms that hold one (kBothSizes: the first
+// blocks, a wave per 4 atoms, most of which find nothing to do) and 8 lanes to the others.
+constexpr int kBothSizes = 0;
+inline int angle_blocks(int n, int G) { return (int)(((long long)n * G + 64 * kAngleWaves - 1) / (64 * kAngleWaves)); }
+// f(integral_constant G, first atom) if the wave has atoms to take
+template <int G, class F>
+__device__ __forceinline__ void wave_atoms(const State& st, int blocks16, F&& f) {
+  if constexpr (G != kBothSizes) {
+    f(std::integral_constant<int, G>{}, wave_atom() * (64 / G));
+  } else {
+    const bool wide = (int)blockIdx.x < blocks16;
+    const int first = wide ? wave_atom() * 4 : (wave_atom() - blocks16 * kAngleWaves) * 8;
+    const int at = first / 8 * 8 + lane_id();
+    const int most = wave_max(lane_id() < 8 && at < st.n ? st.b_cnt[at] : 0);
+    if ((most > 8) != wide) return;
+    if (wide) f(std::integral_constant<int, 16>{}, first);
+    else f(std::integral_constant<int, 8>{}, first);
+  }
+}
+
 // Valence angle, penalty and three-body conjugation at the centre j [reference bonded.cpp:321-474]. Lane p of j's group owns bond
 // slot p and the pairs (p, k) with p < k: the contributions to slot p stay with the lane, those to slot k are summed over the
 // group and kept by lane k, and the centre's are summed over the group at the end. Rows: slot k, then parameter set.
@@ -733,7 +758,7 @@ struct ValenceLds {   // one wave
 
 // the item's angle (slots of lanes a and b of the same group) with parameter set `set`
 template <class TR, class TS, int G>
-__device__ inline void valence_item(const Globals& g, const Tables& t, ValenceLds<TR, TS>& L, int e) {
+__device__ __forceinline__ void valence_item(const Globals& g, const Tables& t, ValenceLds<TR, TS>& L, int e) {
   const int who = L.who[e], a = who & 0xFF, b = who >> 8, c = a / G;
   const TR thb_cut = (TR)g.thb_cut;
   const TR p_val6 = (TR)g.p_val6, p_val10 = (TR)g.p_val10;
@@ -791,9 +816,8 @@ __device__ inline void valence_item(const Globals& g, const Tables& t, ValenceLd
 }
 
 template <class TR, class TS, int G, bool PA>
-__device__ inline void valence_body(const State& st, const Globals& g, const Tables& t, ValenceLds<TR, TS>& L) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = gid / G, p = gid % G, n = st.n, lane = lane_id(), base = lane - p;
+__device__ __forceinline__ void valence_body(const State& st, const Globals& g, const Tables& t, ValenceLds<TR, TS>& L, int first) {
+  const int lane = lane_id(), j = first + lane / G, p = lane % G, n = st.n, base = lane - p;
   const bool live = j < n;
   const int tj = live ? st.type[j] : -1;
   const int nb = live ? min(st.b_cnt[j], st.maxb) : 0;
@@ -1007,14 +1031,18 @@ __device__ inline void valence_body(const State& st, const Globals& g, const Tab
 }
 
 template <class TS, int G, bool PA>
-__global__ void __launch_bounds__(64 * kAngleWaves) k_valence(State st, Globals g, Tables t) {
+__global__ void __launch_bounds__(64 * kAngleWaves) k_valence(State st, Globals g, Tables t, int blocks16) {
   __shared__ ValenceLds<float, TS> L[kAngleWaves];
-  valence_body<float, TS, G, PA>(st, g, t, L[threadIdx.x >> 6]);
+  wave_atoms<G>(st, blocks16, [&](auto gc, int first) {
+    valence_body<float, TS, decltype(gc)::value, PA>(st, g, t, L[threadIdx.x >> 6], first);
+  });
 }
 template <int G, bool PA>
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_valence_d(State st, Globals g, Tables t) {
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_valence_d(State st, Globals g, Tables t, int blocks16) {
   __shared__ ValenceLds<double, double> L[kAngleWaves];
-  valence_body<double, double, G, PA>(st, g, t, L[threadIdx.x >> 6]);
+  wave_atoms<G>(st, blocks16, [&](auto gc, int first) {
+    valence_body<double, double, decltype(gc)::value, PA>(st, g, t, L[threadIdx.x >> 6], first);
+  });
 }
 
 template <class TR>
@@ -1061,7 +1089,7 @@ struct TorsionLds {   // one wave
 
 // item e: the torsion i - j - k - l, its gates on l's image and parameter set first
 template <class TR, class TS, bool PA>
-__device__ inline void torsion_item(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L, int e) {
+__device__ __forceinline__ void torsion_item(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L, int e) {
   const int who = L.who[e], a = who & 63, b = who >> 6 & 63, pl = who >> 12, n = st.n;
   const int k = L.j[a], sk = L.s[a], i = L.j[b], si = L.s[b];
   const size_t ql = sl(pl, k, n);
@@ -1164,9 +1192,8 @@ __device__ inline void torsion_item(const State& st, const Globals& g, const Tab
 }
 
 template <class TR, class TS, int G, bool kCen, bool PA>
-__device__ inline void torsion_body(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = gid / G, pk = gid % G, n = st.n, lane = lane_id(), base = lane - pk;
+__device__ __forceinline__ void torsion_body(const State& st, const Globals& g, const Tables& t, TorsionLds<TR, TS, PA>& L, int first) {
+  const int lane = lane_id(), j = first + lane / G, pk = lane % G, n = st.n, base = lane - pk;
   const bool live = j < n;
   const int tj = live ? st.type[j] : -1;
   const int nbj = live ? min(st.b_cnt[j], st.maxb) : 0;
@@ -1348,14 +1375,18 @@ __device__ inline void torsion_body(const State& st, const Globals& g, const Tab
 // FP32 terms: 156 VGPRs and 45 KB of LDS per block, 3 waves per SIMD; FP64 held to 2 (216 VGPRs, 67 KB). kCen: the variant that also
 // records the torsion census (launched only for a force call that asks for it, so the counter costs the ordinary step nothing)
 template <class TS, int G, bool kCen, bool PA>
-__global__ void __launch_bounds__(64 * kAngleWaves) k_torsion_f(State st, Globals g, Tables t) {
+__global__ void __launch_bounds__(64 * kAngleWaves) k_torsion_f(State st, Globals g, Tables t, int blocks16) {
   __shared__ TorsionLds<float, TS, PA> L[kAngleWaves];
-  torsion_body<float, TS, G, kCen, PA>(st, g, t, L[threadIdx.x >> 6]);
+  wave_atoms<G>(st, blocks16, [&](auto gc, int first) {
+    torsion_body<float, TS, decltype(gc)::value, kCen, PA>(st, g, t, L[threadIdx.x >> 6], first);
+  });
 }
 template <int G, bool kCen, bool PA>
-__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_torsion_d(State st, Globals g, Tables t) {
+__global__ void __attribute__((amdgpu_waves_per_eu(2))) __launch_bounds__(64 * kAngleWaves) k_torsion_d(State st, Globals g, Tables t, int blocks16) {
   __shared__ TorsionLds<double, double, PA> L[kAngleWaves];
-  torsion_body<double, double, G, kCen, PA>(st, g, t, L[threadIdx.x >> 6]);
+  wave_atoms<G>(st, blocks16, [&](auto gc, int first) {
+    torsion_body<double, double, decltype(gc)::value, kCen, PA>(st, g, t, L[threadIdx.x >> 6], first);
+  });
 }
 
 // ================================================================================================================
@@ -1805,29 +1836,46 @@ void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tab
 // a smaller group (the extra lanes add exact zeros ahead of the same butterfly), so a per-atom call leaves the energies and the
 // gradient bitwise unchanged
 template <class TR, class TS, int G, bool PA>
-void launch_terms_g(const State& st, const Globals& g, const Tables& t, hipStream_t s) {
-  const dim3 grid(nblk((long long)st.n * G, 256)), blk(256), wgrid(nblk(st.n, 4));
-  if (sizeof(TR) == 4) hipLaunchKernelGGL((k_valence<TS, G, PA>), grid, blk, 0, s, st, g, t);
-  else hipLaunchKernelGGL((k_valence_d<G, PA>), grid, blk, 0, s, st, g, t);
+void launch_angles(const State& st, const Globals& g, const Tables& t, hipStream_t s) {
+  const int b16 = G == kBothSizes ? angle_blocks(st.n, 16) : 0;
+  const dim3 grid(b16 + angle_blocks(st.n, G == kBothSizes ? 8 : G)), blk(64 * kAngleWaves);
   if (sizeof(TR) == 4) {
-    if (st.census) hipLaunchKernelGGL((k_torsion_f<TS, G, true, PA>), grid, blk, 0, s, st, g, t);
-    else hipLaunchKernelGGL((k_torsion_f<TS, G, false, PA>), grid, blk, 0, s, st, g, t);
+    hipLaunchKernelGGL((k_valence<TS, G, PA>), grid, blk, 0, s, st, g, t, b16);
+    if (st.census) hipLaunchKernelGGL((k_torsion_f<TS, G, true, PA>), grid, blk, 0, s, st, g, t, b16);
+    else hipLaunchKernelGGL((k_torsion_f<TS, G, false, PA>), grid, blk, 0, s, st, g, t, b16);
   } else {
-    if (st.census) hipLaunchKernelGGL((k_torsion_d<G, true, PA>), grid, blk, 0, s, st, g, t);
-    else hipLaunchKernelGGL((k_torsion_d<G, false, PA>), grid, blk, 0, s, st, g, t);
+    hipLaunchKernelGGL((k_valence_d<G, PA>), grid, blk, 0, s, st, g, t, b16);
+    if (st.census) hipLaunchKernelGGL((k_torsion_d<G, true, PA>), grid, blk, 0, s, st, g, t, b16);
+    else hipLaunchKernelGGL((k_torsion_d<G, false, PA>), grid, blk, 0, s, st, g, t, b16);
   }
+}
+
+template <class TR, class TS, bool PA>
+void launch_hbonds(const State& st, const Globals& g, const Tables& t, hipStream_t s) {
   hipLaunchKernelGGL((k_hbond_donor<TR, TS, PA>), dim3(nblk(st.n, kHbWaves)), dim3(64 * kHbWaves), 0, s, st, g, t);
-  hipLaunchKernelGGL(k_hbond_acceptor<TR>, wgrid, blk, 0, s, st, g, t);
+  hipLaunchKernelGGL(k_hbond_acceptor<TR>, dim3(nblk(st.n, 4)), dim3(256), 0, s, st, g, t);
+}
+
+// calls f(integral_constant G) for the smallest group size that holds bmax bonds
+template <class F>
+void with_group(int bmax, F&& f) {
+  if (bmax <= 4) f(std::integral_constant<int, 4>{});
+  else if (bmax <= 8) f(std::integral_constant<int, 8>{});
+  else if (bmax <= 16) f(std::integral_constant<int, 16>{});
+  else if (bmax <= 32) f(std::integral_constant<int, 32>{});
+  else f(std::integral_constant<int, 64>{});
 }
 
 template <class TR, class TS>
-void launch_terms_t(const State& st, const Globals& g, const Tables& t, int bmax, hipStream_t s) {
-  if (st.peratom) launch_terms_g<TR, TS, 64, true>(st, g, t, s);
-  else if (bmax <= 4) launch_terms_g<TR, TS, 4, false>(st, g, t, s);
-  else if (bmax <= 8) launch_terms_g<TR, TS, 8, false>(st, g, t, s);
-  else if (bmax <= 16) launch_terms_g<TR, TS, 16, false>(st, g, t, s);
-  else if (bmax <= 32) launch_terms_g<TR, TS, 32, false>(st, g, t, s);
-  else launch_terms_g<TR, TS, 64, false>(st, g, t, s);
+void launch_terms_t(const State& st, const Globals& g, const Tables& t, int bmax, bool both, hipStream_t s) {
+  if (st.peratom) {
+    launch_angles<TR, TS, 64, true>(st, g, t, s);
+    launch_hbonds<TR, TS, true>(st, g, t, s);
+    return;
+  }
+  if (both && bmax > 8 && bmax <= 16) launch_angles<TR, TS, kBothSizes, false>(st, g, t, s);
+  else with_group(bmax, [&](auto gc) { launch_angles<TR, TS, decltype(gc)::value, false>(st, g, t, s); });
+  launch_hbonds<TR, TS, false>(st, g, t, s);
 }
 
 void launch_atom_terms(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s) {
@@ -1840,10 +1888,10 @@ void launch_atom_terms(Precision p, const State& st, const Globals& g, const Tab
   });
 }
 
-void launch_angle_terms(Precision p, const State& st, const Globals& g, const Tables& t, int bmax, hipStream_t s) {
-  if (p == Precision::FP64) launch_terms_t<double, double>(st, g, t, bmax, s);
-  else if (p == Precision::MIXED) launch_terms_t<float, double>(st, g, t, bmax, s);
-  else launch_terms_t<float, float>(st, g, t, bmax, s);
+void launch_angle_terms(Precision p, const State& st, const Globals& g, const Tables& t, int bmax, bool both, hipStream_t s) {
+  if (p == Precision::FP64) launch_terms_t<double, double>(st, g, t, bmax, both, s);
+  else if (p == Precision::MIXED) launch_terms_t<float, double>(st, g, t, bmax, both, s);
+  else launch_terms_t<float, float>(st, g, t, bmax, both, s);
 }
 
 void launch_bond_derivatives(const State& st, hipStream_t s) {

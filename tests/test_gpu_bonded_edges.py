@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from helpers import new_engine
+from reaxamd import systems
 from oracle.oracle import Oracle
 
 TERMS = ("e_bond", "e_ov", "e_un", "e_lp", "e_ang", "e_pen", "e_coa", "e_tor", "e_con", "e_vdW")
@@ -95,3 +96,24 @@ def test_many_bonds(a, cells, drop):
             assert np.abs(d).max() <= 4e-3 and np.sqrt((d ** 2).mean()) <= 9e-4, n
         for k, name in enumerate(("bonds", "angle_sets", "torsions")):
             assert np.array_equal(cen[k], np.asarray(ref["census"][name])), (n, prec, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,density", [(13003, 1.6), (12000, 1.3)])
+def test_two_group_sizes(n, density):
+    """Disordered carbon with a few atoms of 9 to 16 bonds: the launch that gives 16 lanes to their groups of 8 atoms and 8 to the rest
+    against the per-atom call, which takes 64 lanes for every atom: the sums are the same, bit for bit."""
+    with open(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "ffield.C2013")) as fh:
+        ff = fh.read()
+    w = systems.random_carbon(n, density=density, seed=4)
+    for prec in ("fp64", "mixed", "fp32"):
+        e = new_engine(ff, ["C"], prec, extra=("checkqeq", "no"))
+        e.set_box(w.lo, w.hi)
+        e.set_atoms(w.types, w.tags, w.x)
+        r = e.compute(rebuild=True, census=True)
+        bonds = np.asarray(e.census()[0])
+        ra = e.compute(peratom=True)
+        e.close()
+        assert 8 < bonds.max() <= 16 and 0 < 64 * (bonds > 8).sum() <= n, (bonds.max(), (bonds > 8).sum())   # the launch in question
+        assert r["energy"] == ra["energy"], prec
+        assert np.array_equal(r["grad"], ra["grad"]) and np.array_equal(r["virial"], ra["virial"]), prec
