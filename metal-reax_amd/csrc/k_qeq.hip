@@ -158,14 +158,15 @@ template <> struct FourCols<int> { using T = int4; };
 
 // (H v)_row for both systems (v interleaved), off-diagonal part, summed over the row's lane group (all its lanes get the sum);
 // rows >= n give zero. Columns 32 or 16 bits (TC). The constructor sends the loads of the row's count and first two groups of 64
-// entries out (the CG kernel reduces the last launch's partials meanwhile), finish() does the rest, two groups at a time. A row that
-// ends before the longest of its wave reads its last group again with weights zero: the loads have no branches, whose waits would be
-// for everything in flight.
+// entries out, finish() does the rest, two groups at a time. A row that ends before the longest of its wave reads its last group
+// again with weights zero: the loads have no branches, whose waits would be for everything in flight.
 // Bound by the gathers of v (16 bytes per entry through the L1) and the matrix stream (192,000 rows: 3 TB/s). The products of an MD step
-// (about ten) on water, rows of 422 entries: 24,000 rows 175 us, 192,000 rows with 32-bit columns 1458 us, FP64 24,000 rows 216 us; with
-// the last group in list order, read entry by entry, and the first loads after the reduction 179, 1490 and 227 us. The next two
-// groups' entries in flight during a pair's gathers took 186, 1470 and 216 us (90 VGPRs, 5 waves per SIMD: 24,000 rows no longer fit
-// the chip at once; at 80 they just do, which is why the launch's flags and beta are held in scalar registers).
+// (about ten) on water, rows of 422 entries: 24,000 rows 172 us, 192,000 rows with 32-bit columns 1468 us, FP64 24,000 rows 208 us; with
+// the last group in list order, read entry by entry, 179, 1530 and 227 us. With the first loads sent before the reduction of the last
+// launch's partials, 175, 1526 and 215 us: a launch after both solves have stopped then reads two groups of every row for nothing (28 us
+// instead of 4 at 192,000 rows). The next two groups' entries in flight during a pair's gathers took 186, 1540 and 216 us (90 VGPRs, 5
+// waves per SIMD: 24,000 rows no longer fit the chip at once; at 80 they just do, which is why the launch's flags and beta are held in
+// scalar registers).
 template <class VA, class TC>
 struct RowProduct {
   struct Pair { typename FourCols<TC>::T c[2]; typename VA::Four h[2]; };   // two groups
@@ -320,7 +321,6 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
                                                         int it, int imax, double tol, int chk) {
   __shared__ double sh[2 * kMvThreads / 64];
   const int i = product_row();
-  RowProduct<VA, TC> P(i, n, stride, qb.cnt, col, val, reinterpret_cast<const double2*>(qb.p));
   int act[2];
   double beta[2] = {0.0, 0.0};
   bool fresh = it == 1;
@@ -354,6 +354,7 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
   }
   for (int s = 0; s < 2; ++s) { act[s] = __builtin_amdgcn_readfirstlane(act[s]); beta[s] = read_lane(beta[s], 0); }   // one value per launch
   if (!act[0] && !act[1]) return;
+  RowProduct<VA, TC> P(i, n, stride, qb.cnt, col, val, reinterpret_cast<const double2*>(qb.p));
   const int li = lane_id() % kRowLanes, s = li / (kRowLanes / 2), k = 2 * i + s;   // this lane's system
   const bool mine = i < n && li % (kRowLanes / 2) == 0 && act[s];
   double p = 0, e = 0, d = 0, q = 0;
