@@ -532,7 +532,7 @@ __device__ inline void qeq_build_row(const State& st, const Globals& g, const Ta
     if (nfull > 0) store(64, b0);
     if (nfull > 1) store(64, b1);
   }
-  if (fill > 0) {
+  if (fill > 0 || m == 0) {   // (an empty row gets one group of such places: the product reads a row's last group again)
     Batch b;
     const int count = fill;
     take(count, b);

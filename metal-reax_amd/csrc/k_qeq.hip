@@ -159,7 +159,8 @@ template <> struct FourCols<int> { using T = int4; };
 // (H v)_row for both systems (v interleaved), off-diagonal part, summed over the row's lane group (all its lanes get the sum);
 // rows >= n give zero. Columns 32 or 16 bits (TC). The constructor sends the loads of the row's count and first two groups of 64
 // entries out, finish() does the rest, two groups at a time. A row that ends before the longest of its wave reads its last group
-// again with weights zero: the loads have no branches, whose waits would be for everything in flight.
+// again with weights zero (an empty row its one group of padding): the loads have no branches, whose waits would be for everything in
+// flight.
 // Bound by the gathers of v (16 bytes per entry through the L1) and the matrix stream (192,000 rows: 3 TB/s). The products of an MD step
 // (about ten) on water, rows of 422 entries: 24,000 rows 172 us, 192,000 rows with 32-bit columns 1468 us, FP64 24,000 rows 208 us; with
 // the last group in list order, read entry by entry, 179, 1530 and 227 us. With the first loads sent before the reduction of the last
@@ -194,8 +195,7 @@ struct RowProduct {
     load(A, 0, 0);
     load(A, 1, stride > kRowGroup ? 1 : 0);
     ng = row < n ? (c + kRowGroup - 1) / kRowGroup : 0;
-    if (ng < 1) { A.c[0].x = A.c[0].y = A.c[0].z = A.c[0].w = at; }   // nothing stored there
-    if (ng < 2) A.c[1] = A.c[0];
+    if (ng < 2) A.c[1] = A.c[0];   // nothing stored there
   }
   __device__ double2 at(unsigned j) const { return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(v2) + (j << 4)); }
   __device__ void gather(const typename FourCols<TC>::T& c, double2 (&x)[4]) const { x[0] = at(c.x); x[1] = at(c.y); x[2] = at(c.z); x[3] = at(c.w); }

@@ -69,7 +69,8 @@ void launch_nonbonded(Precision p, const State& st, const Cell& c, const Globals
 
 // Place of the k-th entry of a charge-matrix row in the row's storage: a group of 64 entries puts side by side the four entries
 // k = l, l + 16, l + 32, l + 48 that lane l of the product's 16 lanes per row adds in turn, so the lane reads them as one vector (8
-// bytes of 16-bit columns, 16 bytes of FP32 values). The last group's places past the row's end hold the row's own column and zero.
+// bytes of 16-bit columns, 16 bytes of FP32 values). The last group's places past the row's end hold the row's own column and zero; an
+// empty row has one group of such places.
 // Rows are a multiple of 64 entries apart and start on 128-byte lines.
 constexpr int kRowGroup = 64;
 __host__ __device__ inline int group_slot(int r) { return ((r & 15) << 2) | ((r >> 4) & 3); }
