@@ -12,7 +12,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <limits>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -21,6 +20,7 @@
 #include <unordered_map>
 
 #include "../../include/reaxamd.h"
+#include "bond_reach.hpp"
 #include "common.hpp"
 #include "ffield.hpp"
 #include "launch.hpp"
@@ -340,35 +340,6 @@ struct Engine {
     return overlap && !(timer.on && (timer.mask & bonded_phases)) ? sb : stream;
   }
 
-  // Distance beyond which BO' stays below bo_cut, so that no bond is listed there: each kind of bond falls with the distance when its
-  // coefficient is negative and its power positive (then so does BO'); the bound is where BO' falls to bo_cut less 1e-3 of it,
-  // far beyond the rounding of the single-precision powers. Anything else: infinite, every candidate is evaluated.
-  static double bo_far(const DevPair& p, double bo_cut) {
-    const double inf = std::numeric_limits<double>::infinity();
-    const struct { int on; double a, b, r; } kind[3] = {{p.s_ok, p.p_bo1, p.p_bo2, p.r_s}, {p.pi_ok, p.p_bo3, p.p_bo4, p.r_p}, {p.pp_ok, p.p_bo5, p.p_bo6, p.r_pp}};
-    for (const auto& k : kind)
-      if (k.on && !(k.a < 0.0 && k.b > 0.0 && k.r > 0.0)) return inf;
-    const double limit = bo_cut * (1.0 - 1e-3);
-    if (!(limit > 0.0)) return inf;
-    auto bo = [&](double d) {
-      double v = 0;
-      for (int k = 0; k < 3; ++k)
-        if (kind[k].on) v += (k == 0 ? 1.0 + bo_cut : 1.0) * std::exp(kind[k].a * std::pow(d / kind[k].r, kind[k].b));
-      return v;
-    };
-    double lo = 0.0, hi = 1.0;
-    while (bo(hi) >= limit) {
-      lo = hi;
-      hi *= 2.0;
-      if (!(hi < 1e6)) return inf;
-    }
-    for (int k = 0; k < 100; ++k) {
-      const double m = 0.5 * (lo + hi);
-      (bo(m) >= limit ? lo : hi) = m;
-    }
-    return hi;
-  }
-
   // ---------------------------------------------------------------------------------------------------------------
   void pack_tables() {
     const int nt = ff.ntypes();
@@ -402,7 +373,11 @@ struct Engine {
         d.pgw = std::pow(1.0 / p.gamma_w, ff.gp[28]);
         d.irvdw = 1.0 / p.r_vdW;
         d.ircore = 1.0 / p.rcore;
-        d.bo_far = bo_far(d, ff.bo_cut);
+        // (the table is symmetric)
+        const BondKind kinds[3] = {{d.s_ok != 0, p.p_bo1, p.p_bo2, p.r_s, 1.0 + ff.bo_cut},
+                                   {d.pi_ok != 0, p.p_bo3, p.p_bo4, p.r_p, 1.0},
+                                   {d.pp_ok != 0, p.p_bo5, p.p_bo6, p.r_pp, 1.0}};
+        d.bo_far = j < i ? pr[(size_t)j * nt + i].bo_far : bond_reach(kinds, ff.bo_cut);
         d.re6 = (p.lgre * p.lgre * p.lgre) * (p.lgre * p.lgre * p.lgre);
         pr[(size_t)i * nt + j] = d;
       }
