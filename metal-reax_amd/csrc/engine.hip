@@ -980,6 +980,8 @@ struct Engine {
   // an event on the main stream after which the bonded chain may start (set by the MD loop for a step that keeps its lists:
   // the positions are final there, before the charge matrix of the step is queued); otherwise the fork is recorded here
   hipEvent_t fork_after = nullptr;
+  // the angle kernels' limit of atoms with more than 8 bonds (per-atom calls and doubled groups: one group size)
+  int limit8() const { return g_mult == 1 && !st.peratom ? both_sizes_limit(st.n) : -1; }
   void bonded_begin() {
     const hipStream_t b = bstream();
     if (b != stream) {
@@ -992,7 +994,7 @@ struct Engine {
     launch_bond_build(prec, st, g, tab, b);
     timer.end(PH_BONDS, t0);
     t0 = timer.begin(PH_BOCORR);
-    launch_bo_correct(prec, st, g, tab, b);
+    launch_bo_correct(prec, st, g, tab, limit8(), b);
     timer.end(PH_BOCORR, t0);
     launch_flags_out(st.flags, flags_h, b);
     HIPCHK(hipEventRecord(ev_flags, b));
@@ -1023,7 +1025,7 @@ struct Engine {
     }
     const hipStream_t b = bstream();
     hipEvent_t t0 = timer.begin(PH_TERMS);
-    launch_angle_terms(prec, st, g, tab, std::min(64, bmax * g_mult), g_mult == 1 && both_group_sizes(st.n, flags_h[6]), b);
+    launch_angle_terms(prec, st, g, tab, std::min(64, bmax * g_mult), flags_h[6] <= limit8(), b);
     timer.end(PH_TERMS, t0);
     t0 = timer.begin(PH_DBOND);
     launch_bond_derivatives(st, b);

@@ -7,7 +7,7 @@
 //                                 hold bitwise-identical values [bonded.cpp:164-204, terms.hpp:66-164]; index of the mirror slot of
 //                                 every bond and the step's largest bond count
 //   atom_terms  (thread per atom) bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
-//   valence     (wave per 64 / G atoms, angles spread over its lanes; G: both_group_sizes, with_group) valence angle, penalty, 3-body conjugation at the centre
+//   valence     (wave per 64 / G atoms, angles spread over its lanes; G: both_sizes_limit, with_group) valence angle, penalty, 3-body conjugation at the centre
 //                                 [bonded.cpp:321-474]
 //   torsion     (as valence)      torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
 //                                 and derivative contributions of its own half (its own atom, its outer partner, its outer bond) and
@@ -366,14 +366,15 @@ __device__ inline void each_lane(F&& f) {
 // ================================================================================================================
 // corrected bond orders (always from the canonical end) and atom quantities
 // ================================================================================================================
-// Also finds each slot's mirror on the other atom (b_sym), the step's largest bond count (flags[7]) and the number of atoms with more
-// than 8 bonds (flags[6]); a slot without a mirror
-// sets flags[3]. L lanes per atom, lane p taking slots p, p + L, ...: the slots are independent (the correction reads the
+// Also finds each slot's mirror on the other atom (b_sym), the step's largest bond count (flags[7]) and, where the angle kernels' launch
+// asks for it, the number of atoms with more than 8 bonds (flags[6], exact up to limit8; -1: not counted); a slot without a mirror sets
+// flags[3]. L lanes per atom, lane p taking slots p, p + L, ...: the slots are independent (the correction reads the
 // uncorrected sums of both ends), so a lane's chain of dependent loads is one slot's instead of the atom's; the total bond order
 // is summed in slot order through the group (the order of a serial loop, so the sums are bitwise those of one thread per atom).
 // Bound by latency: four slots of the mirror search are in flight at a time, after the loads that the correction needs. 648 / 24,000 /
 // 192,000 atoms: 17.9 / 41 / 176 us with a search slot by slot and an atomic per wave for the largest count, 15.9 / 37 / 171 us with
-// the search as it is, 14.4 / 23 / 86 us with one atomic per block at most as well.
+// the search as it is, 14.4 / 23 / 86 us with the largest count's atomics as they are. Dense carbon, where most blocks hold an atom with
+// more than 8 bonds: 11,000 atoms 28.6 us with the number of them always counted, 26.4 as it is; 30,000 45 / 41 us.
 
 // the mirror slot, the corrected bond orders and the derivative coefficients of slot p of atom i; returns the corrected BO
 template <class TB>
@@ -460,23 +461,25 @@ __device__ inline TB bo_correct_slot(const State& st, const Globals& g, const Ta
 }
 
 template <class TB, int L>
-__global__ void __launch_bounds__(256) k_bo_correct(State st, Globals g, Tables t) {
+__global__ void __launch_bounds__(256) k_bo_correct(State st, Globals g, Tables t, int limit8) {
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
   const int i = gid / L, p0 = gid % L, n = st.n;
   const bool live = i < n;
   const int nb = live ? min(st.b_cnt[i], st.maxb) : 0;
   const int nbw = wave_max(nb);
-  {   // the largest bond count of this step (flags[7]): one atomic per block, and none where the flag is as large already (atomics
-      // on one address follow one another, about 14 ns each)
+  {   // the largest bond count of this step (flags[7]) and the atoms with more than 8 bonds (flags[6]): at most one atomic each per block,
+      // and none where the flag is as large already, or the count beyond its limit (atomics on one address follow one another, about
+      // 14 ns each)
     __shared__ int most[4], many[4];
     const int bc = live && p0 == 0 ? st.b_cnt[i] : 0, c = wave_max(bc);
     if (lane_id() == 0) most[threadIdx.x >> 6] = c;
-    const int over = __popcll(__ballot(bc > 8));   // atoms with more than 8 bonds: flags[6]
+    const int over = __popcll(__ballot(bc > 8));
     if (lane_id() == 0) many[threadIdx.x >> 6] = over;
     __syncthreads();
     if (threadIdx.x == 0) {
       const int m = max(max(most[0], most[1]), max(most[2], most[3])), k = many[0] + many[1] + many[2] + many[3];
-      if (k > 0) atomicAdd(&st.flags[6], k);
+      if (limit8 >= 0 && k > 0 && __hip_atomic_load(&st.flags[6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= limit8)
+        atomicAdd(&st.flags[6], k);
       if (m > __hip_atomic_load(&st.flags[7], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&st.flags[7], m);
     }
   }
@@ -1823,12 +1826,12 @@ void launch_bond_build(Precision p, const State& st, const Globals& g, const Tab
 }
 
 
-void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s) {
+void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tables& t, int limit8, hipStream_t s) {
   with_lanes(st.lanes, [&](auto lc) {
     constexpr int L = decltype(lc)::value;
     const dim3 grid(nblk((long long)st.n * L, 256)), blk(256);
-    if (p == Precision::FP32) hipLaunchKernelGGL((k_bo_correct<float, L>), grid, blk, 0, s, st, g, t);
-    else hipLaunchKernelGGL((k_bo_correct<double, L>), grid, blk, 0, s, st, g, t);
+    if (p == Precision::FP32) hipLaunchKernelGGL((k_bo_correct<float, L>), grid, blk, 0, s, st, g, t, limit8);
+    else hipLaunchKernelGGL((k_bo_correct<double, L>), grid, blk, 0, s, st, g, t, limit8);
   });
 }
 

@@ -48,15 +48,14 @@ void launch_acceptor_rows(const State& st, const Globals& g, const Tables& t, hi
 
 // ---- bond-order chain and bonded terms (k_bonded.hip)
 void launch_bond_build(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s);
-void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s);
-// bond energy / lone pair / over-under (no group size needed), then valence, torsion, H-bonds with the group size for the
-// largest bond count bmax (both: see both_group_sizes)
+// (limit8: also the number of atoms with more than 8 bonds, exact up to this limit, see both_sizes_limit; -1: not counted)
+void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tables& t, int limit8, hipStream_t s);
 void launch_atom_terms(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s);
-// Whether the angle kernels take 8 and 16 lanes per atom in one launch, given the number of atoms with more than 8 bonds (and none with
-// more than 16). The three term kernels at 30,000 atoms of carbon, 16 lanes for all against both: 0.4 % such atoms 248 / 213 us, 2.1 %
+// The angle kernels take 8 and 16 lanes per atom in one launch where at most this many atoms have more than 8 bonds (and none more than
+// 16); -1: never. The three term kernels at 30,000 atoms of carbon, 16 lanes for all against both: 0.4 % such atoms 248 / 213 us, 2.1 %
 // 279 / 286 us, 5.8 % 323 / 369 us (a group of 8 atoms with one of them costs as before, and its launch finds the others by their
 // counts). 6,000 atoms, one wave per SIMD either way: 0.07 % 97 / 98 us, 1.3 % 125 / 131 us.
-inline bool both_group_sizes(int n, int over8) { return n >= 12000 && over8 * 64LL <= n; }
+inline int both_sizes_limit(int n) { return n < 12000 ? -1 : n / 64; }
 void launch_angle_terms(Precision p, const State& st, const Globals& g, const Tables& t, int bmax, bool both, hipStream_t s);
 // BO-derivative pass (CdDelta, then the per-atom bond sums); the final gather adds the non-bonded gradient and the virial
 void launch_bond_derivatives(const State& st, hipStream_t s);
