@@ -981,7 +981,7 @@ struct Engine {
   // the positions are final there, before the charge matrix of the step is queued); otherwise the fork is recorded here
   hipEvent_t fork_after = nullptr;
   // the angle kernels' limit of atoms with more than 8 bonds (per-atom calls and doubled groups: one group size)
-  int limit8() const { return g_mult == 1 && !st.peratom ? both_sizes_limit(st.n) : -1; }
+  int limit8() const { return g_mult == 1 && !st.peratom ? both_sizes_limit(prec, st.n) : -1; }
   void bonded_begin() {
     const hipStream_t b = bstream();
     if (b != stream) {

@@ -52,10 +52,15 @@ void launch_bond_build(Precision p, const State& st, const Globals& g, const Tab
 void launch_bo_correct(Precision p, const State& st, const Globals& g, const Tables& t, int limit8, hipStream_t s);
 void launch_atom_terms(Precision p, const State& st, const Globals& g, const Tables& t, hipStream_t s);
 // The angle kernels take 8 and 16 lanes per atom in one launch where at most this many atoms have more than 8 bonds (and none more than
-// 16); -1: never. The three term kernels at 30,000 atoms of carbon, 16 lanes for all against both: 0.4 % such atoms 248 / 213 us, 2.1 %
-// 279 / 286 us, 5.8 % 323 / 369 us (a group of 8 atoms with one of them costs as before, and its launch finds the others by their
-// counts). 6,000 atoms, one wave per SIMD either way: 0.07 % 97 / 98 us, 1.3 % 125 / 131 us.
-inline int both_sizes_limit(int n) { return n < 12000 ? -1 : n / 64; }
+// 16); -1: never. With 16 lanes for all a wave takes 4 atoms: up to 12,288 of them (3 waves on each of the 1,024 SIMDs, FP32 terms) run
+// at once, and nothing is gained. Beyond that, the three term kernels of disordered carbon, 16 lanes for all against both (a group of 8
+// atoms with one of those atoms costs as before, and its launch finds the others by their counts):
+//   FP32 terms, 12,000 atoms 0.4 % 133 / 138 us, 1.1 % 135 / 151; 12,400 0.3 % 149 / 138, 1.3 % 163 / 154; 16,000 0.2 % 161 / 135, 1.6 %
+//   189 / 186; 30,000 0.4 % 244 / 209, 1.3 % 264 / 242, 2.1 % 273 / 283. (24,000, two rounds of waves either way: 0.7 % 206 / 207,
+//   1.4 % 220 / 229.)
+//   FP64 terms, 12,400 atoms 0.3 % 173 / 144 us, 0.7 % 180 / 188; 14,000 0.2 % 175 / 165, 1.2 % 199 / 215; 16,000 0.2 % 182 / 181, 1.3 %
+//   210 / 219; 18,000 0.3 % 209 / 188, 1.6 % 248 / 235; 20,000 1.4 % 264 / 245; 30,000 1.3 % 342 / 331, 2.1 % 354 / 377.
+inline int both_sizes_limit(Precision p, int n) { return n <= 12288 ? -1 : p == Precision::FP64 && n < 18000 ? n / 256 : n / 64; }
 void launch_angle_terms(Precision p, const State& st, const Globals& g, const Tables& t, int bmax, bool both, hipStream_t s);
 // BO-derivative pass (CdDelta, then the per-atom bond sums); the final gather adds the non-bonded gradient and the virial
 void launch_bond_derivatives(const State& st, hipStream_t s);
