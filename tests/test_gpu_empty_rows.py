@@ -5,8 +5,8 @@ storage has held other columns.
 
 A solve's charges q = s - mu t, mu = sum(s) / sum(t), from A s = -chi + r_s and A t = -1 + r_t, satisfy A q + chi - mu = r_s - mu r_t in
 every row (A = diag(eta) + H; H q comes from qeq_matvec, whose kernel shares no code with the solve's product). Each residual is
-bounded by the solve's stopping rule, |r|_i <= sqrt(eta_i) tol |b| with |b|^2 = sum b^2 / eta; the bar is twice that, for the
-difference between the recursion's residual and the true one, plus 1e-12 of the largest product for rounding."""
+bounded by the solve's stopping rule sqrt(r.r / eta) <= tol |b|: |r_i| <= sqrt(eta_i) tol |b|; the bar is twice that, for the difference between
+the recursion's residual and the true one, plus 1e-12 of the largest product for rounding."""
 import numpy as np
 import pytest
 
@@ -38,7 +38,7 @@ def check(e, x, types, chi, eta, solve):
     c, n = chi[types], eta[types]
     r = y + c
     mu = (r / n).sum() / (1.0 / n).sum()
-    bar = 2.0 * TOL * np.sqrt(n) * (np.sqrt((c * c / n).sum()) + abs(mu) * np.sqrt((1.0 / n).sum())) + 1e-12 * max(1.0, np.abs(y).max())
+    bar = 2.0 * TOL * np.sqrt(n) * (np.sqrt((c * c).sum()) + abs(mu) * np.sqrt(len(c))) + 1e-12 * max(1.0, np.abs(y).max())
     # mu is taken from the residuals themselves: their weighted mean moves it by no more than the largest of them
     assert (np.abs(r - mu) <= bar + bar.max()).all(), np.abs(r - mu).max()
     assert abs(q.sum()) <= 1e-10 * len(q)
