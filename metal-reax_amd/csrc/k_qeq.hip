@@ -311,9 +311,8 @@ __global__ void __launch_bounds__(kMvThreads) k_spmv2(int n, int stride, const i
 //   then for every row i: w = (diag(eta) + H) p, d_i = p_i + beta d_i, q_i = w_i + beta q_i (= (diag(eta) + H) d_i by
 //   linearity, so the direction never has to be complete before the product), and per-block partials of d.q.
 // Block 0 records sig (slot it-1) and the activity flags of iteration it for the later kernels and the host.
-// chk = 1: a refinement check ran before this launch (after update(it - 1)); if it restarted the solve (its record in slot
-// it - 1 is not the marker -1), iteration it starts afresh from the true residual (beta 0, activity from the record), else the
-// iteration continues as usual.
+// chk = 1: a refinement check that restarts the solve ran before this launch (after update(it - 1)): iteration it starts afresh from the
+// true residual (beta 0, activity from the check's record in slot it - 1).
 // The previous update's partials and the activity flags are loaded together at the start, the row's own vector entries before the
 // walk, and lanes 0 and 8 of a row's group finish one system each.
 template <class VA, class TC>
@@ -326,7 +325,7 @@ __global__ void __launch_bounds__(kMvThreads) k_cg_mvdir(int n, int stride, cons
   bool fresh = it == 1;
   if (fresh) {
     act[0] = ACT(qb.scal, 0)[0]; act[1] = ACT(qb.scal, 0)[1];
-  } else if (chk && RST(qb.scal, it - 1)[0] >= 0) {
+  } else if (chk) {
     fresh = true;
     act[0] = RST(qb.scal, it - 1)[0]; act[1] = RST(qb.scal, it - 1)[1];
     if (blockIdx.x == 0 && threadIdx.x == 0) { put_act(qb, it - 1, 0, act[0]); put_act(qb, it - 1, 1, act[1]); }
