@@ -3,10 +3,10 @@
 // Pipeline per step (one launch each, in stream order):
 //   bond_build  (atoms per wave)  bond list from the skin list: d <= bond_cut and BO' >= bo_cut, uncorrected BO', dBO'/dx, Delta'
 //                                 [reference src/cpu/bonded.cpp:109-162, terms.hpp:50-56]; H-bond partner lists [bonded.cpp:120-124]
-//   bo_correct  (thread per atom) corrected BO and its 11 derivative coefficients, always from the pair's canonical end so both ends
+//   bo_correct  (L lanes per atom, with_lanes) corrected BO and its 11 derivative coefficients, always from the pair's canonical end so both ends
 //                                 hold bitwise-identical values [bonded.cpp:164-204, terms.hpp:66-164]; index of the mirror slot of
-//                                 every bond and the step's largest bond count
-//   atom_terms  (thread per atom) bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
+//                                 every bond, the step's largest bond count and the atoms with more than 8 bonds
+//   atom_terms  (as bo_correct)   bond energy + triple-bond stabilisation, lone pair + C2, over/under coordination [bonded.cpp:219-318]
 //   valence     (wave per 64 / G atoms, angles spread over its lanes; G: both_sizes_limit, with_group) valence angle, penalty, 3-body conjugation at the centre
 //                                 [bonded.cpp:321-474]
 //   torsion     (as valence)      torsion + 4-body conjugation, evaluated at BOTH atoms of the central bond; each end keeps the force
@@ -57,9 +57,6 @@ template <> __device__ inline float racos(float x) { return acosf(x); }
 template <class T> __device__ inline T rsin(T x);
 template <> __device__ inline double rsin(double x) { return sin(x); }
 template <> __device__ inline float rsin(float x) { return sinf(x); }
-template <class T> __device__ inline T rcos(T x);
-template <> __device__ inline double rcos(double x) { return cos(x); }
-template <> __device__ inline float rcos(float x) { return cosf(x); }
 template <class T> __device__ inline T ratan2(T y, T x);
 template <> __device__ inline double ratan2(double y, double x) { return atan2(y, x); }
 template <> __device__ inline float ratan2(float y, float x) { return atan2f(y, x); }
@@ -1375,7 +1372,7 @@ __device__ __forceinline__ void torsion_body(const State& st, const Globals& g, 
   }
 }
 
-// FP32 terms: 156 VGPRs and 45 KB of LDS per block, 3 waves per SIMD; FP64 held to 2 (216 VGPRs, 67 KB). kCen: the variant that also
+// FP32 terms: 155 VGPRs and 45 KB of LDS per block, 3 waves per SIMD; FP64 held to 2 (213 VGPRs, 67 KB). kCen: the variant that also
 // records the torsion census (launched only for a force call that asks for it, so the counter costs the ordinary step nothing)
 template <class TS, int G, bool kCen, bool PA>
 __global__ void __launch_bounds__(64 * kAngleWaves) k_torsion_f(State st, Globals g, Tables t, int blocks16) {

@@ -274,9 +274,11 @@ __global__ void __launch_bounds__(64 * kNbWaves) k_nonbonded_d(State st, Globals
 // pair loop they cost as much address traffic as the positions, and, loads returning in order, a wait for all that is in flight for the
 // next pairs. The non-bonded pass over the rows took 81 us at 24,000 atoms and 661 us at 192,000; with chunks that have no shift taken
 // without one 76 and 588, with these tables 62 and 466, with the row's own data in scalar registers (wave_atom) 58 and 411. Two
-// capacities, since the matrix build's ring leaves room for 8 blocks per CU with 32 shifts (cells wider than the list radius have 27)
-// and for 5 with 128 (125 where one more image is in reach): 40 packed systems with 125 shifts, one capacity of 64 (tables in memory)
-// 23.2 ms for 20 steps, with 128 22.7 ms. Cells with more shifts (thin ones) or force fields with more types read them from memory.
+// capacities: with its ring the matrix build takes 20 KB per block with 32 shifts and 29 KB (5 blocks per CU, as many as its registers
+// allow) with 128. A single periodic cell has 27 shifts from three list radii per side on (the cell search) and at least 125 below (one
+// image more than reaches); packed systems have 27 where all are wider than two radii, 125 down to two thirds of one: 40 of them with
+// 125 shifts, one capacity of 64 (tables in memory) 23.2 ms for 20 steps, with 128 22.7 ms. Cells with more shifts (thin ones) or
+// force fields with more types read them from memory.
 constexpr int kTabTypes = 16;
 // the tables' capacity in shift vectors (0: no tables)
 inline int row_table_shifts(const State& st, const Globals& g) {
@@ -370,7 +372,8 @@ __device__ inline void nb_rows_wave(const State& st, const Globals& g, const Tab
   nb_finish<D>(st, t, i, ti, lane, a);
 }
 
-// (5 waves per SIMD: 96 VGPRs without spills; the compiler's choice, 106 VGPRs and 4 waves, is slower)
+// (asked for 5 waves per SIMD: with the row's data in vector registers 96 VGPRs without spills, where the compiler's own choice of 106 and 4
+// waves was slower; 79 and 6 waves since it is in scalar ones)
 template <class TC, int kTab>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_nonbonded_rows(State st, Globals g, Tables t, const TC* __restrict__ col,
                                                         const unsigned short* __restrict__ key, const int* __restrict__ rcnt, int stride) {
@@ -395,8 +398,9 @@ constexpr int kQbWaves = 4, kQbRing = 256;
 // costly part runs on full waves. Bound by the latency of a wave's chain of loads: doing the arithmetic, the position gathers or the
 // stores twice adds 0 to 5 %. So two chunks go through the chain at once, each round's loads go out in the order in which they are
 // waited for (the guess gathers of the batches, the next positions, the entries after those), and the row's own data sit in scalar
-// registers (79 VGPRs, 6 waves per SIMD). 24,000 / 192,000 atoms of water: 138 / 1064 us a chunk at a time with the tables in memory,
-// 137 / 1075 with the tables in LDS, 123 / 945 two chunks at a time, 117 / 915 us with the row's data in scalar registers. Row entries are kept in skin-list
+// registers. 24,000 / 192,000 atoms of water: 138 / 1064 us a chunk at a time with the tables in memory, 137 / 1075 with the tables in
+// LDS, 123 / 945 two chunks at a time, 117 / 915 us with the row's data in scalar registers (79 VGPRs, 6 waves per SIMD), 113 / 872 us with
+// the stores in whole groups (81 VGPRs, 5 waves). Row entries are kept in skin-list
 // order: slot m of the row is the m-th pair of the list within the cutoff. The 16-bit key is the canonical flag and the
 // shift-table index the distance used.
 // fuse: the row also forms the charge solve's start from the guess in x (k_cg_guess ran before): y = H x with the values as

@@ -166,8 +166,8 @@ template <> struct FourCols<int> { using T = int4; };
 // the last group in list order, read entry by entry, 179, 1530 and 227 us. With the first loads sent before the reduction of the last
 // launch's partials, 175, 1526 and 215 us: a launch after both solves have stopped then reads two groups of every row for nothing (28 us
 // instead of 4 at 192,000 rows). The next two groups' entries in flight during a pair's gathers took 186, 1540 and 216 us (90 VGPRs, 5
-// waves per SIMD: 24,000 rows no longer fit the chip at once; at 80 they just do, which is why the launch's flags and beta are held in
-// scalar registers).
+// waves per SIMD: 24,000 rows no longer fit the chip at once; at 80, the FP32 values with 16-bit columns, they just do, which is why the
+// launch's flags and beta are held in scalar registers). With 32-bit columns the product has 82 VGPRs, with FP64 values 94 to 96: 5 waves.
 template <class VA, class TC>
 struct RowProduct {
   struct Pair { typename FourCols<TC>::T c[2]; typename VA::Four h[2]; };   // two groups
